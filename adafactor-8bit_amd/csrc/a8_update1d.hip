@@ -46,8 +46,10 @@ static int finish_norm_1d(int mode, const Desc1D& one, const Desc1D* table, int 
 
 static int launch_any(int dtype, int sr, int vbits, int mode, const Desc1D& one, const Desc1D* table,
                       int ntab, int64_t nwg, const Hyper1D& h, hipStream_t st) {
-  if (h.krule) return launch_any_kernel_rule(dtype, sr, vbits, mode, one, table, ntab, nwg, h, st);
-  return launch_rule<0>(dtype, sr, vbits, mode, one, table, ntab, nwg, h, st);
+  const bool half = dtype == A8_BF16 || dtype == A8_F16;
+  if (h.krule) return (half ? launch_any_kernel_rule_16bit : launch_any_kernel_rule)(dtype, sr, vbits, mode, one, table, ntab, nwg, h, st);
+  if (half) return launch_any_16bit(dtype, sr, vbits, mode, one, table, ntab, nwg, h, st);
+  return launch_rule<0, true>(dtype, sr, vbits, mode, one, table, ntab, nwg, h, st);
 }
 
 static int check_common(int dtype, int64_t numel, int bv, int bm, int mbits, int mmode, int vbits,
@@ -397,7 +399,9 @@ int a8_set_qmap(const float* qmap8_host, const float* qmap4_host) {
       a8::decode_upload_qmap(qmap8_host, qmap4_host) != hipSuccess ||
       a8::sgd_upload_qmap(qmap8_host, qmap4_host) != hipSuccess ||
       a8::prims_upload_qmap(qmap8_host, qmap4_host) != hipSuccess ||
-      a8::update1d_k_upload_qmap(qmap8_host, qmap4_host) != hipSuccess)
+      a8::update1d_h_upload_qmap(qmap8_host, qmap4_host) != hipSuccess ||
+      a8::update1d_k_upload_qmap(qmap8_host, qmap4_host) != hipSuccess ||
+      a8::update1d_kh_upload_qmap(qmap8_host, qmap4_host) != hipSuccess)
     return set_error(A8_ERR_HIP, "codebook upload failed");
   return 0;
 }

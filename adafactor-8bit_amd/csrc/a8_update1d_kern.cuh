@@ -1,6 +1,7 @@
-// Kernels of the fused 1-D step and their launch templates, shared by the two
-// translation units that instantiate them: a8_update1d.hip (KR = 0, the CPU
-// quantiser's AL rule) and a8_update1d_k.hip (KR = 1, the reference kernels' AL
+// Kernels of the fused 1-D step and their launch templates, shared by the
+// translation units that instantiate them: a8_update1d.hip and a8_update1d_h.hip
+// (KR = 0, the CPU quantiser's AL rule; 16-bit parameters in the second),
+// a8_update1d_k.hip and a8_update1d_kh.hip (KR = 1, the reference kernels' AL
 // rule, A8_AL_KERNEL_RULE).  KR is a template parameter so that each rule's kernel
 // carries only its own refit code.
 #pragma once
@@ -1011,27 +1012,32 @@ static int launch_dispatch(int vbits, int mode, const Desc1D& one, const Desc1D*
 }
 
 // Every instantiation of one AL rule (KR = 0: the CPU quantiser's, 1: the reference
-// kernels'); each rule's instantiations live in their own translation unit.
-template <int KR>
+// kernels') for 32- and 64-bit parameters (WIDE) or for 16-bit ones; each has a
+// translation unit of its own, so that they compile in parallel.
+template <int KR, bool WIDE>
 static int launch_rule(int dtype, int sr, int vbits, int mode, const Desc1D& one, const Desc1D* table,
                        int ntab, int64_t nwg, const Hyper1D& h, hipStream_t st) {
   if ((mode == 1 || mode == 4) && sr) sr = 0;
-  switch (dtype) {
-    case A8_F32: return launch_dispatch<float, false, KR>(vbits, mode, one, table, ntab, nwg, h, st);
-    case A8_BF16:
+  if constexpr (WIDE) {
+    if (dtype == A8_F32) return launch_dispatch<float, false, KR>(vbits, mode, one, table, ntab, nwg, h, st);
+    if (dtype == A8_F64) return launch_dispatch<double, false, KR>(vbits, mode, one, table, ntab, nwg, h, st);
+  } else {
+    if (dtype == A8_BF16)
       return sr ? launch_dispatch<__hip_bfloat16, true, KR>(vbits, mode, one, table, ntab, nwg, h, st)
                 : launch_dispatch<__hip_bfloat16, false, KR>(vbits, mode, one, table, ntab, nwg, h, st);
-    case A8_F16:
+    if (dtype == A8_F16)
       return sr ? launch_dispatch<__half, true, KR>(vbits, mode, one, table, ntab, nwg, h, st)
                 : launch_dispatch<__half, false, KR>(vbits, mode, one, table, ntab, nwg, h, st);
-    case A8_F64: return launch_dispatch<double, false, KR>(vbits, mode, one, table, ntab, nwg, h, st);
-    default: return set_error(A8_ERR_DTYPE, "unsupported param dtype");
   }
+  return set_error(A8_ERR_DTYPE, "unsupported param dtype");
 }
 
-
-// KR = 1 instantiations (a8_update1d_k.hip).
+// 16-bit parameters, KR = 0 (a8_update1d_h.hip); KR = 1 (a8_update1d_k.hip, a8_update1d_kh.hip).
+int launch_any_16bit(int dtype, int sr, int vbits, int mode, const Desc1D& one, const Desc1D* table,
+                     int ntab, int64_t nwg, const Hyper1D& h, hipStream_t st);
 int launch_any_kernel_rule(int dtype, int sr, int vbits, int mode, const Desc1D& one, const Desc1D* table,
                            int ntab, int64_t nwg, const Hyper1D& h, hipStream_t st);
+int launch_any_kernel_rule_16bit(int dtype, int sr, int vbits, int mode, const Desc1D& one, const Desc1D* table,
+                                 int ntab, int64_t nwg, const Hyper1D& h, hipStream_t st);
 
 }  // namespace a8
