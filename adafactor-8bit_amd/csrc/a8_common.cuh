@@ -110,12 +110,77 @@ __device__ __forceinline__ void div_by(float* q, const float* x, float d, float 
   }
 }
 
-__device__ __forceinline__ float log2_exact(float x) {   // x > 0, correctly rounded to fp32
-  return (float)::log2((double)x);
+// A double constant held in scalar registers (S): a VALU fma reads one scalar operand,
+// while a 64-bit literal costs two moves into vector registers before every use.  Worth
+// its twenty scalar registers where a lane evaluates several polynomials.
+template <bool S>
+__device__ __forceinline__ double sconst(double c) {
+  if constexpr (S) asm("" : "+s"(c));
+  return c;
 }
 
+// (2^f - 1) / f on |f| <= 1/2: the degree-9 interpolant at the Chebyshev nodes, within
+// 2^-50; f times it is 2^f - 1 within 2^-51 and keeps its relative accuracy near f = 0.
+template <bool S>
+__device__ __forceinline__ double exp2m1_q(double f) {
+  double q = sconst<S>(0x1.e5e9f548e5725p-28);
+  q = __builtin_fma(q, f, sconst<S>(0x1.b6571de2f2351p-24));
+  q = __builtin_fma(q, f, sconst<S>(0x1.62bfe46117445p-20));
+  q = __builtin_fma(q, f, sconst<S>(0x1.ffcb76789860fp-17));
+  q = __builtin_fma(q, f, sconst<S>(0x1.4309130378460p-13));
+  q = __builtin_fma(q, f, sconst<S>(0x1.5d87fe908f88ap-10));
+  q = __builtin_fma(q, f, sconst<S>(0x1.3b2ab6fba385fp-7));
+  q = __builtin_fma(q, f, sconst<S>(0x1.c6b08d7044119p-5));
+  q = __builtin_fma(q, f, sconst<S>(0x1.ebfbdff82c590p-3));
+  return __builtin_fma(q, f, sconst<S>(0x1.62e42fefa39f7p-1));
+}
+
+// 2^x rounded to fp32 for |x| < 2^20: x = n + f with n the nearest integer (f exact),
+// 2^f in double, scaled and rounded once.
+template <bool S = false>
+__device__ __forceinline__ float exp2_core(float x) {
+  const float n = rintf(x);
+  const double f = (double)(x - n);
+  return (float)__builtin_amdgcn_ldexp(__builtin_fma(exp2m1_q<S>(f), f, 1.0), (int)n);
+}
+
+// log2(x) rounded to fp32, a third of the operations of a double-precision logarithm:
+// the hardware logarithm l (within an ulp or so) corrected by log2(x / 2^l), where
+// x / 2^l = m 2^(k - l) for k the integer nearest l and m = x / 2^k, and
+// e = (m - 1) + m (2^(k - l) - 1) is below 2^-16, so log2(1 + e) needs two terms.  Every
+// step before the last is exact or in double.  Subnormal x is scaled first; zero,
+// infinities and NaN take the hardware's result (uniform branches, rarely taken).
+// Equal to the double-precision logarithm rounded to fp32 on every float.
+template <bool S = false>
+__device__ __forceinline__ float log2_exact(float x) {
+  float xs = x;
+  float off = 0.0f;
+  const bool rare = !(x >= kFltMin && x < __builtin_inff());
+  if (__builtin_amdgcn_ballot_w64(rare)) {
+    if (x < kFltMin) { xs = x * 0x1p32f; off = -32.0f; }
+  }
+  const float l = __builtin_amdgcn_logf(xs);
+  const float k = rintf(l);
+  const float m = __builtin_amdgcn_ldexpf(xs, -(int)k);
+  const double f = (double)(k - l);
+  const double p = exp2m1_q<S>(f) * f;
+  const double e = __builtin_fma((double)m, p, (double)(m - 1.0f));
+  const double c = __builtin_fma(e * -0.5, e, e);
+  float r = (float)__builtin_fma(c, 0x1.71547652b82fep+0, (double)l + (double)off);
+  if (__builtin_amdgcn_ballot_w64(rare)) {
+    if (!(x > 0.0f && x < __builtin_inff())) r = x < 0.0f ? __builtin_nanf("") : __builtin_amdgcn_logf(x);
+  }
+  return r;
+}
+
+template <bool S = false>
 __device__ __forceinline__ float exp2_exact(float x) {
-  return (float)::exp2((double)x);
+  float r = exp2_core<S>(x);
+  const bool rare = !(fabsf(x) < 0x1p20f);
+  if (__builtin_amdgcn_ballot_w64(rare)) {
+    if (rare) r = __builtin_amdgcn_exp2f(x);   // infinities, NaN, and results that are 0 or inf
+  }
+  return r;
 }
 
 __device__ __forceinline__ float fast_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
@@ -187,6 +252,36 @@ __device__ __forceinline__ void al_kfit(float lmax_raw, float lmin_raw, float fl
 template <int LM2>
 __device__ __forceinline__ float al_dec_log(float c1, float s, float lm, bool krule) {
   return krule ? (c1 * (1.0f / (float)LM2)) * s + lm : (c1 * s) / (float)LM2 + lm;
+}
+
+// The values of N codes of one block (s, lm): 0 for code 0, else 2^al_dec_log rounded to
+// fp32.  For any range a refit can produce (and far beyond) the division by the constant
+// LM2 is one Markstein correction of the product with its rounded reciprocal (the
+// correctly rounded quotient; checked for every fp32 mantissa) and the exponent is inside
+// exp2_core's range; a wave that holds anything else adds the IEEE division and
+// exp2_exact's outliers.
+template <int LM2, int N>
+__device__ __forceinline__ void al_decode(const uint32_t* c, float s, float lm, bool krule, float* v) {
+  constexpr float rc = 1.0f / (float)LM2;
+  if (__builtin_amdgcn_ballot_w64(!(s > 0x1p-60f && s < 0x1p18f && fabsf(lm) < 0x1p18f))) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = exp2_exact<(N >= 4)>(al_dec_log<LM2>((float)c[i] - 1.0f, s, lm, krule));
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const float x = __builtin_fmaf((float)c[i], s, -s), q0 = x * rc;   // x = RN((c - 1) s)
+      const float q = krule ? ((float)c[i] - 1.0f) * rc * s : __builtin_fmaf(__builtin_fmaf(-q0, (float)LM2, x), rc, q0);
+      v[i] = exp2_core<(N >= 4)>(q + lm);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] = c[i] ? v[i] : 0.0f;
+}
+template <int LM2>
+__device__ __forceinline__ float al_decode(uint32_t c, float s, float lm, bool krule) {
+  float v;
+  al_decode<LM2, 1>(&c, s, lm, krule, &v);
+  return v;
 }
 
 // krule: vmin_nz is the block minimum including zeros, and the fit is al_kfit's.

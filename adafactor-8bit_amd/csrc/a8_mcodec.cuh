@@ -123,6 +123,68 @@ __device__ __forceinline__ T sr_round(float x, uint64_t seed, uint64_t step, uin
   }
 }
 
+// Stochastic rounding and store of four consecutive elements (base + i0 a multiple of
+// four elements from an aligned address; i0 + 4 <= n in one 8-byte store).  z is the
+// counter of the first, and srs what the counters of a whole unit share: unless the
+// unit crosses a multiple of 2^30 they agree from bit 30 up, so the high word's part of
+// the first product and the low word of z >> 30 are uniform (scalar registers).
+//
+// bf16: when all four values are finite and below the largest that can round up, the
+// guards of sr_bf16_hi fall away: it rounds up when (hv >> 16) < (bits & 0xFFFF), which
+// is when bits + (0xFFFF - (hv >> 16)) carries into the high half, and the high halves
+// of a pair then make one word.
+struct SrUnit {
+  uint32_t sh30, yhc;
+  bool same;
+};
+template <int N>   // elements of the unit
+__device__ __forceinline__ SrUnit sr_unit(uint64_t z) {
+  const uint32_t zl = (uint32_t)z, zh = (uint32_t)(z >> 32);
+  return SrUnit{(zh << 2) | (zl >> 30), sm_yhc(zh), (zl & 0x3FFFFFFFu) <= 0x40000000u - N};
+}
+
+template <typename T>
+__device__ __forceinline__ void sr_store4(T* base, uint32_t i0, uint32_t n, const float* x, uint64_t z,
+                                          const SrUnit& srs) {
+  static_assert(sizeof(T) == 2, "16-bit parameters");
+  uint32_t hv[4];
+  if (srs.same) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) hv[k] = sm_hi_ys((uint32_t)z + (uint32_t)k, srs.sh30, srs.yhc);
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) hv[k] = sm_hi(z + (uint64_t)k);
+  }
+  uint32_t w[2] = {0u, 0u};
+  if constexpr (std::is_same<T, __hip_bfloat16>::value) {
+    uint32_t amax = 0u;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) amax = max(amax, __float_as_uint(x[k]) & 0x7FFFFFFFu);
+    if (amax < 0x7F7F0000u) {
+      uint32_t sv[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) sv[k] = __float_as_uint(x[k]) + (~hv[k] >> 16);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) w[j] = __builtin_amdgcn_perm(sv[2 * j + 1], sv[2 * j], 0x07060302u);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) w[k >> 1] |= (uint32_t)sr_bf16_hi(x[k], hv[k]) << (16 * (k & 1));
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      w[k >> 1] |= (uint32_t)sr_fp16(x[k], (float)(hv[k] >> 8) * (1.0f / 16777216.0f)) << (16 * (k & 1));
+  }
+  A8_G uint16_t* p = gp(reinterpret_cast<uint16_t*>(base));
+  if (i0 + 4 <= n) {
+    *gp(reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(base) + i0)) = u32x2{w[0], w[1]};
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (i0 + k < n) p[i0 + k] = (uint16_t)(w[k >> 1] >> (16 * (k & 1)));
+  }
+}
+
 // ------------------------------------------------------------ M codecs
 __device__ __forceinline__ float m_decode(int mk, uint32_t q, float s) {
   switch (mk) {

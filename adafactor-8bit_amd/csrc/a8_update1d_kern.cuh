@@ -61,6 +61,12 @@ constexpr int kLanes = 256;
 constexpr int kEPT = 8;
 constexpr int kWGElems = kLanes * kEPT;
 constexpr int kHalf = kWGElems / 2;
+// V blocks per unit from which AL8 codes are decoded element by element.  A lane then
+// evaluates 8 powers for its own codes; the tables of 4 / 8 / 16 blocks cost it 4 / 8 / 16
+// powers, as many LDS writes, 8 LDS reads and a barrier.  218 M bf16 parameters with SR,
+// VALU bound: B_V 512 table 667 us, B_V 256 table 707, B_V 128 table over 800, element by
+// element 629 at any of them; B_V 1024 (2 tables) 617, B_V 2048 (1 table) 495.
+constexpr int kDirectBlocks = 4;
 
 // Tensor table in device memory: ntab descriptors, then one int32 first
 // workgroup per tensor.  It is uniform per workgroup and read-only during the
@@ -90,6 +96,8 @@ __device__ __forceinline__ Desc1D load_desc(const Desc1D* tab, int n, int wg) {
 // over the non-zero entries; with koff = 0 (the kernels' rule) zeros count.
 
 // MK: 0 no momentum, 1 UF8 (specialised), 2 UF4/D8/D4 (codec chosen by h.mk).
+// VB: 8 AL8 decoded through LDS tables of the unit's blocks, 9 AL8 decoded element by
+// element (units of kDirectBlocks blocks or more), 16 AL16.
 // MODE: 0 single pass, 1 NORM (V codes + v_buf, sum of squares), 2 APPLY (reads
 // v_buf, writes M and p), 3 LAG (single pass clipped by the previous norm),
 // 4 MNORM (momentum-only: reads v_buf, clips U by the NORM pass's sum of U^2 in
@@ -166,13 +174,15 @@ __device__ __forceinline__ void unit_step(const Desc1D& D, const Hyper1D& h, int
   uint32_t vq8[2] = {0u, 0u}, mq8[2] = {0u, 0u}, mq4[2] = {0u, 0u};
   u32x2 vq16[2] = {{0u, 0u}, {0u, 0u}};
   float ms[2] = {0.0f, 0.0f};
+  float vs[2] = {0.0f, 0.0f}, vl[2] = {0.0f, 0.0f};   // block scale and min_log (no table)
 #pragma unroll
   for (int k = 0; k < kEPT; ++k) { g[k] = 0.0f; pin[k] = 0; }
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     if (vok[j]) {
       if constexpr (!kVbuf) {
-        if constexpr (VB == 8) vq8[j] = *gp(reinterpret_cast<const uint32_t*>(V8u + lo[j]));
+        if constexpr (VB != 8) { vs[j] = gp(VSu)[vloc[j]]; vl[j] = gp(VLu)[vloc[j]]; }
+        if constexpr (VB != 16) vq8[j] = *gp(reinterpret_cast<const uint32_t*>(V8u + lo[j]));
         else vq16[j] = *gp(reinterpret_cast<const u32x2*>(V16u + lo[j]));
       }
       if (mok[j]) {
@@ -182,10 +192,10 @@ __device__ __forceinline__ void unit_step(const Desc1D& D, const Hyper1D& h, int
       }
       if constexpr (FULL) {
         load4v<T>(Gu, lo[j], g + 4 * j);
-        if constexpr (kWrite && !SR) load4v<T>(Pu, lo[j], pin + 4 * j);
+        if constexpr (kWrite) load4v<T>(Pu, lo[j], pin + 4 * j);
       } else {
         load4n<T>(Gu, lo[j], nrem, g + 4 * j);
-        if constexpr (kWrite && !SR) load4n<T>(Pu, lo[j], nrem, pin + 4 * j);
+        if constexpr (kWrite) load4n<T>(Pu, lo[j], nrem, pin + 4 * j);
       }
     }
   }
@@ -202,7 +212,7 @@ __device__ __forceinline__ void unit_step(const Desc1D& D, const Hyper1D& h, int
       if (vb0 < nvb && c != 0) {
         const float sc = cp(D.v_scale)[vb0];
         const float lm = cp(D.v_min_log)[vb0];
-        val = exp2_exact(al_dec_log<254>((float)(c - 1), sc, lm, KR));
+        val = al_decode<254>((uint32_t)c, sc, lm, KR);
       }
       tabs[c] = val;
     } else {
@@ -212,7 +222,7 @@ __device__ __forceinline__ void unit_step(const Desc1D& D, const Hyper1D& h, int
         float val = 0.0f;
         if (b < nvb && c != 0) {
           const float sc = gp(D.v_scale)[b], lm = gp(D.v_min_log)[b];
-          val = exp2_exact(al_dec_log<254>((float)(c - 1), sc, lm, KR));
+          val = al_decode<254>((uint32_t)c, sc, lm, KR);
         }
         tabs[k] = val;
       }
@@ -271,21 +281,19 @@ __device__ __forceinline__ void unit_step(const Desc1D& D, const Hyper1D& h, int
       for (int k = 0; k < kEPT; ++k) vn[k] = (k & 3) < cnth[k >> 2] ? gp(VBu)[lo[k >> 2] + (k & 3)] : 0.0f;
     } else {
       float vo[kEPT];
-      if constexpr (VB == 8) {
+      if constexpr (VB != 8) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          uint32_t c[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            c[i] = VB == 16 ? ((i < 2 ? vq16[j].x : vq16[j].y) >> (16 * (i & 1))) & 0xFFFFu : (vq8[j] >> (8 * i)) & 0xFFu;
+          al_decode<VB == 16 ? 65534 : 254, 4>(c, vs[j], vl[j], KR, vo + 4 * j);
+        }
+      } else {
 #pragma unroll
         for (int k = 0; k < kEPT; ++k)
           vo[k] = tabs[vloc[k >> 2] * 256 + ((vq8[k >> 2] >> (8 * (k & 3))) & 0xFFu)];
-      } else {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          float s_old = 0.0f, lm_old = 0.0f;
-          if (vok[j]) { s_old = gp(VSu)[vloc[j]]; lm_old = gp(VLu)[vloc[j]]; }
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const uint32_t c = ((i < 2 ? vq16[j].x : vq16[j].y) >> (16 * (i & 1))) & 0xFFFFu;
-            vo[4 * j + i] = c ? exp2_exact(al_dec_log<65534>((float)(c - 1), s_old, lm_old, KR)) : 0.0f;
-          }
-        }
       }
       float gsq[kEPT];
 #pragma unroll
@@ -412,22 +420,16 @@ __device__ __forceinline__ void unit_step(const Desc1D& D, const Hyper1D& h, int
     if constexpr (kWrite) {
       const bool has_dec = D.decay || h.has_decay;
       const float dec = D.decay ? *gp(D.decay) : (h.has_decay ? h.decay_val : 1.0f);
+      const uint64_t sr_z = SR ? sr_base(D.sr_seed, h.sr_step) + 0x9E3779B97F4A7C15ULL + (uint64_t)ub : 0u;
+      const SrUnit srs = sr_unit<kWGElems>(sr_z);
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         if (!vok[j]) continue;
         if constexpr (SR) {
+          float x[4];   // (p * decay) - step * u, stochastically rounded below
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            if (i < cnth[j]) {
-              const uint32_t e = lo[j] + i;
-              const float pv = ld1<T>(Pu, e);
-              const T r = sr_round<T>(pv * dec - step * uu[4 * j + i], D.sr_seed, h.sr_step,
-                                      (uint64_t)(ub + (int64_t)e));
-              uint16_t bits;
-              __builtin_memcpy(&bits, &r, 2);
-              gp(reinterpret_cast<uint16_t*>(Pu))[e] = bits;
-            }
-          }
+          for (int i = 0; i < 4; ++i) x[i] = pin[4 * j + i] * dec - step * uu[4 * j + i];
+          sr_store4<T>(Pu, lo[j], nrem, x, sr_z + lo[j], srs);
         } else {
           pval_t<T> p[4];
 #pragma unroll
@@ -446,7 +448,7 @@ __device__ __forceinline__ void unit_step(const Desc1D& D, const Hyper1D& h, int
 
   // ---- V refit + codes
   if constexpr (!kVbuf) {
-    const float lm2 = VB == 8 ? 254.0f : 65534.0f;
+    const float lm2 = VB != 16 ? 254.0f : 65534.0f;
     ALFit f[2];
     if (vwhole) {
       // one block per workgroup: reduce over all lanes and both halves; wave 0
@@ -508,26 +510,29 @@ __device__ __forceinline__ void unit_step(const Desc1D& D, const Hyper1D& h, int
       const int qs = lane & 3;
       const float x = qs == 0 ? bmax[0] : (qs == 1 ? mn0 : (qs == 2 ? bmax[1] : mn1));
       const float l = KR ? al_klog(x, (qs & 1) ? -__builtin_inff() : -1e30f) : log2_exact(fmaxf(x, kLogClampIn));
-      const int qb = lane & ~3;
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const float lmax = __shfl(l, qb + 2 * j, 64);
-        float lmin = __shfl(l, qb + 2 * j + 1, 64);
-        if (KR) {
-          al_kfit(lmax, lmin, h.floor_, lm2, f[j]);
-          continue;
-        }
+      // lanes 4q+0/1 form half 0's fit and 4q+2/3 half 1's, once, with moves inside the
+      // quad (DPP) in place of LDS permutes; then every lane takes both
+      ALFit fo;
+      const float lmax = dpp_f<0xA0>(l);   // quad_perm [0,0,2,2]
+      float lmin = dpp_f<0xF5>(l);         // quad_perm [1,1,3,3]
+      if (KR) {
+        al_kfit(lmax, lmin, h.floor_, lm2, fo);
+      } else {
         lmin = fmaxf(lmin, h.floor_);
         if (lmin >= lmax) lmin = lmax - 1.0f;
-        f[j].lmin = lmin;
-        f[j].s = fmaxf(lmax - lmin, 1e-12f);
-        al_fit_consts(f[j], lm2);
+        fo.lmin = lmin;
+        fo.s = fmaxf(lmax - lmin, 1e-12f);
+        al_fit_consts(fo, lm2);
       }
+      f[0] = ALFit{dpp_f<0x00>(fo.lmin), dpp_f<0x00>(fo.s), dpp_f<0x00>(fo.k),
+                   dpp_f<0x00>(fo.c1), dpp_f<0x00>(fo.kmar), dpp_f<0x00>(fo.cmar)};
+      f[1] = ALFit{dpp_f<0xAA>(fo.lmin), dpp_f<0xAA>(fo.s), dpp_f<0xAA>(fo.k),
+                   dpp_f<0xAA>(fo.c1), dpp_f<0xAA>(fo.kmar), dpp_f<0xAA>(fo.cmar)};
     }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       if (!vok[j]) continue;
-      if constexpr (VB == 8) {
+      if constexpr (VB != 16) {
         float r[4];
         bool bad[4];
 #pragma unroll
@@ -626,9 +631,10 @@ __device__ __forceinline__ void unit_step(const Desc1D& D, const Hyper1D& h, int
 }
 
 // Occupancy 7 waves per SIMD (at most 72 VGPRs): measured best on MI355X for
-// this streaming step (more resident waves hide the HBM latency of the loads).
+// this streaming step (more resident waves hide the HBM latency of the loads).  The
+// forms that VALU issue bounds (stochastic rounding, element-wise decoding) take 6.
 template <typename T, int VB, int MODE, bool SR, int MK, int KR>
-__global__ __launch_bounds__(kLanes) __attribute__((amdgpu_waves_per_eu(7)))
+__global__ __launch_bounds__(kLanes) __attribute__((amdgpu_waves_per_eu((SR || VB != 8) ? 6 : 7)))
 void k_update1d(Desc1D one, const Desc1D* __restrict__ table, int ntab, Hyper1D h) {
   extern __shared__ float s_lds[];  // [nv_wg * 256] AL8 tables | cross-wave partials and fits
   if (h.dsc) {
@@ -702,7 +708,7 @@ __global__ __launch_bounds__(kLanes) void k_update1d_gen(Desc1D one, const Desc1
   const float s_old = kVbuf ? 0.0f : gp(D.v_scale)[blk], lm_old = kVbuf ? 0.0f : gp(D.v_min_log)[blk];
   if (lane == 0) { s_st[0] = 0u; s_st[1] = 0xFFFFFFFFu; }
   for (int i = lane; i < (mpb < kGenMaxMB ? mpb : kGenMaxMB); i += kLanes) s_mab[i] = 0u;
-  if (VB == 8 && !kVbuf) s_tab[lane] = lane ? exp2_exact(al_dec_log<254>((float)(lane - 1), s_old, lm_old, KR)) : 0.0f;
+  if (VB == 8 && !kVbuf) s_tab[lane] = al_decode<254>((uint32_t)lane, s_old, lm_old, KR);
   __syncthreads();
 
   // step scale (unit_step's)
@@ -750,7 +756,7 @@ __global__ __launch_bounds__(kLanes) void k_update1d_gen(Desc1D one, const Desc1
         uint32_t c;
         if constexpr (VB == 8) c = gp(reinterpret_cast<const uint8_t*>(D.v_q))[i0 + k];
         else c = gp(reinterpret_cast<const uint16_t*>(D.v_q))[i0 + k];
-        vo[k] = (VB == 8) ? s_tab[c] : (c ? exp2_exact(al_dec_log<(int)LM2>((float)(c - 1), s_old, lm_old, KR)) : 0.0f);
+        vo[k] = (VB == 8) ? s_tab[c] : al_decode<(int)LM2>(c, s_old, lm_old, KR);
         float gsq = g[k] * g[k];
         if (h.eps_g != 0.0f) gsq = gsq + h.eps_g;
         vn[k] = fabsf(h.bv) < 0.5f ? __builtin_fmaf(h.bv, gsq - vo[k], vo[k])
@@ -964,11 +970,17 @@ static bool gen_shape_ok(int bv, int bm) {
 static int64_t unit_of(int bv, int bm) { return fast_shape_ok(bv, bm) ? kWGElems : bv; }
 
 template <typename T, int VB, int MODE, bool SR, int MK, int KR>
+static int launch_unit(const Desc1D& one, const Desc1D* table, int ntab, int64_t nwg, const Hyper1D& h,
+                       hipStream_t st) {
+  const size_t tab = (VB == 8 && MODE != 2 && MODE != 4) ? (size_t)(kWGElems / h.block_size) * 256 : 0;
+  hipLaunchKernelGGL((k_update1d<T, VB, MODE, SR, MK, KR>), dim3((unsigned)nwg), dim3(kLanes),
+                     (tab + 48) * sizeof(float), st, one, table, ntab, h);
+  return check_launch("k_update1d");
+}
+
+template <typename T, int VB, int MODE, bool SR, int MK, int KR>
 static int launch_t(const Desc1D& one, const Desc1D* table, int ntab, int64_t nwg, const Hyper1D& h,
                     hipStream_t st) {
-  const int nv_wg = h.gen ? 1 : kWGElems / h.block_size;
-  size_t lds = ((VB == 8 && MODE != 2 && MODE != 4) ? (size_t)nv_wg * 256 : 0) * sizeof(float) +
-               48 * sizeof(float);
   if (nwg <= 0) return 0;
   if (nwg > 0x7FFFFFFF) return set_error(A8_ERR_SIZE, "too many workgroups");
   if (h.gen) {
@@ -976,9 +988,13 @@ static int launch_t(const Desc1D& one, const Desc1D* table, int ntab, int64_t nw
                        table, ntab, h);
     return check_launch("k_update1d_gen");
   }
-  hipLaunchKernelGGL((k_update1d<T, VB, MODE, SR, MK, KR>), dim3((unsigned)nwg), dim3(kLanes), lds, st, one,
-                     table, ntab, h);
-  return check_launch("k_update1d");
+  // the V decode exists in the modes that read V codes; the reference kernels' rule and
+  // LAG keep the tables at every block size
+  if constexpr (VB == 8 && KR == 0 && MODE != 2 && MODE != 3 && MODE != 4) {
+    if (kWGElems / h.block_size >= kDirectBlocks)
+      return launch_unit<T, 9, MODE, SR, MK, KR>(one, table, ntab, nwg, h, st);
+  }
+  return launch_unit<T, VB, MODE, SR, MK, KR>(one, table, ntab, nwg, h, st);
 }
 
 template <typename T, bool SR, int MK, int KR>
