@@ -768,15 +768,6 @@ def _dev_scalar(opt, device, key, value):
     return t
 
 
-def _v_buf(opt, device, numel):
-    key = (device, "v_buf")
-    b = opt._ws.get(key)
-    if b is None or b.numel() < numel:
-        b = torch.empty(numel, dtype=torch.float32, device=device)
-        opt._ws[key] = b
-    return b[:numel]
-
-
 def _norm_buf(opt, device, which="norm_buf"):
     key = (device, which)
     b = opt._ws.get(key)
@@ -828,7 +819,7 @@ def _decay_args(P):
     return None, 1.0, 0
 
 
-def _launch_1d(opt, P, mode, alpha_t, alpha_val, norm_buf=None, prev_norm=None, v_buf=None):
+def _launch_1d(opt, P, mode, alpha_t, alpha_val, norm_buf=None, prev_norm=None):
     L = nat.lib()
     st, p, g = P.st, P.p, P.g
     dec_t, dec_val, has_dec = _decay_args(P)
@@ -842,14 +833,14 @@ def _launch_1d(opt, P, mode, alpha_t, alpha_val, norm_buf=None, prev_norm=None, 
         rc = L.a8_fused_update_1d(
             mode, int(P.sr), nat.dtype_code(p.dtype), nat.ptr(p), nat.ptr(g), nat.ptr(m_q),
             nat.ptr(m_scale), nat.ptr(vq), nat.ptr(st["variance_scale"]), nat.ptr(st["variance_min_log"]),
-            nat.ptr(v_buf), nat.ptr(norm_buf), nat.ptr(parts), nat.ptr(alpha_t), nat.ptr(prev_norm),
+            None, nat.ptr(norm_buf), nat.ptr(parts), nat.ptr(alpha_t), nat.ptr(prev_norm),
             nat.ptr(dec_t), int(st.get("sr_seed", 0)), int(P.step), P.beta1 if P.has_m else 0.0, P.beta_val, P.eps_d,
             int(P.adam_denom), P.al_floor, P.eps_g, P.eps_sq, p.numel(), P.bs,
             P.mbs if P.has_m else P.bs, m_bits, m_mode, P.d, P.al_vbits,
             int(P.mom_only), float(alpha_val), float(dec_val), int(has_dec),
             nat.stream_of(p.device))
         nat.check(rc, "a8_fused_update_1d")
-        if mode != nat.MODE_APPLY:
+        if mode in (nat.MODE_NOCLIP, nat.MODE_APPLYC):
             _block_view(st, "variance", P.bs)
     else:
         m = st.get("m") if P.has_m else None
@@ -1131,17 +1122,19 @@ def _run_single(opt, P):
         return
     st = P.st
     nb = _norm_buf(opt, dev)
-    vb = _v_buf(opt, dev, P.p.numel()) if P.path == "q1d" else None
-    _launch_1d(opt, P, nat.MODE_NORM, None, 0.0, norm_buf=nb, v_buf=vb)
+    # quantised V: the passes read the old codes, and the last one re-encodes them
+    sums, msums, apply = (nat.MODE_SUM, nat.MODE_MSUM, nat.MODE_APPLYC) if P.path == "q1d" else \
+        (nat.MODE_NORM, nat.MODE_MNORM, nat.MODE_APPLY)
+    _launch_1d(opt, P, sums, None, 0.0, norm_buf=nb)
     if P.fira and P.has_m and P.mom_only:
         # momentum-only: the U-clip uses ||U|| (NORM), Fira the new momentum's
         # norm ||M'|| (optimizer.py:890-896, _apply_update_pytorch 866-875)
         nbm = _norm_buf(opt, dev, "norm_buf_m")
-        _launch_1d(opt, P, nat.MODE_MNORM, None, 0.0, norm_buf=nbm, prev_norm=nb, v_buf=vb)
+        _launch_1d(opt, P, msums, None, 0.0, norm_buf=nbm, prev_norm=nb)
         alpha_t, _ = _fira_apply(opt, st, nbm, alpha_t, alpha_val, P.margin, dev)
     elif P.fira:
         alpha_t, nb = _fira_apply(opt, st, nb, alpha_t, alpha_val, P.margin, dev)
-    _launch_1d(opt, P, nat.MODE_APPLY, alpha_t, alpha_val, norm_buf=nb, v_buf=vb)
+    _launch_1d(opt, P, apply, alpha_t, alpha_val, norm_buf=nb)
 
 
 def _run_batch_f1dc(opt, key, plans):
@@ -1244,10 +1237,10 @@ def _run_batch_f1dc(opt, key, plans):
 
 
 def _run_batch_q1dc(opt, key, plans):
-    """Quantised 1-D tensors with an RMS clip or Fira as one group: NORM (V' to
-    each tensor's slice of one v_buf, sum u^2) -> MNORM (momentum-only Fira) ->
-    one Fira launch over all tensors -> APPLY, each one multi-tensor launch (the
-    per-tensor sequence of _run_single / _dispatch_1d_cuda, optimizer.py:1080-1170,
+    """Quantised 1-D tensors with an RMS clip or Fira as one group: SUM (sum u^2)
+    -> MSUM (momentum-only Fira) -> one Fira launch over all tensors -> APPLYC,
+    each one multi-tensor launch that forms V' from the old codes (the per-tensor
+    sequence of _run_single / _dispatch_1d_cuda, optimizer.py:1080-1170,
     785-793).  Fira's scale reaches APPLY as each tensor's fira_scale."""
     P0 = plans[0]
     dev = P0.p.device
@@ -1263,11 +1256,6 @@ def _run_batch_q1dc(opt, key, plans):
             for pl in plans]
     ent = ws.get(ck)
     if ent is None or ent["refs"] != refs:
-        offs, tot = [], 0
-        for pl in plans:   # v_buf slices start 16-byte aligned
-            offs.append(tot)
-            tot += (pl.p.numel() + 3) // 4 * 4
-        vbuf = torch.empty(max(tot, 4), dtype=torch.float32, device=dev)
         poffs, ptot = [], 0
         for pl in plans:   # per-tensor slices of the passes' partial-sum workspace
             poffs.append(ptot)
@@ -1275,30 +1263,30 @@ def _run_batch_q1dc(opt, key, plans):
         parts = torch.empty(max(ptot, 1), dtype=torch.float64, device=dev)
         acc = torch.zeros(2 * n, dtype=torch.float32, device=dev)    # sum u^2 | sum M'^2
         fout = torch.zeros(3 * n, dtype=torch.float32, device=dev)   # Fira: scale | prev norm | clean sum
-        a0, f0, v0 = acc.data_ptr(), fout.data_ptr(), vbuf.data_ptr()
+        a0, f0 = acc.data_ptr(), fout.data_ptr()
         arrs = {}
-        for mode in (nat.MODE_NORM, nat.MODE_MNORM, nat.MODE_APPLY):
-            if mode == nat.MODE_MNORM and not mnorm:
+        for mode in (nat.MODE_SUM, nat.MODE_MSUM, nat.MODE_APPLYC):
+            if mode == nat.MODE_MSUM and not mnorm:
                 continue
             arr = (nat.Tensor1D * n)()
             for i, pl in enumerate(plans):
                 st = pl.st
                 nb, prev, fs = a0 + 4 * i, None, None
-                if mode == nat.MODE_MNORM:
+                if mode == nat.MODE_MSUM:
                     nb, prev = a0 + 4 * (n + i), a0 + 4 * i
-                elif mode == nat.MODE_APPLY and fira:
+                elif mode == nat.MODE_APPLYC and fira:
                     fs = f0 + 4 * i
                     if not mnorm:   # the update clip reads the Fira launch's finite sum
                         nb = f0 + 4 * (2 * n + i)
-                ap = mode == nat.MODE_APPLY and pl.pers
+                ap = mode == nat.MODE_APPLYC and pl.pers
                 arr[i] = nat.Tensor1D(
                     pl.p.data_ptr(), pl.g.data_ptr(), nat.ptr(st.get("m_q") if pl.has_m else None),
                     nat.ptr(st.get("m_scale") if pl.has_m else None), st["variance_q"].data_ptr(),
-                    st["variance_scale"].data_ptr(), st["variance_min_log"].data_ptr(), v0 + 4 * offs[i], nb,
+                    st["variance_scale"].data_ptr(), st["variance_min_log"].data_ptr(), None, nb,
                     nat.ptr(pl.alpha_t if ap else None), prev, nat.ptr(pl.decay_t if ap else None),
                     pl.p.numel(), int(st.get("sr_seed", 0)), fs, parts.data_ptr() + 8 * poffs[i])
             arrs[mode] = [arr, torch.empty(int(L.a8_table_bytes_1d(n)), dtype=torch.uint8, device=dev), 1]
-        ent = {"refs": refs, "acc": acc, "fout": fout, "vbuf": vbuf, "parts": parts, "arrs": arrs}
+        ent = {"refs": refs, "acc": acc, "fout": fout, "parts": parts, "arrs": arrs}
         if len(ws) > 16:
             ws.clear()
         ws[ck] = ent
@@ -1321,11 +1309,9 @@ def _run_batch_q1dc(opt, key, plans):
         ent["arrs"][mode][2] = 0
 
     acc.zero_()
-    launch(nat.MODE_NORM)
-    for pl in plans:
-        _block_view(pl.st, "variance", pl.bs)
+    launch(nat.MODE_SUM)
     if mnorm:
-        launch(nat.MODE_MNORM)
+        launch(nat.MODE_MSUM)
     if fira:
         # A tensor without a previous norm behaves as one whose previous norm is
         # below 1e-6 (scale 1, next = current), so every slot takes has_prev = 1.
@@ -1348,7 +1334,9 @@ def _run_batch_q1dc(opt, key, plans):
         if not prev_ok:
             for i, pl in enumerate(plans):
                 pl.st["fira_prev_norm"] = fout[n + i].view(())
-    launch(nat.MODE_APPLY)
+    launch(nat.MODE_APPLYC)
+    for pl in plans:
+        _block_view(pl.st, "variance", pl.bs)
 
 
 def _run_batch_sgdc(opt, key, plans):

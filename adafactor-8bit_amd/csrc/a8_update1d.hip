@@ -22,7 +22,7 @@
 
 namespace a8 {
 
-// Second launch of a NORM / LAG / MNORM pass: one workgroup per tensor adds the
+// Second launch of a pass that sums squares: one workgroup per tensor adds the
 // tensor's workgroup partials in index order (sum_parts) and adds the sum to its
 // norm_buf, which the caller zeroed.  The sum is the same bits whatever order
 // the pass's workgroups ran in, and the same in a batched launch as alone.
@@ -38,7 +38,7 @@ __global__ __launch_bounds__(kLanes) void k_update1d_fin(Desc1D one, const Desc1
 
 static int finish_norm_1d(int mode, const Desc1D& one, const Desc1D* table, int ntab, int64_t nwg,
                           hipStream_t st) {
-  if (mode != 1 && mode != 3 && mode != 4) return 0;
+  if (!is_norm_mode(mode)) return 0;
   hipLaunchKernelGGL(k_update1d_fin, dim3(table ? (unsigned)ntab : 1u), dim3(kLanes), 0, st, one, table, ntab,
                      nwg);
   return check_launch("k_update1d_fin");
@@ -46,10 +46,10 @@ static int finish_norm_1d(int mode, const Desc1D& one, const Desc1D* table, int 
 
 static int launch_any(int dtype, int sr, int vbits, int mode, const Desc1D& one, const Desc1D* table,
                       int ntab, int64_t nwg, const Hyper1D& h, hipStream_t st) {
-  const bool half = dtype == A8_BF16 || dtype == A8_F16;
-  if (h.krule) return (half ? launch_any_kernel_rule_16bit : launch_any_kernel_rule)(dtype, sr, vbits, mode, one, table, ntab, nwg, h, st);
-  if (half) return launch_any_16bit(dtype, sr, vbits, mode, one, table, ntab, nwg, h, st);
-  return launch_rule<0, true>(dtype, sr, vbits, mode, one, table, ntab, nwg, h, st);
+  const auto unit = dtype == A8_BF16 ? (h.krule ? launch_1d_kb : launch_1d_b)
+                    : dtype == A8_F16 ? (h.krule ? launch_1d_kh : launch_1d_h)
+                    : h.krule ? launch_1d_k : launch_rule<0, 0>;
+  return unit(dtype, sr, vbits, mode, one, table, ntab, nwg, h, st);
 }
 
 static int check_common(int dtype, int64_t numel, int bv, int bm, int mbits, int mmode, int vbits,
@@ -99,15 +99,15 @@ static int update1d_entry(int mode, int sr, int dtype, void* param, const void* 
   if (rc) return rc;
   if (!v_q || !v_scale || !v_min_log || !grad || (has_m && !m_scale))
     return set_error(A8_ERR_ARG, "null state pointer");
-  if (mode < 0 || mode > 4) return set_error(A8_ERR_ARG, "mode must be 0..4");
-  if (mode != 1 && mode != 4 && !param) return set_error(A8_ERR_ARG, "null param");
+  if (mode < 0 || mode > 7) return set_error(A8_ERR_ARG, "mode must be 0..7");
+  if ((!is_norm_mode(mode) || mode == 3) && !param) return set_error(A8_ERR_ARG, "null param");
   if ((mode == 1 || mode == 2 || mode == 4) && !v_buf) return set_error(A8_ERR_ARG, "NORM/APPLY/MNORM need v_buf");
-  if (mode == 4 && !(norm_buf && prev_norm && has_m && momentum_only))
+  if ((mode == 4 || mode == 7) && !(norm_buf && prev_norm && has_m && momentum_only))
     return set_error(A8_ERR_ARG, "MNORM needs momentum codes, momentum_only, norm_buf and prev_norm");
-  if ((mode == 1 || mode == 3) && !norm_buf) return set_error(A8_ERR_ARG, "NORM/LAG need norm_buf");
-  if (mode == 2 && !norm_buf) return set_error(A8_ERR_ARG, "APPLY needs norm_buf");
+  if ((mode == 1 || mode == 3 || mode == 5) && !norm_buf) return set_error(A8_ERR_ARG, "NORM/LAG need norm_buf");
+  if ((mode == 2 || mode == 6) && !norm_buf) return set_error(A8_ERR_ARG, "APPLY needs norm_buf");
   if (mode == 3 && !prev_norm) return set_error(A8_ERR_ARG, "LAG needs prev_norm");
-  if ((mode == 1 || mode == 3 || mode == 4) && !norm_parts)
+  if (is_norm_mode(mode) && !norm_parts)
     return set_error(A8_ERR_ARG, "NORM/LAG/MNORM need norm_parts (a8_norm_parts_1d doubles)");
   if (!aligned16(param) || !aligned16(grad) || !aligned16(v_q) || (has_m && !aligned16(m_q)))
     return set_error(A8_ERR_ALIGN, "param/grad/code buffers must be 16-byte aligned");
@@ -147,8 +147,8 @@ static int table_image_1d(int mode, int dtype, const a8_tensor1d* tensors, int n
   const bool has_m = tensors[0].m_q != nullptr;
   int rc = check_common(dtype, 0, block_size, m_block_size, m_bits, m_mode, v_bits & ~A8_AL_KERNEL_RULE, has_m);
   if (rc) return rc;
-  if (mode < 0 || mode > 4) return set_error(A8_ERR_ARG, "mode must be 0..4");
-  if (mode == 4 && !momentum_only) return set_error(A8_ERR_ARG, "MNORM needs momentum_only");
+  if (mode < 0 || mode > 7) return set_error(A8_ERR_ARG, "mode must be 0..7");
+  if ((mode == 4 || mode == 7) && !momentum_only) return set_error(A8_ERR_ARG, "MNORM needs momentum_only");
   Desc1D* tab = reinterpret_cast<Desc1D*>(image);
   int32_t* first = image ? reinterpret_cast<int32_t*>(image + sizeof(Desc1D) * (size_t)ntensors) : nullptr;
   const int64_t unit = unit_of(block_size, has_m ? m_block_size : block_size);
@@ -158,14 +158,14 @@ static int table_image_1d(int mode, int dtype, const a8_tensor1d* tensors, int n
     if ((t.m_q != nullptr) != has_m) return set_error(A8_ERR_ARG, "mixed M / no-M tensors in one launch");
     if (!t.grad || !t.v_q || !t.v_scale || !t.v_min_log || (has_m && !t.m_scale))
       return set_error(A8_ERR_ARG, "null state pointer");
-    if (mode != 1 && mode != 4 && !t.param) return set_error(A8_ERR_ARG, "null param");
+    if ((!is_norm_mode(mode) || mode == 3) && !t.param) return set_error(A8_ERR_ARG, "null param");
     if ((mode == 1 || mode == 2 || mode == 4) && !t.v_buf)
       return set_error(A8_ERR_ARG, "NORM/APPLY/MNORM need v_buf");
     if (mode != 0 && !t.norm_buf) return set_error(A8_ERR_ARG, "NORM/APPLY/LAG/MNORM need norm_buf");
-    if ((mode == 3 || mode == 4) && !t.prev_norm) return set_error(A8_ERR_ARG, "LAG/MNORM need prev_norm");
-    if ((mode == 1 || mode == 3 || mode == 4) && !t.norm_parts)
+    if ((mode == 3 || mode == 4 || mode == 7) && !t.prev_norm) return set_error(A8_ERR_ARG, "LAG/MNORM need prev_norm");
+    if (is_norm_mode(mode) && !t.norm_parts)
       return set_error(A8_ERR_ARG, "NORM/LAG/MNORM need norm_parts (a8_norm_parts_1d doubles per tensor)");
-    if (mode == 4 && !has_m) return set_error(A8_ERR_ARG, "MNORM needs momentum codes");
+    if ((mode == 4 || mode == 7) && !has_m) return set_error(A8_ERR_ARG, "MNORM needs momentum codes");
     if (!aligned16(t.param) || !aligned16(t.grad) || !aligned16(t.v_q) || (has_m && !aligned16(t.m_q)))
       return set_error(A8_ERR_ALIGN, "param/grad/code buffers must be 16-byte aligned");
     if (t.numel < 0) return set_error(A8_ERR_SIZE, "numel < 0");
@@ -399,8 +399,10 @@ int a8_set_qmap(const float* qmap8_host, const float* qmap4_host) {
       a8::decode_upload_qmap(qmap8_host, qmap4_host) != hipSuccess ||
       a8::sgd_upload_qmap(qmap8_host, qmap4_host) != hipSuccess ||
       a8::prims_upload_qmap(qmap8_host, qmap4_host) != hipSuccess ||
+      a8::update1d_b_upload_qmap(qmap8_host, qmap4_host) != hipSuccess ||
       a8::update1d_h_upload_qmap(qmap8_host, qmap4_host) != hipSuccess ||
       a8::update1d_k_upload_qmap(qmap8_host, qmap4_host) != hipSuccess ||
+      a8::update1d_kb_upload_qmap(qmap8_host, qmap4_host) != hipSuccess ||
       a8::update1d_kh_upload_qmap(qmap8_host, qmap4_host) != hipSuccess)
     return set_error(A8_ERR_HIP, "codebook upload failed");
   return 0;

@@ -1,14 +1,11 @@
-// The fused 1-D step for 16-bit parameters (bf16, fp16) under the default AL rule:
-// these instantiations of a8_update1d_kern.cuh in a translation unit of their own,
-// so that they compile in parallel with the 32- and 64-bit ones.
+// The fused 1-D step for fp16 parameters: these instantiations of
+// a8_update1d_kern.cuh in a translation unit of their own, so that they compile in
+// parallel with the others.
 #include "a8_update1d_kern.cuh"
 
 namespace a8 {
 
-int launch_any_16bit(int dtype, int sr, int vbits, int mode, const Desc1D& one, const Desc1D* table,
-                     int ntab, int64_t nwg, const Hyper1D& h, hipStream_t st) {
-  return launch_rule<0, false>(dtype, sr, vbits, mode, one, table, ntab, nwg, h, st);
-}
+A8_UNIT(launch_1d_h) { return launch_rule<0, 2>(dtype, sr, vbits, mode, one, table, ntab, nwg, h, st); }
 
 hipError_t update1d_h_upload_qmap(const float* q8, const float* q4) { return upload_qmap_tu(q8, q4); }
 

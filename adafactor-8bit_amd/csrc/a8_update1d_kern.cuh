@@ -1,8 +1,8 @@
 // Kernels of the fused 1-D step and their launch templates, shared by the
-// translation units that instantiate them: a8_update1d.hip and a8_update1d_h.hip
-// (KR = 0, the CPU quantiser's AL rule; 16-bit parameters in the second),
-// a8_update1d_k.hip and a8_update1d_kh.hip (KR = 1, the reference kernels' AL
-// rule, A8_AL_KERNEL_RULE).  KR is a template parameter so that each rule's kernel
+// translation units that instantiate them: a8_update1d.hip, a8_update1d_b.hip and
+// a8_update1d_h.hip (KR = 0, the CPU quantiser's AL rule; 32- and 64-bit, bf16 and fp16
+// parameters), a8_update1d_k.hip, a8_update1d_kb.hip and a8_update1d_kh.hip (KR = 1, the
+// reference kernels' AL rule, A8_AL_KERNEL_RULE).  KR is a template parameter so that each rule's kernel
 // carries only its own refit code.
 #pragma once
 #include "a8_common.cuh"
@@ -101,7 +101,12 @@ __device__ __forceinline__ Desc1D load_desc(const Desc1D* tab, int n, int wg) {
 // MODE: 0 single pass, 1 NORM (V codes + v_buf, sum of squares), 2 APPLY (reads
 // v_buf, writes M and p), 3 LAG (single pass clipped by the previous norm),
 // 4 MNORM (momentum-only: reads v_buf, clips U by the NORM pass's sum of U^2 in
-// prev_norm, and sums M'^2 for Fira; writes no state).
+// prev_norm, and sums M'^2 for Fira; writes no state), 5 SUM, 6 APPLYC, 7 MSUM: NORM,
+// APPLY and MNORM without v_buf.  SUM and MSUM write nothing, so APPLYC forms V' again
+// from the same old codes and gradient -- the same bits -- and re-encodes both states in
+// its one pass.  A clipped step then moves 6 + 16 bytes per fp32 parameter instead of
+// 11 + 19 with V' written and read back in fp32, and the 4 bytes of v_buf per parameter
+// are not allocated: 137.5 M parameters 267 + 437 -> 131 + 395 us.
 //
 // Lane t of a workgroup holds elements j*1024 + 4t + i of its 2048-element
 // unit (half j = 0, 1; i = 0..3), at register index k = 4j + i: every
@@ -118,8 +123,9 @@ template <typename T, int VB, int MODE, bool SR, int MK, bool FULL, int KR>
 __device__ __forceinline__ void unit_step(const Desc1D& D, const Hyper1D& h, int64_t wl, float* s_lds) {
   constexpr bool kHasM = MK != 0;
   constexpr bool kVbuf = MODE == 2 || MODE == 4;     // V comes from the NORM pass
-  constexpr bool kSq = MODE == 1 || MODE == 3 || MODE == 4;
-  constexpr bool kWrite = MODE == 0 || MODE == 2 || MODE == 3;   // p and M
+  constexpr bool kSq = MODE == 1 || MODE == 3 || MODE == 4 || MODE == 5 || MODE == 7;
+  constexpr bool kWrite = MODE == 0 || MODE == 2 || MODE == 3 || MODE == 6;   // p and M
+  constexpr bool kWriteV = MODE == 0 || MODE == 1 || MODE == 3 || MODE == 6;  // V codes
   const int lane = threadIdx.x;
   const int wave = lane >> 6;
   const int64_t n = D.numel;
@@ -212,7 +218,7 @@ __device__ __forceinline__ void unit_step(const Desc1D& D, const Hyper1D& h, int
       if (vb0 < nvb && c != 0) {
         const float sc = cp(D.v_scale)[vb0];
         const float lm = cp(D.v_min_log)[vb0];
-        val = al_decode<254>((uint32_t)c, sc, lm, KR);
+        val = exp2_lib(al_dec_log<254>((float)(c - 1), sc, lm, KR));
       }
       tabs[c] = val;
     } else {
@@ -232,16 +238,16 @@ __device__ __forceinline__ void unit_step(const Desc1D& D, const Hyper1D& h, int
 
   // ---- step scale
   float step = 0.0f, ut_clip = 1.0f;
-  if constexpr (MODE != 1) {
+  if constexpr (MODE != 1 && MODE != 5) {
     float a = D.alpha ? *gp(D.alpha) : h.alpha_val;
-    if (MODE == 2 && D.fira_scale) a = a * *gp(D.fira_scale);
+    if ((MODE == 2 || MODE == 6) && D.fira_scale) a = a * *gp(D.fira_scale);
     if constexpr (MODE == 0) {
       step = a;
     } else {
       float denom = 1.0f;
       if (h.d > 0.0f) {
-        const float nrm = (MODE == 2) ? sqrtf(*gp(D.norm_buf))
-                          : (MODE == 4 ? sqrtf(*gp(D.prev_norm)) : *gp(D.prev_norm));
+        const float nrm = (MODE == 2 || MODE == 6) ? sqrtf(*gp(D.norm_buf))
+                          : ((MODE == 4 || MODE == 7) ? sqrtf(*gp(D.prev_norm)) : *gp(D.prev_norm));
         // U-clip of momentum_only divides by sqrt(n) then d (optimizer.py:894-895);
         // the update clip divides by sqrt(n)*d (optimizer.py:859-863)
         if (MODE == 3)   // LAG has no CPU branch: the CUDA kernels' pn / (sqrtf(numel) * d) in fp32 (kernels.cu:651-655)
@@ -397,7 +403,7 @@ __device__ __forceinline__ void unit_step(const Desc1D& D, const Hyper1D& h, int
       // NORM / LAG: the update (momentum-only: U = g*inv before clipping); MNORM: M'
 #pragma unroll
       for (int k = 0; k < kEPT; ++k) {
-        const float t = (MODE == 4) ? mn[k] : ((mom && (k & 3) < cnth[k >> 2]) ? g[k] * inv[k] : uu[k]);
+        const float t = (MODE == 4 || MODE == 7) ? mn[k] : ((mom && (k & 3) < cnth[k >> 2]) ? g[k] * inv[k] : uu[k]);
         sq = __builtin_fmaf(t, t, sq);
       }
     }
@@ -447,7 +453,7 @@ __device__ __forceinline__ void unit_step(const Desc1D& D, const Hyper1D& h, int
   }
 
   // ---- V refit + codes
-  if constexpr (!kVbuf) {
+  if constexpr (kWriteV) {
     const float lm2 = VB != 16 ? 254.0f : 65534.0f;
     ALFit f[2];
     if (vwhole) {
@@ -676,8 +682,9 @@ __global__ __launch_bounds__(kLanes) void k_update1d_gen(Desc1D one, const Desc1
                                                          Hyper1D h) {
   constexpr bool kHasM = MK != 0;
   constexpr bool kVbuf = MODE == 2 || MODE == 4;
-  constexpr bool kSq = MODE == 1 || MODE == 3 || MODE == 4;
-  constexpr bool kWrite = MODE == 0 || MODE == 2 || MODE == 3;
+  constexpr bool kSq = MODE == 1 || MODE == 3 || MODE == 4 || MODE == 5 || MODE == 7;
+  constexpr bool kWrite = MODE == 0 || MODE == 2 || MODE == 3 || MODE == 6;
+  constexpr bool kWriteV = MODE == 0 || MODE == 1 || MODE == 3 || MODE == 6;
   constexpr float LM2 = VB == 8 ? 254.0f : 65534.0f;
   __shared__ float s_tab[256];
   __shared__ uint32_t s_st[2];           // V max bits, V non-zero minimum key
@@ -713,16 +720,16 @@ __global__ __launch_bounds__(kLanes) void k_update1d_gen(Desc1D one, const Desc1
 
   // step scale (unit_step's)
   float step = 0.0f, ut_clip = 1.0f;
-  if constexpr (MODE != 1) {
+  if constexpr (MODE != 1 && MODE != 5) {
     float a = D.alpha ? *gp(D.alpha) : h.alpha_val;
-    if (MODE == 2 && D.fira_scale) a = a * *gp(D.fira_scale);
+    if ((MODE == 2 || MODE == 6) && D.fira_scale) a = a * *gp(D.fira_scale);
     if constexpr (MODE == 0) {
       step = a;
     } else {
       float denom = 1.0f;
       if (h.d > 0.0f) {
-        const float nrm = (MODE == 2) ? sqrtf(*gp(D.norm_buf))
-                          : (MODE == 4 ? sqrtf(*gp(D.prev_norm)) : *gp(D.prev_norm));
+        const float nrm = (MODE == 2 || MODE == 6) ? sqrtf(*gp(D.norm_buf))
+                          : ((MODE == 4 || MODE == 7) ? sqrtf(*gp(D.prev_norm)) : *gp(D.prev_norm));
         if (MODE == 3)   // LAG has no CPU branch: the CUDA kernels' pn / (sqrtf(numel) * d) in fp32 (kernels.cu:651-655)
           denom = fmaxf(1.0f, nrm / (sqrtf((float)n) * h.d));
         else if (h.momentum_only && kHasM)
@@ -837,7 +844,7 @@ __global__ __launch_bounds__(kLanes) void k_update1d_gen(Desc1D one, const Desc1
         uu[k] = kHasM ? (mom ? mn[k] : mn[k] * inv[k]) : g[k] * inv[k];
         if (k >= cnt) uu[k] = 0.0f;
         if constexpr (kSq) {
-          const float t = (MODE == 4) ? mn[k] : ((mom && k < cnt) ? g[k] * inv[k] : uu[k]);
+          const float t = (MODE == 4 || MODE == 7) ? mn[k] : ((mom && k < cnt) ? g[k] * inv[k] : uu[k]);
           sq = __builtin_fmaf(t, t, sq);
         }
         vmax = max(vmax, __float_as_uint(vn[k]));
@@ -895,7 +902,7 @@ __global__ __launch_bounds__(kLanes) void k_update1d_gen(Desc1D one, const Desc1
       }
     }
   }
-  if constexpr (!kVbuf) {
+  if constexpr (kWriteV) {
     vmax = grp_red_u(vmax, 64, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
     vkey = grp_umin(vkey, 64);
     if ((lane & 63) == 0) {
@@ -909,12 +916,12 @@ __global__ __launch_bounds__(kLanes) void k_update1d_gen(Desc1D one, const Desc1
     if (lane == 0) gp(D.norm_part)[blk] = t;
   }
   __syncthreads();
-  if constexpr (kVbuf && !(kWrite && kHasM)) return;   // MNORM: no state written
+  if constexpr (!kWriteV && !(kWrite && kHasM)) return;   // no state written
   if (kVbuf && nseg > 1) return;   // APPLY in segments: M codes and scales are written, V has none
 
   // ---- block fit (one lane pair) and pass 2: codes
   ALFit f{};
-  if constexpr (!kVbuf) {
+  if constexpr (kWriteV) {
     if (lane < 64) {
       const uint32_t key = s_st[1];
       const float mnz = key == 0xFFFFFFFFu ? __builtin_inff() : __uint_as_float(key + koff);
@@ -932,7 +939,7 @@ __global__ __launch_bounds__(kLanes) void k_update1d_gen(Desc1D one, const Desc1
     bool m_ok;
     quad_state(q, g, vn, mn, inv, cnt, mb, m_ok, nseg == 1);
     const int64_t i0 = base + 4 * q;
-    if constexpr (!kVbuf) {
+    if constexpr (kWriteV) {
       uint32_t code[4];
       al_codes<(int)LM2, 4>(vn, f, code, KR);
       if constexpr (VB == 8) {
@@ -948,7 +955,7 @@ __global__ __launch_bounds__(kLanes) void k_update1d_gen(Desc1D one, const Desc1
     }
   }
   __syncthreads();   // every lane has read the old block metadata
-  if (!kVbuf && lane == 0) { gp(D.v_scale)[blk] = f.s; gp(D.v_min_log)[blk] = f.lmin; }
+  if (kWriteV && lane == 0) { gp(D.v_scale)[blk] = f.s; gp(D.v_min_log)[blk] = f.lmin; }
   if constexpr (kSegM) {
     if (nseg == 1) {
       for (int i = lane; i < mpb; i += kLanes)
@@ -958,6 +965,8 @@ __global__ __launch_bounds__(kLanes) void k_update1d_gen(Desc1D one, const Desc1
 }
 
 // ------------------------------------------------------------ launch glue
+// Modes that sum squares (NORM, LAG, MNORM, SUM, MSUM).
+static bool is_norm_mode(int m) { return m == 1 || m == 3 || m == 4 || m == 5 || m == 7; }
 static bool fast_shape_ok(int bv, int bm) {
   auto pow2 = [](int x) { return x > 0 && (x & (x - 1)) == 0; };
   return pow2(bv) && bv >= 128 && bv <= 2048 && pow2(bm) && bm >= 32 && bm <= bv;
@@ -1001,18 +1010,28 @@ template <typename T, bool SR, int MK, int KR>
 static int launch_mode(int vbits, int mode, const Desc1D& one, const Desc1D* table, int ntab,
                        int64_t nwg, const Hyper1D& h, hipStream_t st) {
 #define A8_L(VB, MO) return launch_t<T, VB, MO, SR, MK, KR>(one, table, ntab, nwg, h, st)
-  if (mode == 4) {
+  if (mode == 4 || mode == 7) {
     if constexpr (MK == 0 || SR) {
       return set_error(A8_ERR_ARG, "MNORM needs momentum codes");
     } else {
-      if (vbits == 8) A8_L(8, 4);
-      A8_L(16, 4);
+      if (mode == 4) { if (vbits == 8) A8_L(8, 4); A8_L(16, 4); }
+      if (vbits == 8) A8_L(8, 7);
+      A8_L(16, 7);
+    }
+  }
+  if (mode == 1 || mode == 5) {   // no parameter is written: one form for SR and not
+    if constexpr (SR) {
+      return set_error(A8_ERR_ARG, "a norm pass does not round");
+    } else {
+      if (mode == 1) { if (vbits == 8) A8_L(8, 1); A8_L(16, 1); }
+      if (vbits == 8) A8_L(8, 5);
+      A8_L(16, 5);
     }
   }
   if (vbits == 8) {
-    switch (mode) { case 0: A8_L(8, 0); case 1: A8_L(8, 1); case 2: A8_L(8, 2); default: A8_L(8, 3); }
+    switch (mode) { case 0: A8_L(8, 0); case 2: A8_L(8, 2); case 6: A8_L(8, 6); default: A8_L(8, 3); }
   } else {
-    switch (mode) { case 0: A8_L(16, 0); case 1: A8_L(16, 1); case 2: A8_L(16, 2); default: A8_L(16, 3); }
+    switch (mode) { case 0: A8_L(16, 0); case 2: A8_L(16, 2); case 6: A8_L(16, 6); default: A8_L(16, 3); }
   }
 #undef A8_L
 }
@@ -1028,32 +1047,32 @@ static int launch_dispatch(int vbits, int mode, const Desc1D& one, const Desc1D*
 }
 
 // Every instantiation of one AL rule (KR = 0: the CPU quantiser's, 1: the reference
-// kernels') for 32- and 64-bit parameters (WIDE) or for 16-bit ones; each has a
+// kernels') for 32- and 64-bit parameters (KIND 0), bf16 (1) or fp16 (2); each has a
 // translation unit of its own, so that they compile in parallel.
-template <int KR, bool WIDE>
+template <int KR, int KIND>
 static int launch_rule(int dtype, int sr, int vbits, int mode, const Desc1D& one, const Desc1D* table,
                        int ntab, int64_t nwg, const Hyper1D& h, hipStream_t st) {
-  if ((mode == 1 || mode == 4) && sr) sr = 0;
-  if constexpr (WIDE) {
+  if (is_norm_mode(mode) && mode != 3) sr = 0;
+  if constexpr (KIND == 0) {
     if (dtype == A8_F32) return launch_dispatch<float, false, KR>(vbits, mode, one, table, ntab, nwg, h, st);
     if (dtype == A8_F64) return launch_dispatch<double, false, KR>(vbits, mode, one, table, ntab, nwg, h, st);
   } else {
-    if (dtype == A8_BF16)
-      return sr ? launch_dispatch<__hip_bfloat16, true, KR>(vbits, mode, one, table, ntab, nwg, h, st)
-                : launch_dispatch<__hip_bfloat16, false, KR>(vbits, mode, one, table, ntab, nwg, h, st);
-    if (dtype == A8_F16)
-      return sr ? launch_dispatch<__half, true, KR>(vbits, mode, one, table, ntab, nwg, h, st)
-                : launch_dispatch<__half, false, KR>(vbits, mode, one, table, ntab, nwg, h, st);
+    using T = std::conditional_t<KIND == 1, __hip_bfloat16, __half>;
+    return sr ? launch_dispatch<T, true, KR>(vbits, mode, one, table, ntab, nwg, h, st)
+              : launch_dispatch<T, false, KR>(vbits, mode, one, table, ntab, nwg, h, st);
   }
   return set_error(A8_ERR_DTYPE, "unsupported param dtype");
 }
 
-// 16-bit parameters, KR = 0 (a8_update1d_h.hip); KR = 1 (a8_update1d_k.hip, a8_update1d_kh.hip).
-int launch_any_16bit(int dtype, int sr, int vbits, int mode, const Desc1D& one, const Desc1D* table,
-                     int ntab, int64_t nwg, const Hyper1D& h, hipStream_t st);
-int launch_any_kernel_rule(int dtype, int sr, int vbits, int mode, const Desc1D& one, const Desc1D* table,
-                           int ntab, int64_t nwg, const Hyper1D& h, hipStream_t st);
-int launch_any_kernel_rule_16bit(int dtype, int sr, int vbits, int mode, const Desc1D& one, const Desc1D* table,
-                                 int ntab, int64_t nwg, const Hyper1D& h, hipStream_t st);
+// The other translation units: bf16 and fp16 (a8_update1d_b.hip, a8_update1d_h.hip), and
+// KR = 1 (a8_update1d_k.hip, a8_update1d_kb.hip, a8_update1d_kh.hip).
+#define A8_UNIT(NAME)                                                                                       \
+  int NAME(int dtype, int sr, int vbits, int mode, const Desc1D& one, const Desc1D* table, int ntab, int64_t nwg, \
+           const Hyper1D& h, hipStream_t st)
+A8_UNIT(launch_1d_b);
+A8_UNIT(launch_1d_h);
+A8_UNIT(launch_1d_k);
+A8_UNIT(launch_1d_kb);
+A8_UNIT(launch_1d_kh);
 
 }  // namespace a8

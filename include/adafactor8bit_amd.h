@@ -71,6 +71,11 @@ extern "C" {
  * reads v_buf, clips U by sqrt(*prev_norm) (the NORM pass's sum of U^2) and
  * accumulates sum(M'^2) into norm_buf; writes no state. */
 #define A8_MODE_MNORM 4
+/* NORM, APPLY and MNORM without v_buf: SUM and MSUM write no state, so APPLYC forms
+ * V' from the same codes and re-encodes V and M in its one pass. */
+#define A8_MODE_SUM 5
+#define A8_MODE_APPLYC 6
+#define A8_MODE_MSUM 7
 
 const char* a8_last_error(void);
 const char* a8_version(void);
@@ -90,12 +95,12 @@ int a8_set_qmap(const float* qmap8_host, const float* qmap4_host);
  *   v_q         AL8 uint8 / AL16 int16 codes padded to block_size; v_scale,
  *               v_min_log fp32 per block
  *   v_buf       fp32[numel] exact V written by NORM, read by APPLY
- *   norm_buf    fp32[1] sum of squares accumulated by NORM/LAG, read by APPLY
- *   norm_parts  NORM/LAG/MNORM: a8_norm_parts_1d(numel, block_size, m_block_size)
+ *   norm_buf    fp32[1] sum of squares accumulated by NORM/SUM/LAG, read by APPLY/APPLYC
+ *   norm_parts  NORM/SUM/LAG/MNORM/MSUM: a8_norm_parts_1d(numel, block_size, m_block_size)
  *               doubles of workspace.  The pass writes one partial sum per workgroup
  *               there and a second launch adds them in index order to norm_buf, so
  *               the sum has the same bits run to run (the reference adds with float
- *               atomics, kernels.cu:297-316); NULL is allowed for modes 0 and 2
+ *               atomics, kernels.cu:297-316); NULL is allowed for modes 0, 2 and 6
  *   alpha, prev_norm, decay: device fp32 scalars; alpha == NULL uses alpha_val,
  *               decay == NULL uses decay_val when has_decay (p := p*decay before
  *               the update, the decoupled weight decay of optimizer.py:2034-2039)
