@@ -143,6 +143,7 @@ _SIGS = {
                                 _c_i, _c_i, _c_d, _c_i, _c_i, _c_i, _c_u64, _c_i, _c_d, _c_f, _c_i,
                                 _c_vp, _c_vp]),
     "a8_factored_workspace_floats": (_c_i64, [_c_i64, _c_i64, _c_i64]),
+    "a8_factored_group_workspace_floats": (_c_i64, [_c_i64, _c_i64, _c_i64, _c_i64]),
     "a8_table_bytes_2d": (_c_i64, [_c_i]),
     "a8_apollo_step": (_c_i, [_c_i, _c_i, ctypes.POINTER(ApolloTensor), _c_i, _c_i, _c_d, _c_d, _c_i, _c_f,
                               _c_f, _c_i, _c_i, _c_i, _c_i, _c_i, _c_i, _c_i, _c_f, _c_i, _c_i, _c_f, _c_f,

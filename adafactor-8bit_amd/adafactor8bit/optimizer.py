@@ -1976,12 +1976,12 @@ def _run_factored(opt, plans):
     ent = wsd.get(tkey)
     upload = 0
     if ent is None or ent["sig"] != sig:
-        sizes = []
+        sizes, total = [], sum(pl.g.numel() for pl in plans)
         for pl in plans:
             sh = pl.g.shape
             R, C = int(sh[-2]), int(sh[-1])
             B = pl.g.numel() // (R * C)
-            sizes.append((B, R, C, int(L.a8_factored_workspace_floats(B, R, C))))
+            sizes.append((B, R, C, int(L.a8_factored_group_workspace_floats(B, R, C, total))))
         offs, tot = [], 0
         for (_, _, _, w) in sizes:
             offs.append(tot)

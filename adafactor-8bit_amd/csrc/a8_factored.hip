@@ -79,15 +79,26 @@ struct FWs {
 constexpr int kTRS = A8_TRS;
 constexpr int kSplit = 32;
 
-__host__ __device__ inline int64_t fws_tile_rows(int64_t R) {
-  const int64_t r = (R + kTR - 1) / kTR * kTR;
-  return r < kTRS ? r : kTRS;
+// Rows of the statistics tiles of a group of `total` elements: the tallest tiles that
+// still make about 2048 of them, eight workgroups for each of the 256 CUs.  256 rows from
+// 512 M elements on; a 44 M-parameter layer had 176 tiles of 256 rows, less than one
+// workgroup per CU, and takes 32 (k_fstats 64 -> 21 us, k_came1 144 -> 38).
+static int64_t group_tile_rows(int64_t total) {
+  int64_t tr = kTR;
+  while (tr < kTRS && tr * kTC * 2048 < total) tr *= 2;
+  return tr;
 }
 
-__host__ __device__ inline FWs fws_layout(int64_t B, int64_t R, int64_t C) {
+// A tensor's tile rows in such a group.
+static int64_t fws_tile_rows(int64_t R, int64_t group_rows) {
+  const int64_t r = (R + kTR - 1) / kTR * kTR;
+  return r < group_rows ? r : group_rows;
+}
+
+__host__ __device__ inline FWs fws_layout(int64_t B, int64_t R, int64_t C, int64_t tr) {
   FWs w;
   w.nchunk = (C + kTC - 1) / kTC;
-  w.tr = fws_tile_rows(R);
+  w.tr = tr;
   w.nstrip = (R + w.tr - 1) / w.tr;
   w.ntile = B * w.nstrip * w.nchunk;
   w.nustrip = (R + kTR - 1) / kTR;
@@ -148,7 +159,8 @@ struct DescF {
   uint64_t sr_seed;
   int has_fira_prev;
   int vec4;            // every row starts 16-byte aligned
-  int tiled;           // update runs on the statistics tiles (k_fupdt), else flat units
+  int tiled;           // update runs on tiles (k_fupdt), else flat units
+  int tr;              // rows per statistics tile
 };
 
 struct HyperF {
@@ -228,19 +240,21 @@ __device__ __forceinline__ double wg_sum_d(double x, double* s4) {
 
 __device__ __forceinline__ uint32_t nz_key_f(float v) { return __float_as_uint(v) - 1u; }
 
-__device__ __forceinline__ void wg_maxkey(float& mx, uint32_t& key, float* s8) {
+// Maximum and minimum key over a workgroup of up to 16 waves; s32: 32 floats of LDS.
+__device__ __forceinline__ void wg_maxkey(float& mx, uint32_t& key, float* s32) {
   mx = grp_max(mx, 64);
   key = grp_umin(key, 64);
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x, nw = (int)blockDim.x >> 6;
   __syncthreads();
   if ((lane & 63) == 0) {
-    s8[lane >> 6] = mx;
-    s8[4 + (lane >> 6)] = __uint_as_float(key);
+    s32[lane >> 6] = mx;
+    s32[16 + (lane >> 6)] = __uint_as_float(key);
   }
   __syncthreads();
-  mx = fmaxf(fmaxf(s8[0], s8[1]), fmaxf(s8[2], s8[3]));
-  key = min(min(__float_as_uint(s8[4]), __float_as_uint(s8[5])),
-            min(__float_as_uint(s8[6]), __float_as_uint(s8[7])));
+  for (int w = 0; w < nw; ++w) {
+    mx = fmaxf(mx, s32[w]);
+    key = min(key, __float_as_uint(s32[16 + w]));
+  }
 }
 
 // Four consecutive row elements starting at column c0 (zero beyond C).
@@ -436,7 +450,7 @@ __global__ __launch_bounds__(256) void k_fstats(const DescF* __restrict__ table,
   __shared__ double s_row[4 * kTRS];
   __shared__ double s4[4];
   const DescF D = *find_tile(table, ntab, (int64_t)blockIdx.x);
-  const FWs W = fws_layout(D.B, D.R, D.C);
+  const FWs W = fws_layout(D.B, D.R, D.C, D.tr);
   const TilePos q = tile_pos<false>(D, W);
   const int lane = threadIdx.x, wl = lane & 63;
   const int wave = __builtin_amdgcn_readfirstlane(lane >> 6);
@@ -620,7 +634,7 @@ template <typename T, int MK>
 __global__ __launch_bounds__(256) void k_came1(const DescF* __restrict__ table, int ntab, HyperF h) {
   __shared__ double s_row[4 * kTRS];
   const DescF D = *find_tile(table, ntab, (int64_t)blockIdx.x);
-  const FWs W = fws_layout(D.B, D.R, D.C);
+  const FWs W = fws_layout(D.B, D.R, D.C, D.tr);
   const TilePos q = tile_pos<false>(D, W);
   const int lane = threadIdx.x, wl = lane & 63;
   const int wave = __builtin_amdgcn_readfirstlane(lane >> 6);
@@ -652,14 +666,12 @@ __device__ __forceinline__ float fv_decode(const void* q, const float* sc, const
                                            int64_t bsz) {
   if constexpr (VB == 8) {
     const uint32_t c = gp(reinterpret_cast<const uint8_t*>(q))[i];
-    if (!c) return 0.0f;
     const int64_t bi = i / bsz;
-    return exp2_exact(((float)(c - 1) * gp(sc)[bi]) / 254.0f + gp(ml)[bi]);
+    return al_decode<254>(c, gp(sc)[bi], gp(ml)[bi], false);
   } else {
     const uint32_t c = gp(reinterpret_cast<const uint16_t*>(q))[i];
-    if (!c) return 0.0f;
     const int64_t bi = i / bsz;
-    return exp2_exact(((float)(c - 1) * gp(sc)[bi]) / 65534.0f + gp(ml)[bi]);
+    return al_decode<65534>(c, gp(sc)[bi], gp(ml)[bi], false);
   }
 }
 
@@ -678,7 +690,7 @@ __device__ __forceinline__ const DescF* find_cs(const DescF* tab, int n, int64_t
 // group sums in order.
 __global__ __launch_bounds__(256) void k_fcolsum(const DescF* __restrict__ table, int ntab) {
   const DescF D = *find_cs(table, ntab, (int64_t)blockIdx.x);
-  const FWs W = fws_layout(D.B, D.R, D.C);
+  const FWs W = fws_layout(D.B, D.R, D.C, D.tr);
   if (W.nsplit <= 1) return;
   const int64_t C = D.C;
   const int64_t ncg = (C + 255) / 256;
@@ -723,11 +735,12 @@ __device__ __forceinline__ const DescF* find_fblk(const DescF* tab, int n, int64
 // 951-953).  VB is the state's codec (8 / 16 bits, 0 = fp32 state, blocks of the
 // same size only partition the work).
 template <int VB, bool CONF>
-__global__ __launch_bounds__(256) void k_fblock(const DescF* __restrict__ table, int ntab, HyperF h) {
+__global__ __launch_bounds__(1024) void k_fblock(const DescF* __restrict__ table, int ntab, HyperF h) {
   hf_step(h);
-  __shared__ float sf[8];
+  __shared__ float sf[32];
+  const int nl = (int)blockDim.x;
   const DescF D = *find_fblk(table, ntab, (int64_t)blockIdx.x);
-  const FWs W = fws_layout(D.B, D.R, D.C);
+  const FWs W = fws_layout(D.B, D.R, D.C, D.tr);
   const int64_t lb = (int64_t)blockIdx.x - D.fblk_begin;
   const bool is_row = lb < D.nbr;
   const int64_t bi = is_row ? lb : lb - D.nbr;
@@ -760,10 +773,19 @@ __global__ __launch_bounds__(256) void k_fblock(const DescF* __restrict__ table,
   // 1. means and EMA (each lane keeps its own entries for step 2)
   float mx = 0.0f;
   uint32_t key = 0xFFFFFFFFu;
-  for (int64_t i = i0 + lane; i < i1; i += 256) {
+  for (int64_t i = i0 + lane; i < i1; i += nl) {
     double sum = 0.0;
     if (is_row) {
-      for (int64_t k = 0; k < W.nchunk; ++k) sum += gp(ws_dp(ws, W.rowpart))[k * n + i];
+      const double* rp = ws_dp(ws, W.rowpart) + i;
+      int64_t k = 0;
+      for (; k + 4 <= W.nchunk; k += 4) {   // loads in flight, summed in order
+        double t[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) t[u] = gp(rp)[(k + u) * n];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) sum += t[u];
+      }
+      for (; k < W.nchunk; ++k) sum += gp(rp)[k * n];
     } else {
       // the column's strip partials, or k_fcolsum's sums of kSplit strips each
       const int64_t b = i / C, c = i - b * C;
@@ -800,10 +822,11 @@ __global__ __launch_bounds__(256) void k_fblock(const DescF* __restrict__ table,
     wg_maxkey(mx, key, sf);
     const float mnz = (key == 0xFFFFFFFFu) ? __builtin_inff() : __uint_as_float(key + 1u);
     const ALFit f = al_refit(mx, mnz, h.floor_, (float)LM2);
-    for (int64_t k = lane; k < bsz; k += 256) {
+    for (int64_t k = lane; k < bsz; k += nl) {
       const int64_t i = i0 + k;
       const float v = i < n ? gp(vec)[i] : 0.0f;
-      const uint32_t code = al_finish<LM2>(v, al_round_exact<LM2>(v, f));
+      uint32_t code;
+      al_codes<LM2, 1>(&v, f, &code);
       if constexpr (VB == 8) gp(reinterpret_cast<uint8_t*>(q))[i] = (uint8_t)code;
       else gp(reinterpret_cast<uint16_t*>(q))[i] = (uint16_t)code;
       if (!is_row && i < n) gp(vec)[i] = 1.0f / sqrtf(v);
@@ -821,7 +844,7 @@ __global__ __launch_bounds__(256) void k_frows(const DescF* __restrict__ table, 
   hf_step(h);
   __shared__ double sd[4];
   const DescF D = table[blockIdx.x];
-  const FWs W = fws_layout(D.B, D.R, D.C);
+  const FWs W = fws_layout(D.B, D.R, D.C, D.tr);
   const int lane = threadIdx.x;
   const int64_t B = D.B, R = D.R;
   float* ws = D.ws;
@@ -891,7 +914,7 @@ __global__ __launch_bounds__(256) void k_fupdate(const DescF* __restrict__ table
   constexpr bool kHasM = MK != 0;
   const DescF D = *find_unit(table, ntab, (int64_t)blockIdx.x);
   if (D.tiled) return;   // updated by k_fupdt
-  const FWs W = fws_layout(D.B, D.R, D.C);
+  const FWs W = fws_layout(D.B, D.R, D.C, D.tr);
   const int64_t wl = (int64_t)blockIdx.x - D.unit_begin;
   const int lane = threadIdx.x;
   const int64_t n = D.numel;
@@ -1090,7 +1113,7 @@ __global__ __launch_bounds__(256) void k_fupdate_gen(const DescF* __restrict__ t
   __shared__ double s4d[4];
   const DescF D = *find_unit(table, ntab, (int64_t)blockIdx.x);
   if (D.tiled) return;
-  const FWs W = fws_layout(D.B, D.R, D.C);
+  const FWs W = fws_layout(D.B, D.R, D.C, D.tr);
   const int lane = threadIdx.x;
   const int BM = h.bm, U = h.unit, mpu = U / BM;
   const int64_t wl = (int64_t)blockIdx.x - D.unit_begin;
@@ -1276,7 +1299,7 @@ __global__ __launch_bounds__(256) void k_fupdt(const DescF* __restrict__ table, 
   constexpr bool kHasM = MK != 0;
   const DescF D = *find_utile(table, ntab, (int64_t)blockIdx.x);
   if (!D.tiled) return;   // updated by k_fupdate
-  const FWs W = fws_layout(D.B, D.R, D.C);
+  const FWs W = fws_layout(D.B, D.R, D.C, D.tr);
   const TilePos q = tile_pos<true>(D, W);
   const int64_t R = D.R, C = D.C, b = q.b, c_base = q.c_base;
   const int lane = threadIdx.x, wl = lane & 63;
@@ -1494,7 +1517,7 @@ __global__ __launch_bounds__(256) void k_fupdt(const DescF* __restrict__ table, 
 __global__ __launch_bounds__(256) void k_fnorm(const DescF* __restrict__ table, HyperF h) {
   __shared__ double sd[4];
   const DescF D = table[blockIdx.x];
-  const FWs W = fws_layout(D.B, D.R, D.C);
+  const FWs W = fws_layout(D.B, D.R, D.C, D.tr);
   float* ws = D.ws;
   double s = 0.0;
   const int64_t np = D.tiled ? W.nutile : W.nunit;
@@ -1532,7 +1555,7 @@ __global__ __launch_bounds__(256) void k_fnorm(const DescF* __restrict__ table, 
 __global__ __launch_bounds__(256) void k_fclip(const DescF* __restrict__ table, HyperF h) {
   __shared__ double sd[4];
   const DescF D = table[blockIdx.x];
-  const FWs W = fws_layout(D.B, D.R, D.C);
+  const FWs W = fws_layout(D.B, D.R, D.C, D.tr);
   float* ws = D.ws;
   double s = 0.0;
   const int64_t np = D.tiled ? W.nutile : W.nunit;
@@ -1627,11 +1650,11 @@ static int launch_colsum(const DescF* tab, int ntab, int64_t ncs, hipStream_t st
 template <bool CONF>
 static int launch_finish(int bits, const DescF* tab, int ntab, int64_t nfblk, const HyperF& h,
                          hipStream_t st) {
-  const dim3 g((unsigned)nfblk), b(256);
+  const dim3 g((unsigned)nfblk), b(256), bb(h.block_size >= 1024 ? 1024 : 256);
   switch (bits) {
-    case 8: hipLaunchKernelGGL((k_fblock<8, CONF>), g, b, 0, st, tab, ntab, h); break;
-    case 16: hipLaunchKernelGGL((k_fblock<16, CONF>), g, b, 0, st, tab, ntab, h); break;
-    default: hipLaunchKernelGGL((k_fblock<0, CONF>), g, b, 0, st, tab, ntab, h); break;
+    case 8: hipLaunchKernelGGL((k_fblock<8, CONF>), g, bb, 0, st, tab, ntab, h); break;
+    case 16: hipLaunchKernelGGL((k_fblock<16, CONF>), g, bb, 0, st, tab, ntab, h); break;
+    default: hipLaunchKernelGGL((k_fblock<0, CONF>), g, bb, 0, st, tab, ntab, h); break;
   }
   int rc = check_launch("k_fblock");
   if (rc) return rc;
@@ -1687,8 +1710,12 @@ using namespace a8;
 extern "C" {
 
 int64_t a8_factored_workspace_floats(int64_t batch, int64_t rows, int64_t cols) {
+  return a8_factored_group_workspace_floats(batch, rows, cols, batch * rows * cols);
+}
+
+int64_t a8_factored_group_workspace_floats(int64_t batch, int64_t rows, int64_t cols, int64_t total) {
   if (batch <= 0 || rows <= 0 || cols <= 0) return 0;
-  return fws_layout(batch, rows, cols).total;
+  return fws_layout(batch, rows, cols, fws_tile_rows(rows, group_tile_rows(total))).total;
 }
 
 int64_t a8_table_bytes_2d(int ntensors) { return (int64_t)sizeof(DescF) * (int64_t)ntensors; }
@@ -1731,6 +1758,9 @@ int a8_factored_step(int dtype, int stochastic, const a8_tensor2d* tensors, int 
   int64_t tiles = 0, utiles = 0, units = 0, fblks = 0, csw = 0;
   bool any_tiled = false, any_flat = false;
   const size_t esz = dtype == A8_F32 ? 4 : (dtype == A8_F64 ? 8 : 2);
+  int64_t total = 0;
+  for (int i = 0; i < ntensors; ++i) total += tensors[i].batch * tensors[i].rows * tensors[i].cols;
+  const int64_t group_rows = group_tile_rows(total);
   for (int i = 0; i < ntensors; ++i) {
     const a8_tensor2d& t = tensors[i];
     if (t.batch <= 0 || t.rows <= 0 || t.cols <= 0) return set_error(A8_ERR_SIZE, "empty factored tensor");
@@ -1763,7 +1793,8 @@ int a8_factored_step(int dtype, int stochastic, const a8_tensor2d* tensors, int 
     D.tiled = (t.cols % 4 == 0) &&
               (!has_m || m32 || (lbm >= 0 && m_block_size <= 256 && t.cols % m_block_size == 0)) ? 1 : 0;
     (D.tiled ? any_tiled : any_flat) = true;
-    const FWs W = fws_layout(t.batch, t.rows, t.cols);
+    D.tr = (int)fws_tile_rows(t.rows, group_rows);
+    const FWs W = fws_layout(t.batch, t.rows, t.cols, D.tr);
     D.tile_begin = tiles;
     D.utile_begin = utiles;
     D.unit_begin = units;
