@@ -85,9 +85,10 @@ __device__ __forceinline__ float lerp_u(float s, float e, LerpW L) {
 // the correctly rounded reciprocal and q0 within an ulp of x / d, so the
 // remainder x - q0 d is exact in one fma and q0 + r rd rounds to the correctly
 // rounded quotient).  The theorem needs quotient and remainder in the normal
-// range: when any lane holds a value with |q0| < 2^-100, zero or non-finite, the
-// wave redoes those elements with the IEEE division (a uniform branch, so the
-// division is not executed otherwise).  Three operations in place of ten.
+// range: a zero is its own quotient (gradients hold zeros), and when any lane holds
+// another value with |q0| < 2^-100 or a non-finite one, the wave redoes those
+// elements with the IEEE division (a uniform branch, so the division is not
+// executed otherwise).  Five operations in place of ten.
 __device__ __forceinline__ bool div_fast_ok(float q0) {
   const float a = fabsf(q0);
   return a >= 0x1p-100f && a <= 0x1.fffffep127f;   // false for NaN
@@ -100,13 +101,14 @@ __device__ __forceinline__ void div_by(float* q, const float* x, float d, float 
   for (int i = 0; i < N; ++i) {
     const float q0 = x[i] * rd;
     const float r = __builtin_fmaf(-q0, d, x[i]);
-    q[i] = __builtin_fmaf(r, rd, q0);
-    bad = bad || !div_fast_ok(q0);
+    const bool odd = !div_fast_ok(q0);
+    q[i] = odd ? q0 : __builtin_fmaf(r, rd, q0);
+    bad = bad || (odd && x[i] != 0.0f);
   }
   if (__builtin_amdgcn_ballot_w64(bad)) {
 #pragma unroll
     for (int i = 0; i < N; ++i)
-      if (!div_fast_ok(x[i] * rd)) q[i] = x[i] / d;
+      if (!div_fast_ok(x[i] * rd) && x[i] != 0.0f) q[i] = x[i] / d;
   }
 }
 

@@ -158,8 +158,7 @@ struct DescF {
   int64_t nbr;         // AL blocks of the row vector (the column vector follows)
   uint64_t sr_seed;
   int has_fira_prev;
-  int vec4;            // every row starts 16-byte aligned
-  int tiled;           // update runs on tiles (k_fupdt), else flat units
+  int tiled;           // update runs on tiles (k_fupdt; 2: C % 4 != 0), 0: flat units
   int tr;              // rows per statistics tile
 };
 
@@ -257,28 +256,6 @@ __device__ __forceinline__ void wg_maxkey(float& mx, uint32_t& key, float* s32) 
   }
 }
 
-// Four consecutive row elements starting at column c0 (zero beyond C).
-template <typename T, typename V>
-__device__ __forceinline__ void load4(const T* base, int64_t rowbase, int64_t c0, int64_t C, bool vec,
-                                      V* out) {
-  if (vec && c0 + 4 <= C) {
-    if constexpr (sizeof(T) == 8) {
-      ld4d<V>(reinterpret_cast<const double*>(base) + rowbase + c0, out);
-    } else if constexpr (sizeof(T) == 4) {
-      const f32x4 a = *gp(reinterpret_cast<const f32x4*>(base + rowbase + c0));
-      out[0] = a.x; out[1] = a.y; out[2] = a.z; out[3] = a.w;
-    } else {
-      const u32x2 a = *gp(reinterpret_cast<const u32x2*>(base + rowbase + c0));
-      const T* h = reinterpret_cast<const T*>(&a);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) out[k] = to_f<T>(h[k]);
-    }
-  } else {
-#pragma unroll
-    for (int k = 0; k < 4; ++k) out[k] = (c0 + k < C) ? ld1<T, V>(base, rowbase + c0 + k) : (V)0;
-  }
-}
-
 // ------------------------------------------------------------ statistics
 // Tile layout of the two statistics kernels (k_fstats, k_came1): wave w of the
 // workgroup owns columns c_base + 256 w .. + 255 of every row of the tile, a lane
@@ -328,19 +305,61 @@ __device__ __forceinline__ const char* at_off(const T* row, uint32_t off) {
   return reinterpret_cast<const char*>(((uint64_t)hi << 32) | lo) + (off * (uint32_t)sizeof(T));
 }
 
+// The types say what alignment the address has: a row of a tensor whose column count is
+// no multiple of the vector starts on any element, and global loads need no more (one
+// instruction all the same; a lane that straddles a cache line costs a second request).
+typedef f32x4 f32x4_e __attribute__((aligned(4)));
+typedef u32x2 u32x2_e __attribute__((aligned(2)));
+typedef uint32_t u32_e __attribute__((aligned(1)));
+typedef f64x2 f64x2_e __attribute__((aligned(8)));
+
 template <typename T, typename V>
 __device__ __forceinline__ void load4o(const T* row, uint32_t off, V* out) {
   if constexpr (sizeof(T) == 8) {
-    ld4d<V>(reinterpret_cast<const double*>(at_off(row, off)), out);
+    const A8_G f64x2_e* p = ((const A8_G f64x2_e*)(at_off(row, off)));
+    const f64x2 a = __builtin_nontemporal_load(p), b = __builtin_nontemporal_load(p + 1);
+    out[0] = (V)a.x; out[1] = (V)a.y; out[2] = (V)b.x; out[3] = (V)b.y;
   } else if constexpr (sizeof(T) == 4) {
-    const f32x4 a = __builtin_nontemporal_load(gp(reinterpret_cast<const f32x4*>(at_off(row, off))));
+    const f32x4 a = __builtin_nontemporal_load(((const A8_G f32x4_e*)(at_off(row, off))));
     out[0] = a.x; out[1] = a.y; out[2] = a.z; out[3] = a.w;
   } else {
-    const u32x2 a = __builtin_nontemporal_load(gp(reinterpret_cast<const u32x2*>(at_off(row, off))));
+    const u32x2 a = __builtin_nontemporal_load(((const A8_G u32x2_e*)(at_off(row, off))));
     const T* h = reinterpret_cast<const T*>(&a);
 #pragma unroll
     for (int k = 0; k < 4; ++k) out[k] = to_f<T>(h[k]);
   }
+}
+
+// A lane's window of four columns in a row of C (a multiple of 4 or not, C >= 4).  The
+// window that C cuts loads the row's last four elements instead and moves its own to the
+// front (win_fix), zeros behind them, so every load is a full one inside the row.
+struct Win {
+  uint32_t cl;   // column the load starts at
+  int n;         // columns of the window inside C (0: none, the load reads the base column)
+};
+__device__ __forceinline__ Win win_at(int64_t c0, int64_t C, int64_t base) {
+  Win w;
+  w.n = c0 >= C ? 0 : (C - c0 >= 4 ? 4 : (int)(C - c0));
+  // an empty window reads the base column's window, itself moved left when C cuts it
+  const int64_t c = w.n > 0 ? c0 : base;
+  w.cl = (uint32_t)(c + 4 <= C ? c : C - 4);
+  return w;
+}
+// cut: the columns a cut window keeps, C % 4 (uniform)
+template <typename V>
+__device__ __forceinline__ void win_fix(const Win& w, int cut, V* v) {
+  V t[4] = {v[3], (V)0, (V)0, (V)0};
+  if (cut == 2) { t[0] = v[2]; t[1] = v[3]; }
+  if (cut == 3) { t[0] = v[1]; t[1] = v[2]; t[2] = v[3]; }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) v[k] = (w.n & 3) ? t[k] : v[k];
+}
+
+// A window of a matrix of fewer than four columns, element by element.
+template <typename T, typename V>
+__device__ __forceinline__ void load_tiny(const T* row, int64_t c0, int64_t C, V* out) {
+#pragma unroll
+  for (int k = 0; k < 4; ++k) out[k] = (c0 + k < C) ? ld1<T, V>(row, c0 + k) : (V)0;
 }
 
 // Where a statistics workgroup sits: tensor-local tile t, chunk, strip, batch.
@@ -375,15 +394,17 @@ __device__ __forceinline__ void tile_rows_out(const double* s_row, double* rowpa
   }
 }
 
-template <typename T, bool PSQ, bool RAGGED>
-__device__ __forceinline__ void fstats_tile(const DescF& D, const TilePos& q, int64_t c0, bool act, double* acc,
+// CUT: C cuts one of the wave's windows (C % 4 columns remain of it).  TINY: C < 4.
+template <typename T, bool PSQ, bool CUT, bool TINY>
+__device__ __forceinline__ void fstats_tile(const DescF& D, const TilePos& q, int64_t c0, double* acc,
                                             double& psq, double* s_row) {
   const T* G = reinterpret_cast<const T*>(D.grad);
   const T* P = reinterpret_cast<const T*>(D.param);
   const int64_t R = D.R, C = D.C;
   const int wl = threadIdx.x & 63;
-  const uint32_t cl = act ? (uint32_t)c0 : 0u;
-  const bool vec = D.vec4 != 0;
+  const Win w = win_at(c0, C, 0);
+  const bool act = w.n > 0;
+  const int cut = (int)(C & 3);
   float g[kRB][4], pv[kRB][PSQ ? 4 : 1];
   bool rv[kRB];
   auto issue = [&](int64_t r0) {
@@ -392,12 +413,12 @@ __device__ __forceinline__ void fstats_tile(const DescF& D, const TilePos& q, in
       const int64_t r = r0 + k;
       rv[k] = r < q.r_hi;
       const int64_t rowbase = (q.b * R + (rv[k] ? r : q.r_lo)) * C;
-      if constexpr (RAGGED) {
-        load4<T>(G, rowbase, c0, C, vec, g[k]);
-        if constexpr (PSQ) load4<T>(P, rowbase, c0, C, vec, pv[k]);
+      if constexpr (TINY) {
+        load_tiny<T>(G + rowbase, c0, C, g[k]);
+        if constexpr (PSQ) load_tiny<T>(P + rowbase, c0, C, pv[k]);
       } else {
-        load4o<T>(G + rowbase, cl, g[k]);
-        if constexpr (PSQ) load4o<T>(P + rowbase, cl, pv[k]);
+        load4o<T>(G + rowbase, w.cl, g[k]);
+        if constexpr (PSQ) load4o<T>(P + rowbase, w.cl, pv[k]);
       }
     }
   };
@@ -405,6 +426,10 @@ __device__ __forceinline__ void fstats_tile(const DescF& D, const TilePos& q, in
   auto consume = [&]() {
 #pragma unroll
     for (int k = 0; k < kRB; ++k) {
+      if constexpr (CUT) {
+        win_fix(w, cut, g[k]);
+        if constexpr (PSQ) win_fix(w, cut, pv[k]);
+      }
       const bool ok = rv[k] && act;
       double rk = 0.0;
 #pragma unroll
@@ -455,16 +480,16 @@ __global__ __launch_bounds__(256) void k_fstats(const DescF* __restrict__ table,
   const int lane = threadIdx.x, wl = lane & 63;
   const int wave = __builtin_amdgcn_readfirstlane(lane >> 6);
   const int64_t C = D.C;
-  const int64_t c0 = q.c_base + 256 * wave + 4 * wl;
-  const bool act = c0 < C;
+  const int64_t cw = q.c_base + 256 * wave, c0 = cw + 4 * wl;   // the wave's first column, the lane's
   double acc[4] = {0.0, 0.0, 0.0, 0.0};
   double psq = 0.0;
   double* srow = s_row + kTRS * wave;
-  if (q.c_base + 256 * wave >= C) {   // the wave's columns lie beyond C
+  if (cw >= C) {   // the wave's columns lie beyond C
     for (int i = wl; i < kTRS; i += 64) srow[i] = 0.0;
   }
-  else if ((C & 3) == 0) fstats_tile<T, PSQ, false>(D, q, c0, act, acc, psq, srow);
-  else fstats_tile<T, PSQ, true>(D, q, c0, act, acc, psq, srow);
+  else if (C < 4) fstats_tile<T, PSQ, false, true>(D, q, c0, acc, psq, srow);
+  else if ((C & 3) == 0 || cw + 256 <= C) fstats_tile<T, PSQ, false, false>(D, q, c0, acc, psq, srow);
+  else fstats_tile<T, PSQ, true, false>(D, q, c0, acc, psq, srow);
   float* ws = D.ws;
   double* colp = ws_dp(ws, W.colpart) + (q.b * W.nstrip + q.s) * C;
 #pragma unroll
@@ -496,44 +521,31 @@ __device__ __forceinline__ float m_old_at(int mk, const uint8_t* mq, const float
   return m_decode(mk, q, ms);
 }
 
-// Old momentum of four consecutive elements e .. e+3 of one row (zero beyond
-// `avail`).  The vector form needs e % 4 == 0 (the four share an M block).
+// Old momentum of four consecutive elements e .. e+3 of one row (zero beyond `avail`).
 template <int MK>
 __device__ __forceinline__ void m_old4(int mkr, const uint8_t* mq, const float* msc, int64_t e, int64_t avail,
-                                       bool vec, int lbm, int bm, float* out) {
+                                       int lbm, int bm, float* out) {
   const int mk = MK == 1 ? 1 : mkr;
-  if (vec && avail >= 4) {
-    const float ms = gp(msc)[m_blk(e, lbm, bm)];
-    if (mk == 2 || mk == 4) {
-      const uint32_t w = *gp(reinterpret_cast<const uint16_t*>(mq + (e >> 1)));
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const uint32_t byte = (w >> (8 * (k >> 1))) & 0xFFu;
-        out[k] = m_decode(mk, (k & 1) ? (byte & 0x0Fu) : (byte >> 4), ms);
-      }
-    } else {
-      const uint32_t w = *gp(reinterpret_cast<const uint32_t*>(mq + e));
-#pragma unroll
-      for (int k = 0; k < 4; ++k) out[k] = m_decode(mk, (w >> (8 * k)) & 0xFFu, ms);
-    }
-  } else {
-#pragma unroll
-    for (int k = 0; k < 4; ++k) out[k] = (k < avail) ? m_old_at(mk, mq, msc, e + k, lbm, bm) : 0.0f;
-  }
+  for (int k = 0; k < 4; ++k) out[k] = (k < avail) ? m_old_at(mk, mq, msc, e + k, lbm, bm) : 0.0f;
 }
 
 // CAME pass 1 over the statistics tiles of one workgroup (layout of fstats_tile):
 // U = ((g * inv_row) * inv_col) / clip, M' = lerp(M, U, 1 - beta1),
 // res = (U - M')^2 + eps_came, row and column sums of res (optimizer.py:929-937).
-template <typename T, int MK, bool RAGGED>
+// RAGGED: C is no multiple of 4, so rows start anywhere and a window's codes may straddle
+// two M blocks.  TINY: C < 4.
+template <typename T, int MK, bool RAGGED, bool TINY>
 __device__ __forceinline__ void came1_tile(const DescF& D, const FWs& W, const TilePos& q, const HyperF& h,
-                                           int64_t c0, bool act, const float* icol, float clip, double* acc,
+                                           int64_t c0, const float* icol, float clip, double* acc,
                                            double* s_row) {
   const T* G = reinterpret_cast<const T*>(D.grad);
   const int64_t R = D.R, C = D.C;
   const int wl = threadIdx.x & 63;
-  const uint32_t cl = act ? (uint32_t)c0 : 0u;
-  const bool vec = D.vec4 != 0;
+  const Win w = win_at(c0, C, 0);
+  const uint32_t cl = w.cl;
+  const bool act = w.n > 0;
+  const int cut = (int)(C & 3);
   const float* ws = D.ws;
   const int mk = MK == 1 ? 1 : h.mk;
   const bool nib = (mk == 2 || mk == 4);
@@ -541,7 +553,8 @@ __device__ __forceinline__ void came1_tile(const DescF& D, const FWs& W, const T
   const float rclip = 1.0f / clip;
   float g[kRB][4], mo[kRB][4], ir[kRB];
   uint32_t qv[kRB];
-  float ms[kRB];
+  float ms[kRB], ms3[RAGGED ? kRB : 1];
+  int nf[RAGGED ? kRB : 1];   // elements of the window in its first M block
   bool rv[kRB];
   auto issue = [&](int64_t r0) {
 #pragma unroll
@@ -551,14 +564,31 @@ __device__ __forceinline__ void came1_tile(const DescF& D, const FWs& W, const T
       const int64_t rr = rv[k] ? r : q.r_lo;
       const int64_t rowbase = (q.b * R + rr) * C;
       ir[k] = cp(ws)[W.invr + q.b * R + rr];
-      if constexpr (RAGGED) {
-        load4<T>(G, rowbase, c0, C, vec, g[k]);
-        if constexpr (MK == 3) load4<float>(D.m, rowbase, c0, C, vec, mo[k]);
-        else m_old4<MK>(h.mk, D.m_q, D.m_scale, rowbase + c0, C - c0, vec, h.lbm, h.bm, mo[k]);
+      if constexpr (TINY) {
+        load_tiny<T>(G + rowbase, c0, C, g[k]);
+        if constexpr (MK == 3) load_tiny<float>(D.m + rowbase, c0, C, mo[k]);
+        else m_old4<MK>(h.mk, D.m_q, D.m_scale, rowbase + c0, C - c0, h.lbm, h.bm, mo[k]);
       } else {
         load4o<T>(G + rowbase, cl, g[k]);
         if constexpr (MK == 3) {
           load4o<float>(D.m + rowbase, cl, mo[k]);
+        } else if constexpr (RAGGED) {
+          // codes of elements e .. e + 3 from any e, and the scales of the first's and
+          // the last's M block
+          const int64_t e = rowbase + cl;
+          const int64_t b0 = m_blk(e, h.lbm, h.bm), b3 = m_blk(e + 3, h.lbm, h.bm);
+          ms[k] = gp(D.m_scale)[b0];
+          ms3[k] = gp(D.m_scale)[b3];
+          nf[k] = b3 == b0 ? 4 : (int)(b3 * (h.lbm >= 0 ? (int64_t)1 << h.lbm : (int64_t)h.bm) - e);
+          if (MK == 1 || !nib) {
+            qv[k] = *((const A8_G u32_e*)(D.m_q + e));
+          } else {   // five nibbles from byte e / 2 on, read inside the codes
+            const uint32_t lo16 = gp(D.m_q)[e >> 1] | ((uint32_t)gp(D.m_q)[(e >> 1) + 1] << 8);
+            const uint32_t w24 = lo16 | ((uint32_t)gp(D.m_q)[(e + 3) >> 1] << 16);
+            // nibbles in element order (the even element of a byte is its high nibble)
+            const uint32_t sw = ((w24 & 0x0F0F0Fu) << 4) | ((w24 >> 4) & 0x0F0F0Fu);
+            qv[k] = (e & 1) ? sw >> 4 : sw;
+          }
         } else {
           const int64_t e = rowbase + cl;
           ms[k] = gp(D.m_scale)[m_blk(e, h.lbm, h.bm)];
@@ -573,7 +603,11 @@ __device__ __forceinline__ void came1_tile(const DescF& D, const FWs& W, const T
     float mk4[kRB][4];
 #pragma unroll
     for (int k = 0; k < kRB; ++k) {
-      if constexpr (!RAGGED && MK != 3) {
+      if constexpr (RAGGED && !TINY && MK != 3) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          mk4[k][e] = m_decode(mk, nib ? (qv[k] >> (4 * e)) & 0xFu : (qv[k] >> (8 * e)) & 0xFFu, e < nf[k] ? ms[k] : ms3[k]);
+      } else if constexpr (!TINY && MK != 3) {
         if (MK == 1 || !nib) {
 #pragma unroll
           for (int e = 0; e < 4; ++e) mk4[k][e] = m_decode(mk, (qv[k] >> (8 * e)) & 0xFFu, ms[k]);
@@ -591,6 +625,10 @@ __device__ __forceinline__ void came1_tile(const DescF& D, const FWs& W, const T
     }
 #pragma unroll
     for (int k = 0; k < kRB; ++k) {
+      if constexpr (RAGGED && !TINY) {
+        win_fix(w, cut, g[k]);
+        win_fix(w, cut, mk4[k]);
+      }
       float xs[4], ug[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) xs[e] = (scrub(g[k][e]) * ir[k]) * icol[e];
@@ -598,7 +636,7 @@ __device__ __forceinline__ void came1_tile(const DescF& D, const FWs& W, const T
       double rk = 0.0;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const bool ok = rv[k] && (RAGGED ? c0 + e < C : act);
+        const bool ok = rv[k] && (RAGGED ? e < w.n : act);
         const float mn = lerp_u(mk4[k][e], ug[e], lw);
         const float dd = ug[e] - mn;
         const double res = ok ? (double)(dd * dd + h.eps_came) : 0.0;
@@ -640,7 +678,6 @@ __global__ __launch_bounds__(256) void k_came1(const DescF* __restrict__ table, 
   const int wave = __builtin_amdgcn_readfirstlane(lane >> 6);
   const int64_t C = D.C;
   const int64_t c0 = q.c_base + 256 * wave + 4 * wl;
-  const bool act = c0 < C;
   float* ws = D.ws;
   const float clip = cp(ws)[W.scal + 4];
   float icol[4];
@@ -651,8 +688,9 @@ __global__ __launch_bounds__(256) void k_came1(const DescF* __restrict__ table, 
   if (q.c_base + 256 * wave >= C) {   // the wave's columns lie beyond C
     for (int i = wl; i < kTRS; i += 64) srow[i] = 0.0;
   }
-  else if ((C & 3) == 0) came1_tile<T, MK, false>(D, W, q, h, c0, act, icol, clip, acc, srow);
-  else came1_tile<T, MK, true>(D, W, q, h, c0, act, icol, clip, acc, srow);
+  else if ((C & 3) == 0) came1_tile<T, MK, false, false>(D, W, q, h, c0, icol, clip, acc, srow);
+  else if (C < 4) came1_tile<T, MK, true, true>(D, W, q, h, c0, icol, clip, acc, srow);
+  else came1_tile<T, MK, true, false>(D, W, q, h, c0, icol, clip, acc, srow);
   double* colp = ws_dp(ws, W.colpart) + (q.b * W.nstrip + q.s) * C;
 #pragma unroll
   for (int e = 0; e < 4; ++e)
@@ -1009,17 +1047,16 @@ __global__ __launch_bounds__(256) void k_fupdate(const DescF* __restrict__ table
       }
       T* P = reinterpret_cast<T*>(D.param);
       if constexpr (SR) {
+        float p[8];
+        load8<T>(P, e0, n, p);
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-          if (k < cnt) {
-            const float pv = ld1<T>(P, e0 + k);
-            const T r = sr_round<T>((has_dec ? pv * dec : pv) - step * u[k], D.sr_seed, h.sr_step,
-                                    (uint64_t)(e0 + k));
-            uint16_t bits;
-            __builtin_memcpy(&bits, &r, 2);
-            gp(reinterpret_cast<uint16_t*>(P))[e0 + k] = bits;
-          }
-        }
+        for (int k = 0; k < 8; ++k) p[k] = (has_dec ? p[k] * dec : p[k]) - step * u[k];
+        const uint64_t z = sr_base(D.sr_seed, h.sr_step) + 0x9E3779B97F4A7C15ULL + (uint64_t)(wl * kUnit);
+        const SrUnit srs = sr_unit<kUnit>(z);
+        T* Pu = P + wl * kUnit;
+        const uint32_t i0 = (uint32_t)lane * 8u, in = (uint32_t)(n - wl * kUnit < kUnit ? n - wl * kUnit : kUnit);
+        sr_store4<T>(Pu, i0, in, p, z + i0, srs);
+        if (i0 + 4 < in) sr_store4<T>(Pu, i0 + 4, in, p + 4, z + i0 + 4, srs);
       } else {
         pval_t<T> p[8];
         load8<T>(P, e0, n, p);
@@ -1274,8 +1311,8 @@ __global__ __launch_bounds__(256) void k_fupdate_gen(const DescF* __restrict__ t
   }
 }
 
-// Tiled form of k_fupdate for tensors whose columns allow it (C % 4 == 0 and,
-// with momentum, B_M <= 256 dividing C): the statistics tiles (tr rows x 1024
+// Tiled form of k_fupdate for tensors whose columns allow it (C >= 4 and, with coded
+// momentum, B_M <= 256 dividing C): the statistics tiles (tr rows x 1024
 // columns), each wave walking rows, lanes holding 4 consecutive columns of each
 // 256-column chunk (1 KB-contiguous accesses).  The tile's inv_col (and CAME
 // inv_conf_col) are staged in LDS once, a row's inv_row arrives through a scalar
@@ -1290,7 +1327,33 @@ __device__ __forceinline__ void keep4(const V* v) {
   asm volatile("" ::"v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]));
 }
 
-template <typename T, int MODE, bool SR, int MK, bool CM>
+// Stores columns c0 .. c0 + 3 of a row of C (those inside it), from any element alignment.
+template <typename T, typename V>
+__device__ __forceinline__ void store4e(T* row, uint32_t c0, uint32_t C, const V* v) {
+  if (c0 + 4 <= C) {
+    if constexpr (sizeof(T) == 8) {
+      A8_G f64x2_e* p = ((A8_G f64x2_e*)(reinterpret_cast<double*>(row) + c0));
+      __builtin_nontemporal_store(f64x2{(double)v[0], (double)v[1]}, p);
+      __builtin_nontemporal_store(f64x2{(double)v[2], (double)v[3]}, p + 1);
+    } else if constexpr (sizeof(T) == 4) {
+      __builtin_nontemporal_store(f32x4{v[0], v[1], v[2], v[3]}, ((A8_G f32x4_e*)(row + c0)));
+    } else {
+      u32x2 a;
+      T* h = reinterpret_cast<T*>(&a);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) h[k] = from_f<T>(v[k]);
+      __builtin_nontemporal_store(a, ((A8_G u32x2_e*)(row + c0)));
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (c0 + k < C) st1<T, V>(row, c0 + k, v[k]);
+  }
+}
+
+// CUT: tensors whose column count is no multiple of 4 (a kernel of its own: its window
+// moves and partial stores would take the plain update from three waves a SIMD to two).
+template <typename T, int MODE, bool SR, int MK, bool CM, bool CUT>
 __global__ __launch_bounds__(256) void k_fupdt(const DescF* __restrict__ table, int ntab, HyperF h) {
   if constexpr (SR) hf_step(h);
   static_assert(!CM || MK != 0, "CAME needs momentum");
@@ -1298,7 +1361,8 @@ __global__ __launch_bounds__(256) void k_fupdt(const DescF* __restrict__ table, 
   __shared__ double s4d[4];
   constexpr bool kHasM = MK != 0;
   const DescF D = *find_utile(table, ntab, (int64_t)blockIdx.x);
-  if (!D.tiled) return;   // updated by k_fupdate
+  if (D.tiled != (CUT ? 2 : 1)) return;   // updated by another launch
+  static_assert(!CUT || MK == 0 || MK == 3, "coded momentum: whole M blocks per row");
   const FWs W = fws_layout(D.B, D.R, D.C, D.tr);
   const TilePos q = tile_pos<true>(D, W);
   const int64_t R = D.R, C = D.C, b = q.b, c_base = q.c_base;
@@ -1325,26 +1389,28 @@ __global__ __launch_bounds__(256) void k_fupdt(const DescF* __restrict__ table, 
     dec = cp(sl)[3];
   }
   const bool has_dec = h.wd_mode != 0;
+  const uint64_t sr_z = SR ? sr_base(D.sr_seed, h.sr_step) + 0x9E3779B97F4A7C15ULL : 0u;
   const T* G0 = reinterpret_cast<const T*>(D.grad);
   T* P0 = reinterpret_cast<T*>(D.param);
-  // A lane's four 4-column windows.  C % 4 == 0, so a window holds all four
-  // columns or none; one beyond C is pointed at the tile's first window (a valid
-  // address), computed on like the others and never stored.  Loads and their
-  // arithmetic are unconditional, so nothing is left in flight across rows.
-  uint32_t cl[4];
-  bool act[4];
+  // A lane's four 4-column windows (Win); one beyond C is pointed at the tile's first
+  // window (a valid address), computed on like the others and never stored.  Loads and
+  // their arithmetic are unconditional, so nothing is left in flight across rows.
+  const int cut = (int)(C & 3);                     // columns of the window that C cuts
+  Win win[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int64_t c0 = c_base + 256 * j + 4 * wl;
-    act[j] = c0 < C;
-    cl[j] = act[j] ? (uint32_t)c0 : (uint32_t)c_base;
+    if constexpr (CUT) win[j] = win_at(c0, C, c_base);
+    else win[j] = Win{c0 < C ? (uint32_t)c0 : (uint32_t)c_base, c0 < C ? 4 : 0};
   }
+
   // Rows r, r + 4, r + 8 and r + 12 in one pass for the plain update (the loads
   // of all four in flight together: 2.40 -> 2.33 ms at C2 against two rows); one
-  // row per pass with momentum (two rows measured slower there: 172 registers)
+  // row per pass with momentum (two rows measured slower there: 172 registers), two with
+  // stochastic rounding or cut windows (four: 112 registers and scalar spills)
   // and in the read-only norm pass, where registers are better spent on
   // occupancy.  A row beyond the tile reads the first one again and stores nothing.
-  constexpr int NRW = (kHasM || MODE == 1) ? 1 : 4;
+  constexpr int NRW = (kHasM || MODE == 1) ? 1 : ((SR || CUT) ? 2 : 4);
   double sq = 0.0;   // sum u^2 (MODE 1), accumulated in double
   for (int64_t r0 = q.r_lo + wave; r0 < q.r_hi; r0 += 4 * NRW) {
     int64_t rowb[NRW];
@@ -1363,16 +1429,17 @@ __global__ __launch_bounds__(256) void k_fupdt(const DescF* __restrict__ table, 
       icrw[rr] = CM ? cp(ws)[W.icr + b * R + r] : 0.0f;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const int64_t e = rowb[rr] + cl[j];
-        load4o<T>(G0 + rowb[rr], cl[j], gj[rr][j]);
+        const uint32_t cl = win[j].cl;
+        const int64_t e = rowb[rr] + cl;
+        load4o<T>(G0 + rowb[rr], cl, gj[rr][j]);
         if constexpr (MK == 3) {
-          load4o<float>(D.m + rowb[rr], cl[j], mfj[rr][j]);
+          load4o<float>(D.m + rowb[rr], cl, mfj[rr][j]);
         } else if constexpr (kHasM) {
           msj[rr][j] = gp(D.m_scale)[e >> lbm];
           if (MK == 1 || !(mk == 2 || mk == 4)) qj[rr][j] = *gp(reinterpret_cast<const uint32_t*>(D.m_q + e));
           else qj[rr][j] = *gp(reinterpret_cast<const uint16_t*>(D.m_q + (e >> 1)));
         }
-        if constexpr (MODE != 1 && !SR) load4o<T>(P0 + rowb[rr], cl[j], pj[rr][j]);
+        if constexpr (MODE != 1) load4o<T>(P0 + rowb[rr], cl, pj[rr][j]);
       }
     }
     __builtin_amdgcn_sched_barrier(0);   // every load of the pass is issued before its arithmetic
@@ -1381,9 +1448,14 @@ __global__ __launch_bounds__(256) void k_fupdt(const DescF* __restrict__ table, 
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int q0 = 256 * j + 4 * wl;
-      const int64_t e = rowb[rr] + cl[j];
+      const int64_t e = rowb[rr] + win[j].cl;
       const float ir = irw[rr], icrr = icrw[rr];
-      const bool st = rv[rr] && act[j];   // this window of this row is stored
+      const bool st = rv[rr] && win[j].n > 0;   // this window of this row is stored
+      if constexpr (CUT) {
+        win_fix(win[j], cut, gj[rr][j]);
+        if constexpr (MODE != 1) win_fix(win[j], cut, pj[rr][j]);
+        if constexpr (MK == 3) win_fix(win[j], cut, mfj[rr][j]);
+      }
       float mo[4] = {0.0f, 0.0f, 0.0f, 0.0f};
       float mn[4] = {0.0f, 0.0f, 0.0f, 0.0f}, u[4];
       pval_t<T>* pv = pj[rr][j];
@@ -1437,19 +1509,16 @@ __global__ __launch_bounds__(256) void k_fupdt(const DescF* __restrict__ table, 
 #pragma unroll
           for (int i = 0; i < 4; ++i) u[i] = u[i] * fs;
         }
+        const uint32_t c0 = (uint32_t)(c_base + q0), cn = (uint32_t)C;
         if constexpr (SR) {
-          keep4(u);
-          if (st) {
+          float x[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const float p = ld1<T>(P0, e + i);
-              const T rr = sr_round<T>((has_dec ? p * dec : p) - step * u[i], D.sr_seed, h.sr_step,
-                                       (uint64_t)(e + i));
-              uint16_t bits;
-              __builtin_memcpy(&bits, &rr, 2);
-              gp(reinterpret_cast<uint16_t*>(P0))[e + i] = bits;
-            }
-          }
+          for (int i = 0; i < 4; ++i) x[i] = (has_dec ? pv[i] * dec : pv[i]) - step * u[i];
+          keep4(x);
+          // the SR counters of the row's part of the tile, and what they share
+          const uint64_t z = sr_z + (uint64_t)rowb[rr];
+          const SrUnit srs = sr_unit<kTC>(z + (uint64_t)c_base);
+          if (st) sr_store4<T>(P0 + rowb[rr], c0, cn, x, z + c0, srs);
         } else {
           if (has_dec) {
 #pragma unroll
@@ -1458,11 +1527,13 @@ __global__ __launch_bounds__(256) void k_fupdt(const DescF* __restrict__ table, 
 #pragma unroll
           for (int i = 0; i < 4; ++i) pv[i] = pupd(step, u[i], pv[i]);
           keep4(pv);
-          if (st) store4n<T>(P0, e, e + 4, pv);
+          if constexpr (CUT) { if (st) store4e<T>(P0 + rowb[rr], c0, cn, pv); }
+          else if (st) store4n<T>(P0, e, e + 4, pv);
         }
         if constexpr (MK == 3) {
           keep4(mn);
-          if (st) store4n<float>(D.m, e, e + 4, mn);
+          if constexpr (CUT) { if (st) store4e<float>(D.m + rowb[rr], c0, cn, mn); }
+          else if (st) store4n<float>(D.m, e, e + 4, mn);
         } else if constexpr (kHasM) {
           // momentum re-encode: absmax over the block's G lanes.  C is a multiple
           // of the M block, so a block is wholly inside or wholly beyond C.
@@ -1581,7 +1652,7 @@ static int launch_stats(bool psq, const DescF* tab, int ntab, int64_t ntiles, hi
 // over the statistics tiles) and the rest (k_fupdate, over flat units).
 struct UpdGrid {
   int64_t ntiles, nunits;
-  bool any_tiled, any_flat;
+  bool any_tiled, any_cut, any_flat;
 };
 
 template <typename T, int MODE, bool SR, bool CM>
@@ -1591,17 +1662,25 @@ static int launch_update_m(int mk, const DescF* tab, int ntab, const UpdGrid& ug
   if (ug.any_tiled) {
     const dim3 g((unsigned)ug.ntiles);
     if constexpr (CM) {
-      if (mk == 1) hipLaunchKernelGGL((k_fupdt<T, MODE, SR, 1, true>), g, b, 0, st, tab, ntab, h);
-      else if (mk == kMkFp32) hipLaunchKernelGGL((k_fupdt<T, MODE, SR, 3, true>), g, b, 0, st, tab, ntab, h);
-      else hipLaunchKernelGGL((k_fupdt<T, MODE, SR, 2, true>), g, b, 0, st, tab, ntab, h);
+      if (mk == 1) hipLaunchKernelGGL((k_fupdt<T, MODE, SR, 1, true, false>), g, b, 0, st, tab, ntab, h);
+      else if (mk == kMkFp32) hipLaunchKernelGGL((k_fupdt<T, MODE, SR, 3, true, false>), g, b, 0, st, tab, ntab, h);
+      else hipLaunchKernelGGL((k_fupdt<T, MODE, SR, 2, true, false>), g, b, 0, st, tab, ntab, h);
     } else {
       switch (mk) {
-        case 0: hipLaunchKernelGGL((k_fupdt<T, MODE, SR, 0, false>), g, b, 0, st, tab, ntab, h); break;
-        case 1: hipLaunchKernelGGL((k_fupdt<T, MODE, SR, 1, false>), g, b, 0, st, tab, ntab, h); break;
-        case kMkFp32: hipLaunchKernelGGL((k_fupdt<T, MODE, SR, 3, false>), g, b, 0, st, tab, ntab, h); break;
-        default: hipLaunchKernelGGL((k_fupdt<T, MODE, SR, 2, false>), g, b, 0, st, tab, ntab, h); break;
+        case 0: hipLaunchKernelGGL((k_fupdt<T, MODE, SR, 0, false, false>), g, b, 0, st, tab, ntab, h); break;
+        case 1: hipLaunchKernelGGL((k_fupdt<T, MODE, SR, 1, false, false>), g, b, 0, st, tab, ntab, h); break;
+        case kMkFp32: hipLaunchKernelGGL((k_fupdt<T, MODE, SR, 3, false, false>), g, b, 0, st, tab, ntab, h); break;
+        default: hipLaunchKernelGGL((k_fupdt<T, MODE, SR, 2, false, false>), g, b, 0, st, tab, ntab, h); break;
       }
     }
+    int rc = check_launch("k_fupdt");
+    if (rc) return rc;
+  }
+  if (ug.any_cut) {   // no momentum, or fp32 momentum
+    const dim3 g((unsigned)ug.ntiles);
+    if constexpr (CM) hipLaunchKernelGGL((k_fupdt<T, MODE, SR, 3, true, true>), g, b, 0, st, tab, ntab, h);
+    else if (mk == kMkFp32) hipLaunchKernelGGL((k_fupdt<T, MODE, SR, 3, false, true>), g, b, 0, st, tab, ntab, h);
+    else hipLaunchKernelGGL((k_fupdt<T, MODE, SR, 0, false, true>), g, b, 0, st, tab, ntab, h);
     int rc = check_launch("k_fupdt");
     if (rc) return rc;
   }
@@ -1756,8 +1835,7 @@ int a8_factored_step(int dtype, int stochastic, const a8_tensor2d* tensors, int 
   if (stochastic && dtype == A8_F32) stochastic = 0;
   std::vector<DescF> tab((size_t)ntensors);
   int64_t tiles = 0, utiles = 0, units = 0, fblks = 0, csw = 0;
-  bool any_tiled = false, any_flat = false;
-  const size_t esz = dtype == A8_F32 ? 4 : (dtype == A8_F64 ? 8 : 2);
+  bool any_tiled = false, any_cut = false, any_flat = false;
   int64_t total = 0;
   for (int i = 0; i < ntensors; ++i) total += tensors[i].batch * tensors[i].rows * tensors[i].cols;
   const int64_t group_rows = group_tile_rows(total);
@@ -1789,10 +1867,11 @@ int a8_factored_step(int dtype, int stochastic, const a8_tensor2d* tensors, int 
     D.ws = t.workspace; D.lr = t.lr; D.fira_prev = t.fira_prev_norm; D.has_fira_prev = t.has_fira_prev;
     D.B = t.batch; D.R = t.rows; D.C = t.cols; D.numel = numel;
     D.sr_seed = t.sr_seed;
-    D.vec4 = ((t.cols * esz) % 16 == 0) ? 1 : 0;
-    D.tiled = (t.cols % 4 == 0) &&
-              (!has_m || m32 || (lbm >= 0 && m_block_size <= 256 && t.cols % m_block_size == 0)) ? 1 : 0;
-    (D.tiled ? any_tiled : any_flat) = true;
+    // coded momentum: whole M blocks per row (then C % 4 == 0 too)
+    D.tiled = t.cols >= 4 &&
+              (!has_m || m32 || (lbm >= 0 && m_block_size <= 256 && t.cols % m_block_size == 0)) ?
+              (t.cols % 4 ? 2 : 1) : 0;
+    (D.tiled == 0 ? any_flat : D.tiled == 1 ? any_tiled : any_cut) = true;
     D.tr = (int)fws_tile_rows(t.rows, group_rows);
     const FWs W = fws_layout(t.batch, t.rows, t.cols, D.tr);
     D.tile_begin = tiles;
@@ -1833,7 +1912,7 @@ int a8_factored_step(int dtype, int stochastic, const a8_tensor2d* tensors, int 
   h.dsc = reinterpret_cast<const a8_step_scalars*>(step_scalars);
   const bool clip = d > 0.0f || fira;
   const DescF* dt = reinterpret_cast<const DescF*>(table_dev);
-  const UpdGrid ug{utiles, units, any_tiled, any_flat};
+  const UpdGrid ug{utiles, units, any_tiled, any_cut, any_flat};
   switch (dtype) {
     case A8_F32: return run_group<float, false>(dt, ntensors, tiles, ug, fblks, csw, v_bits, c_bits, clip, h, st);
     case A8_BF16:

@@ -123,8 +123,8 @@ __device__ __forceinline__ T sr_round(float x, uint64_t seed, uint64_t step, uin
   }
 }
 
-// Stochastic rounding and store of four consecutive elements (base + i0 a multiple of
-// four elements from an aligned address; i0 + 4 <= n in one 8-byte store).  z is the
+// Stochastic rounding and store of the four consecutive elements from i0 on that lie below
+// n (all four: one 8-byte store, from any element alignment).  z is the
 // counter of the first, and srs what the counters of a whole unit share: unless the
 // unit crosses a multiple of 2^30 they agree from bit 30 up, so the high word's part of
 // the first product and the low word of z >> 30 are uniform (scalar registers).
@@ -177,7 +177,8 @@ __device__ __forceinline__ void sr_store4(T* base, uint32_t i0, uint32_t n, cons
   }
   A8_G uint16_t* p = gp(reinterpret_cast<uint16_t*>(base));
   if (i0 + 4 <= n) {
-    *gp(reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(base) + i0)) = u32x2{w[0], w[1]};
+    typedef u32x2 u32x2_a2 __attribute__((aligned(2)));
+    *((A8_G u32x2_a2*)(reinterpret_cast<uint16_t*>(base) + i0)) = u32x2{w[0], w[1]};
   } else {
 #pragma unroll
     for (int k = 0; k < 4; ++k)
