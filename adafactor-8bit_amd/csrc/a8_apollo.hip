@@ -41,6 +41,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kApTile = 64;     // G columns per left-side projection tile (and fp32 G's right-side tile)
 constexpr int kApRB = 3;        // 32-row blocks per right-side bf16 projection tile
 constexpr int kApTileR = 32 * kApRB;   // G rows per right-side bf16 projection tile
+constexpr int kApTileS = 32;           // the same in a group with few of them (ap_few_tiles)
 constexpr int kApPass = 256;    // low-rank outputs per projection pass (4 waves x 64)
 constexpr int kApUnit = 2048;   // low-rank elements per k_ap_low workgroup (8 per lane)
 constexpr int kApScR = 16;      // right side: g_low rows per k_ap_scale workgroup
@@ -53,9 +54,10 @@ static_assert(kApWide == kApPass, "a wide tile covers one output pass");
 
 // G channels per projection tile of a matrix: wide tiles for bf16 G at ranks
 // that are a multiple of 256, else kApTileR rows (bf16, right side) or kApTile.
-__host__ __device__ inline int64_t ap_tile(bool g16, int64_t R, int64_t C, int64_t r) {
+// few: kApTileS rows in place of kApTileR.
+__host__ __device__ inline int64_t ap_tile(bool g16, int64_t R, int64_t C, int64_t r, bool few) {
   if (g16 && r % kApWide == 0) return kApWide;
-  return (g16 && R >= C) ? kApTileR : kApTile;
+  return (g16 && R >= C) ? (few ? kApTileS : kApTileR) : kApTile;
 }
 
 // Workspace of one matrix (offsets in floats; partial arrays hold doubles).
@@ -86,11 +88,13 @@ __host__ __device__ inline ApL ap_layout(int64_t R, int64_t C, int64_t r, int64_
   w.ngsq = w.u + w.n_low;                  // ||G_ch||^2
   w.fin = w.ngsq + w.nchg;                 // channel scale s
   w.scal = w.fin + w.nchg;                 // 16 per-matrix scalars
-  w.gpart = (w.scal + 16 + 1) / 2 * 2;     // double[ntr]  ||G||^2 per tile
+  // bf16[3][rp][Kp]: P rows, three terms.  Kept from step to step, so its place depends on
+  // the matrix alone (the tile height may change with the group)
+  w.psplit = (w.scal + 16 + 63) / 64 * 64;
+  w.gpart = w.psplit + (3 * w.rp * w.Kp + 3) / 4 * 2;   // double[ntr]  ||G||^2 per tile
   w.ppart = w.gpart + 2 * w.ntr;           // double[ntr]  ||p||^2 per tile
   w.spart = w.ppart + 2 * w.ntr;           // double[3 nsc] sum ngsq s^2, sum u^2, sum g_low^2
-  w.psplit = (w.spart + 6 * w.nsc + 63) / 64 * 64;   // bf16[3][rp][Kp]  P rows, three terms
-  w.total = w.psplit + (3 * w.rp * w.Kp + 1) / 2;
+  w.total = w.spart + 6 * w.nsc;
   return w;
 }
 
@@ -185,10 +189,14 @@ __device__ __forceinline__ double ap_wg_sum(double x, double* s4) {
 }
 
 // ------------------------------------------------------------ bf16 helpers
-// Eight bf16 of a row: one 16-byte load when all eight are in range and the row
-// is 16-byte aligned, element loads otherwise (cnt in 0..8, the rest zero).
-__device__ __forceinline__ u32x4 ldg8(const uint16_t* base, int64_t off, int cnt, int vec) {
-  if (vec && cnt == 8) return *gp(reinterpret_cast<const u32x4*>(base + off));
+// Eight bf16 of a row: one 16-byte load when all eight are in range, from any element
+// alignment (rows of a matrix whose column count is no multiple of 8 start anywhere; the
+// type says so, and global loads need no more), element loads otherwise (cnt in 0..8, the
+// rest zero).
+typedef u32x4 u32x4_e2 __attribute__((aligned(2)));
+typedef f32x4 f32x4_e4 __attribute__((aligned(4)));
+__device__ __forceinline__ u32x4 ldg8(const uint16_t* base, int64_t off, int cnt) {
+  if (cnt == 8) return *((const A8_G u32x4_e2*)(base + off));
   uint32_t w[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
   for (int j = 0; j < 8; ++j)
@@ -453,26 +461,57 @@ __device__ __forceinline__ float sq8f(u32x4 q) {
 constexpr int kApGS = 72;   // LDS row stride (halves) of the right side's 64-row x 64-k G slab
 constexpr int kApTS = 40;   // LDS row stride (halves) of the left side's transposed 32-row slab
 
-// Right side: tile = kApTileR rows of G (kApRB blocks of 32) x 256 outputs (one
-// pass); wave w owns outputs [64w, 64w + 64) of the pass as two 32-column blocks
-// (NB of them active), for every row block of the tile.  Each 64-k slab of the
+// How the four waves of a narrow tile share its outputs and its reduction: NKG = 1, a wave
+// to each 64 outputs of a 256-output pass; for ranks up to 128, NKG = 2 waves, and up to 64,
+// all four, take the same 64 outputs on different parts of every k slab (a 32-k chunk, or
+// one 16-k sub-step of one), and add their accumulators through LDS at the end in a fixed
+// order.  Without the split three of four waves had no MFMAs at rank 64.
+__device__ __forceinline__ int ap_nkg(int64_t rp) { return rp <= 64 ? 4 : (rp <= 128 ? 2 : 1); }
+
+// acc += the accumulators of the group's other waves (kg > 0), in wave order; every wave
+// of the workgroup calls it the same number of times.  og: the wave's output group.
+template <int NKG>
+__device__ __forceinline__ void kg_sum(f32x16& acc, float* lds, int og, int kg, int l) {
+  if constexpr (NKG > 1) {
+    __syncthreads();
+    if (kg > 0) {
+      float* o = lds + (og * (NKG - 1) + kg - 1) * 1024 + l;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) o[64 * v] = acc[v];
+    }
+    __syncthreads();
+    if (kg == 0) {
+#pragma unroll
+      for (int k = 0; k < NKG - 1; ++k)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[v] += lds[(og * (NKG - 1) + k) * 1024 + 64 * v + l];
+    }
+  }
+}
+
+// Right side: tile = 32 RB rows of G x 256 outputs (one pass); a wave owns 64 outputs of
+// the pass as two 32-column blocks (NB of them active), for every row block of the tile,
+// and the part of every k slab that ap_nkg gives it.  Each 64-k slab of the
 // tile's G rows is loaded once per workgroup with row loads (eight lanes per
-// 128-byte row segment, kApRB rows per lane), scrubbed, squared into the row
+// 128-byte row segment, RB rows per lane), scrubbed, squared into the row
 // norms and stored to LDS (double buffered); the MFMA A fragments come from LDS,
 // the B fragments (P) from the fragment-ordered split.  A wave's B fragments
-// serve all kApRB row blocks, so the split P streamed through L1 per MFMA falls
-// as the tile grows.  FULL: all rows exist, K % 64 == 0 and rows are 16-byte
-// aligned.
-template <bool FULL, int NB>
+// serve all RB row blocks, so the split P streamed through L1 per MFMA falls
+// as the tile grows; a group of few tiles takes RB = 1 for more workgroups.  FULL: all
+// rows exist, K % 64 == 0 and rows are 16-byte aligned.
+template <bool FULL, int NB, int NKG, int RB>
 __device__ __forceinline__ void proj_right(const ApDesc& D, const ApL& L, int tile, uint16_t* lds, double* sred) {
-  constexpr int RB = kApRB;
+  constexpr int kRows = 32 * RB;
+  constexpr int NC = NKG == 1 ? 2 : 1, NJ = NKG == 4 ? 1 : 2;   // chunks of a slab, sub-steps of a chunk
   const int lane = threadIdx.x, l = lane & 63, l32 = l & 31, hi = l >> 5;
   const int w = __builtin_amdgcn_readfirstlane(lane >> 6);
+  const int og = w / NKG, kg = w % NKG;
+  const int kc0 = NKG == 1 ? 0 : (NKG == 2 ? kg : kg >> 1), j0 = NKG == 4 ? kg & 1 : 0;
   const int pass = (int)(tile / L.ntr);
   const int64_t rt = tile - (int64_t)pass * L.ntr;
   const int64_t R = D.R, C = D.C, r = D.r, K = C;
-  const int64_t row0 = rt * kApTileR;
-  const int64_t cb0 = (int64_t)pass * kApPass + w * 64;
+  const int64_t row0 = rt * kRows;
+  const int64_t cb0 = (int64_t)pass * kApPass + og * 64;
   constexpr bool act1 = NB >= 2;
   const int64_t nblk = L.rp / 32, nkc = L.Kp / 32;
   const int64_t blk0 = cb0 / 32;
@@ -495,21 +534,21 @@ __device__ __forceinline__ void proj_right(const ApDesc& D, const ApL& L, int ti
       } else {
         const int64_t k = k0 + lc;
         const int cnt = K - k >= 8 ? 8 : (K - k > 0 ? (int)(K - k) : 0);
-        x[q] = ldg8(G, ga * C + k, ga < R ? cnt : 0, D.valign);
+        x[q] = ldg8(G, ga * C + k, ga < R ? cnt : 0);
       }
     }
   };
   auto ldB = [&](int64_t kc, int t, u32x4* x0, u32x4* x1) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      x0[j] = gp(Ps)[psw_unit(t, blk0, kc, j, l, nblk, nkc)];
-      if constexpr (act1) x1[j] = gp(Ps)[psw_unit(t, blk0 + 1, kc, j, l, nblk, nkc)];
+    for (int j = 0; j < NJ; ++j) {
+      x0[j] = gp(Ps)[psw_unit(t, blk0, kc, j0 + j, l, nblk, nkc)];
+      if constexpr (act1) x1[j] = gp(Ps)[psw_unit(t, blk0 + 1, kc, j0 + j, l, nblk, nkc)];
     }
   };
   u32x4 f[RB];   // the next slab's G, prefetched
   ldG(0, f);
-  u32x4 b0[2], b1[2], c0[2], c1[2];
-  if constexpr (NB > 0) ldB(0, 0, b0, b1);
+  u32x4 b0[NJ], b1[NJ], c0[NJ], c1[NJ];
+  if constexpr (NB > 0) ldB(kc0, 0, b0, b1);
   int buf = 0;
   for (int64_t k0 = 0; k0 < K; k0 += 64) {
     u32x4 x[RB];
@@ -520,30 +559,31 @@ __device__ __forceinline__ void proj_right(const ApDesc& D, const ApL& L, int ti
 #pragma unroll
       for (int q = 0; q < RB; ++q) nr[q] += (double)sq8f(x[q]);
     }
-    uint16_t* sl = lds + buf * (kApTileR * kApGS);
+    uint16_t* sl = lds + buf * (kRows * kApGS);
 #pragma unroll
     for (int q = 0; q < RB; ++q) *reinterpret_cast<u32x4*>(&sl[(lr + 32 * q) * kApGS + lc]) = x[q];
     __syncthreads();   // the slab is in LDS; the other buffer's readers finished a barrier ago
     if constexpr (NB > 0) {
 #pragma unroll
-      for (int kc = 0; kc < 2; ++kc) {
+      for (int i = 0; i < NC; ++i) {
+        const int kc = kc0 + i;
         const int64_t kcg = k0 / 32 + kc;
-        u32x4 ar[RB][2];
+        u32x4 ar[RB][NJ];
 #pragma unroll
         for (int q = 0; q < RB; ++q) {
 #pragma unroll
-          for (int j = 0; j < 2; ++j)
-            ar[q][j] = *reinterpret_cast<const u32x4*>(&sl[(32 * q + l32) * kApGS + 32 * kc + 16 * hi + 8 * j]);
+          for (int j = 0; j < NJ; ++j)
+            ar[q][j] = *reinterpret_cast<const u32x4*>(&sl[(32 * q + l32) * kApGS + 32 * kc + 16 * hi + 8 * (j0 + j)]);
         }
 #pragma unroll
         for (int t = 0; t < 3; ++t) {
-          // the next term's (or the next chunk's first term's) P fragments
-          const bool last = kc == 1 && t == 2;
+          // the next term's (or the wave's next chunk's first term's) P fragments
           if (t < 2) ldB(kcg, t + 1, c0, c1);
-          else if (!last || k0 + 64 < K) ldB(kcg + 1, 0, c0, c1);
+          else if (i + 1 < NC) ldB(kcg + 1, 0, c0, c1);
+          else if (k0 + 64 < K) ldB(k0 / 32 + 2 + kc0, 0, c0, c1);
           __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int j = 0; j < 2; ++j) {
+          for (int j = 0; j < NJ; ++j) {
 #pragma unroll
             for (int q = 0; q < RB; ++q) {
               acc0[q] = mfma(as_bf8(ar[q][j]), as_bf8(b0[j]), acc0[q]);
@@ -552,7 +592,7 @@ __device__ __forceinline__ void proj_right(const ApDesc& D, const ApL& L, int ti
           }
           __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-          for (int j = 0; j < 2; ++j) {
+          for (int j = 0; j < NJ; ++j) {
             b0[j] = c0[j];
             if constexpr (act1) b1[j] = c1[j];
           }
@@ -564,8 +604,12 @@ __device__ __forceinline__ void proj_right(const ApDesc& D, const ApL& L, int ti
   float* glow = D.ws + L.glow;
 #pragma unroll
   for (int q = 0; q < RB; ++q) {
-    if constexpr (NB > 0) store_acc(acc0[q], glow, r, row0 + 32 * q, cb0 + l32, R, r, hi);
-    if constexpr (act1) store_acc(acc1[q], glow, r, row0 + 32 * q, cb0 + 32 + l32, R, r, hi);
+    kg_sum<NKG>(acc0[q], reinterpret_cast<float*>(lds), og, kg, l);
+    kg_sum<NKG>(acc1[q], reinterpret_cast<float*>(lds), og, kg, l);
+    if (kg == 0) {
+      if constexpr (NB > 0) store_acc(acc0[q], glow, r, row0 + 32 * q, cb0 + l32, R, r, hi);
+      if constexpr (act1) store_acc(acc1[q], glow, r, row0 + 32 * q, cb0 + 32 + l32, R, r, hi);
+    }
   }
   if (!pass0) return;
   // row norms: the eight lanes of a row (consecutive lanes) combine
@@ -588,16 +632,22 @@ __device__ __forceinline__ void proj_right(const ApDesc& D, const ApL& L, int ti
 // operand needs consecutive rows of G per lane, so each 32-row slab of the tile
 // is loaded with row loads (eight lanes per 128-byte row segment) and stored
 // transposed to LDS (double buffered).  The loading lanes also sum squares per
-// column.  FULL: all 64 columns exist, K % 32 == 0 and rows are 16-byte aligned.
-template <bool FULL, int NB>
+// column.  For ranks up to 128 two waves share 64 outputs, one sub-step of every slab each,
+// and up to 64 also one 32-column half each (ap_nkg).  FULL: all 64 columns exist, K % 32
+// == 0 and rows are 16-byte aligned.
+template <bool FULL, int NB, int NKG>
 __device__ __forceinline__ void proj_left(const ApDesc& D, const ApL& L, int tile, uint16_t* ldsT, double* sred) {
   const int lane = threadIdx.x, l = lane & 63, l32 = l & 31, hi = l >> 5;
   const int w = __builtin_amdgcn_readfirstlane(lane >> 6);
+  constexpr int NJ = NKG == 1 ? 2 : 1;       // sub-steps of a slab per wave
+  constexpr bool kHalf = NKG == 4;           // one 32-column half per wave
+  const int kg = NKG == 1 ? 0 : w & 1, og = NKG == 1 ? w : (NKG == 2 ? w >> 1 : 0);
+  const int half = kHalf ? w >> 1 : 0, j0 = kg;
   const int pass = (int)(tile / L.ntr);
   const int64_t ct = tile - (int64_t)pass * L.ntr;
   const int64_t C = D.C, r = D.r, K = D.R;
   const int64_t n0 = ct * kApTile;
-  const int64_t mb0 = (int64_t)pass * kApPass + w * 64;
+  const int64_t mb0 = (int64_t)pass * kApPass + og * 64;
   constexpr bool act1 = NB >= 2;
   const int64_t nblk = L.rp / 32, nkc = L.Kp / 32;
   const int64_t blk0 = mb0 / 32;
@@ -613,17 +663,17 @@ __device__ __forceinline__ void proj_left(const ApDesc& D, const ApL& L, int til
   for (int j = 0; j < 8; ++j) cs[j] = 0.0;
   auto ldG = [&](int64_t row) {
     if constexpr (FULL) return ldu(G, (uint32_t)((row * C + gc) * 2));
-    else return ldg8(G, row * C + gc, row < K ? cc : 0, D.valign);
+    else return ldg8(G, row * C + gc, row < K ? cc : 0);
   };
   auto ldA = [&](int64_t kc, int t, u32x4* x0, u32x4* x1) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      x0[j] = gp(Ps)[psw_unit(t, blk0, kc, j, l, nblk, nkc)];
-      if constexpr (act1) x1[j] = gp(Ps)[psw_unit(t, blk0 + 1, kc, j, l, nblk, nkc)];
+    for (int j = 0; j < NJ; ++j) {
+      x0[j] = gp(Ps)[psw_unit(t, blk0, kc, j0 + j, l, nblk, nkc)];
+      if constexpr (act1) x1[j] = gp(Ps)[psw_unit(t, blk0 + 1, kc, j0 + j, l, nblk, nkc)];
     }
   };
   u32x4 f = ldG(lr);   // the next slab's row, prefetched
-  u32x4 p0[2], p1[2], q0[2], q1[2];
+  u32x4 p0[NJ], p1[NJ], q0[NJ], q1[NJ];
   if constexpr (NB > 0) ldA(0, 0, p0, p1);
   int buf = 0;
   for (int64_t k0 = 0; k0 < K; k0 += 32) {
@@ -643,11 +693,11 @@ __device__ __forceinline__ void proj_left(const ApDesc& D, const ApL& L, int til
     __syncthreads();   // the slab is in LDS; the other buffer's readers finished a barrier ago
     if constexpr (NB > 0) {
       const int64_t kcg = k0 / 32;
-      u32x4 bc0[2], bc1[2];
+      u32x4 bc0[NJ], bc1[NJ];   // kHalf: the wave's half in bc0
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        bc0[j] = *reinterpret_cast<const u32x4*>(&sl[l32 * kApTS + 16 * hi + 8 * j]);
-        bc1[j] = *reinterpret_cast<const u32x4*>(&sl[(32 + l32) * kApTS + 16 * hi + 8 * j]);
+      for (int j = 0; j < NJ; ++j) {
+        bc0[j] = *reinterpret_cast<const u32x4*>(&sl[(32 * half + l32) * kApTS + 16 * hi + 8 * (j0 + j)]);
+        if constexpr (!kHalf) bc1[j] = *reinterpret_cast<const u32x4*>(&sl[(32 + l32) * kApTS + 16 * hi + 8 * (j0 + j)]);
       }
 #pragma unroll
       for (int t = 0; t < 3; ++t) {
@@ -655,17 +705,17 @@ __device__ __forceinline__ void proj_left(const ApDesc& D, const ApL& L, int til
         else if (k0 + 32 < K) ldA(kcg + 1, 0, q0, q1);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+        for (int j = 0; j < NJ; ++j) {
           a00 = mfma(as_bf8(p0[j]), as_bf8(bc0[j]), a00);
-          a01 = mfma(as_bf8(p0[j]), as_bf8(bc1[j]), a01);
+          if constexpr (!kHalf) a01 = mfma(as_bf8(p0[j]), as_bf8(bc1[j]), a01);
           if constexpr (act1) {
             a10 = mfma(as_bf8(p1[j]), as_bf8(bc0[j]), a10);
-            a11 = mfma(as_bf8(p1[j]), as_bf8(bc1[j]), a11);
+            if constexpr (!kHalf) a11 = mfma(as_bf8(p1[j]), as_bf8(bc1[j]), a11);
           }
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+        for (int j = 0; j < NJ; ++j) {
           p0[j] = q0[j];
           if constexpr (act1) p1[j] = q1[j];
         }
@@ -674,13 +724,24 @@ __device__ __forceinline__ void proj_left(const ApDesc& D, const ApL& L, int til
     buf ^= 1;
   }
   float* glow = D.ws + L.glow;
-  if constexpr (NB > 0) {
-    store_acc(a00, glow, C, mb0, n0 + l32, r, C, hi);
-    store_acc(a01, glow, C, mb0, n0 + 32 + l32, r, C, hi);
+  // the two sub-steps' sums: pairs of waves
+  constexpr int NP = NKG == 1 ? 1 : 2;
+  float* lf = reinterpret_cast<float*>(ldsT);
+  kg_sum<NP>(a00, lf, w >> 1, kg, l);
+  kg_sum<NP>(a10, lf, w >> 1, kg, l);
+  if constexpr (!kHalf) {
+    kg_sum<NP>(a01, lf, w >> 1, kg, l);
+    kg_sum<NP>(a11, lf, w >> 1, kg, l);
   }
-  if constexpr (act1) {
-    store_acc(a10, glow, C, mb0 + 32, n0 + l32, r, C, hi);
-    store_acc(a11, glow, C, mb0 + 32, n0 + 32 + l32, r, C, hi);
+  if (kg == 0) {
+    if constexpr (NB > 0) {
+      store_acc(a00, glow, C, mb0, n0 + 32 * half + l32, r, C, hi);
+      if constexpr (!kHalf) store_acc(a01, glow, C, mb0, n0 + 32 + l32, r, C, hi);
+    }
+    if constexpr (act1) {
+      store_acc(a10, glow, C, mb0 + 32, n0 + 32 * half + l32, r, C, hi);
+      if constexpr (!kHalf) store_acc(a11, glow, C, mb0 + 32, n0 + 32 + l32, r, C, hi);
+    }
   }
   if (!pass0) return;
   // column sums: lanes with equal (lane & 7) share columns; xor over 8, 16, 32
@@ -759,12 +820,12 @@ __device__ __forceinline__ void proj_wide8(const ApDesc& D, const ApL& L, int ti
       const int64_t row = ch0 + (tid >> 2) + 128 * i, k = k0 + 8 * (tid & 3);
       if constexpr (FULL) return ldu(G, (uint32_t)((row * C + k) * 2));
       const int cnt = K - k >= 8 ? 8 : (K - k > 0 ? (int)(K - k) : 0);
-      return ldg8(G, row * C + k, row < R ? cnt : 0, D.valign);
+      return ldg8(G, row * C + k, row < R ? cnt : 0);
     } else {
       const int64_t row = k0 + 2 * (tid & 15) + i, col = ch0 + 8 * (tid >> 4);
       if constexpr (FULL) return ldu(G, (uint32_t)((row * C + col) * 2));
       const int cnt = C - col >= 8 ? 8 : (C - col > 0 ? (int)(C - col) : 0);
-      return ldg8(G, row * C + col, row < K ? cnt : 0, D.valign);
+      return ldg8(G, row * C + col, row < K ? cnt : 0);
     }
   };
   // G store, piece i of 2: right, row piece i; left, columns 4 i .. 4 i + 3 of the
@@ -949,12 +1010,12 @@ __device__ __forceinline__ void split8(const float* x, u32x4* pl, double& sq) {
 #pragma unroll
   for (int t = 0; t < 3; ++t) pl[t] = u32x4{w[t][0], w[t][1], w[t][2], w[t][3]};
 }
-// Eight fp32 of a row at element offset off: two 16-byte loads when all eight exist
-// and the row is aligned, element loads otherwise (missing ones zero).
-__device__ __forceinline__ void ldf8(const float* base, int64_t off, int cnt, int vec, float* x) {
-  if (vec && cnt == 8) {
-    const f32x4 a = *gp(reinterpret_cast<const f32x4*>(base + off));
-    const f32x4 b = *gp(reinterpret_cast<const f32x4*>(base + off + 4));
+// Eight fp32 of a row at element offset off: two 16-byte loads when all eight exist,
+// from any element alignment, element loads otherwise (missing ones zero).
+__device__ __forceinline__ void ldf8(const float* base, int64_t off, int cnt, float* x) {
+  if (cnt == 8) {
+    const f32x4 a = *((const A8_G f32x4_e4*)(base + off));
+    const f32x4 b = *((const A8_G f32x4_e4*)(base + off + 4));
     x[0] = a[0]; x[1] = a[1]; x[2] = a[2]; x[3] = a[3];
     x[4] = b[0]; x[5] = b[1]; x[6] = b[2]; x[7] = b[3];
     return;
@@ -988,8 +1049,8 @@ __device__ __forceinline__ void proj_right32(const ApDesc& D, const ApL& L, int 
   auto ldG = [&](int64_t k0, float* x, float* y) {
     const int64_t k = k0 + lc;
     const int cnt = FULL ? 8 : (K - k >= 8 ? 8 : (K - k > 0 ? (int)(K - k) : 0));
-    ldf8(G, ga * C + k, (FULL || ga < R) ? cnt : 0, FULL ? 1 : D.valign, x);
-    ldf8(G, gb * C + k, (FULL || gb < R) ? cnt : 0, FULL ? 1 : D.valign, y);
+    ldf8(G, ga * C + k, (FULL || ga < R) ? cnt : 0, x);
+    ldf8(G, gb * C + k, (FULL || gb < R) ? cnt : 0, y);
   };
   auto ldB = [&](int64_t kc, int t, u32x4* x0, u32x4* x1) {
 #pragma unroll
@@ -1108,7 +1169,7 @@ __device__ __forceinline__ void proj_left32(const ApDesc& D, const ApL& L, int t
 #pragma unroll
   for (int j = 0; j < 8; ++j) cs[j] = 0.0;
   auto ldG = [&](int64_t row, float* x) {
-    ldf8(G, row * C + gc, (FULL || row < K) ? (FULL ? 8 : cc) : 0, FULL ? 1 : D.valign, x);
+    ldf8(G, row * C + gc, (FULL || row < K) ? (FULL ? 8 : cc) : 0, x);
   };
   auto ldA = [&](int64_t kc, int t, u32x4* x0, u32x4* x1) {
 #pragma unroll
@@ -1223,6 +1284,18 @@ __device__ __forceinline__ int xcd_order(int b, int nwg) {
   return x < rem ? x * (q + 1) + slot : rem * (q + 1) + (x - rem) * q + slot;
 }
 
+// nb: the wave's active 32-output blocks (uniform per wave; every wave runs the slab loop,
+// which holds the workgroup barriers).
+template <bool FULL, int NKG, int RB>
+__device__ __forceinline__ void proj_right_nb(const ApDesc& D, const ApL& L, int tile, uint16_t* lds, double* sred) {
+  const int64_t cb0 = (int64_t)(tile / L.ntr) * kApPass + (threadIdx.x >> 6) / NKG * 64;
+  const int nb = cb0 + 32 < L.rp ? 2 : (cb0 < L.rp ? 1 : 0);
+  if (nb == 2) proj_right<FULL, 2, NKG, RB>(D, L, tile, lds, sred);
+  else if (nb == 1) proj_right<FULL, 1, NKG, RB>(D, L, tile, lds, sred);
+  else proj_right<FULL, 0, NKG, RB>(D, L, tile, lds, sred);
+}
+
+template <int RB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 void k_ap_proj_r(ApDesc one, const ApDesc* tab, int ntab) {
   __shared__ __attribute__((aligned(16))) uint16_t lds[2 * kApTileR * kApGS];
@@ -1230,41 +1303,49 @@ void k_ap_proj_r(ApDesc one, const ApDesc* tab, int ntab) {
   int local;
   const ApDesc D = ap_pick(one, tab, ntab, 0, xcd_order((int)blockIdx.x, (int)gridDim.x), local);
   const ApL L = ap_layout(D.R, D.C, D.r, D.trows);
-  const int64_t row0 = (local % L.ntr) * kApTileR;
-  const bool full = D.valign && row0 + kApTileR <= D.R && D.C % 64 == 0;
-  const int64_t cb0 = (int64_t)(local / L.ntr) * kApPass + (threadIdx.x >> 6) * 64;
-  const int nb = cb0 + 32 < L.rp ? 2 : (cb0 < L.rp ? 1 : 0);   // uniform per wave
-  // every wave runs the slab loop (it holds the workgroup barriers)
+  const int64_t row0 = (local % L.ntr) * (32 * RB);
+  const bool full = D.valign && row0 + 32 * RB <= D.R && D.C % 64 == 0;
+  const int nkg = ap_nkg(L.rp);
   if (full) {
-    if (nb == 2) proj_right<true, 2>(D, L, local, lds, sred);
-    else if (nb == 1) proj_right<true, 1>(D, L, local, lds, sred);
-    else proj_right<true, 0>(D, L, local, lds, sred);
+    if (nkg == 4) proj_right_nb<true, 4, RB>(D, L, local, lds, sred);
+    else if (nkg == 2) proj_right_nb<true, 2, RB>(D, L, local, lds, sred);
+    else proj_right_nb<true, 1, RB>(D, L, local, lds, sred);
   } else {
-    if (nb == 2) proj_right<false, 2>(D, L, local, lds, sred);
-    else if (nb == 1) proj_right<false, 1>(D, L, local, lds, sred);
-    else proj_right<false, 0>(D, L, local, lds, sred);
+    if (nkg == 4) proj_right_nb<false, 4, RB>(D, L, local, lds, sred);
+    else if (nkg == 2) proj_right_nb<false, 2, RB>(D, L, local, lds, sred);
+    else proj_right_nb<false, 1, RB>(D, L, local, lds, sred);
   }
+}
+
+template <bool FULL, int NKG>
+__device__ __forceinline__ void proj_left_nb(const ApDesc& D, const ApL& L, int tile, uint16_t* ldsT, double* sred) {
+  const int w = (int)threadIdx.x >> 6, og = NKG == 1 ? w : (NKG == 2 ? w >> 1 : 0);
+  const int64_t mb0 = (int64_t)(tile / L.ntr) * kApPass + og * 64;
+  const int nb = mb0 + 32 < L.rp ? 2 : (mb0 < L.rp ? 1 : 0);
+  if (nb == 2) proj_left<FULL, 2, NKG>(D, L, tile, ldsT, sred);
+  else if (nb == 1) proj_left<FULL, 1, NKG>(D, L, tile, ldsT, sred);
+  else proj_left<FULL, 0, NKG>(D, L, tile, ldsT, sred);
 }
 
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 void k_ap_proj_l(ApDesc one, const ApDesc* tab, int ntab) {
   __shared__ __attribute__((aligned(16))) uint16_t ldsT[2 * kApTile * kApTS];
   __shared__ double sred[4 * 64 + 4];
+  static_assert(sizeof(ldsT) >= 2 * 1024 * sizeof(float), "kg_sum: two waves' accumulators");
   int local;
   const ApDesc D = ap_pick(one, tab, ntab, 1, xcd_order((int)blockIdx.x, (int)gridDim.x), local);
   const ApL L = ap_layout(D.R, D.C, D.r, D.trows);
   const int64_t n0 = (local % L.ntr) * kApTile;
   const bool full = D.valign && n0 + kApTile <= D.C && D.R % 32 == 0;
-  const int64_t mb0 = (int64_t)(local / L.ntr) * kApPass + (threadIdx.x >> 6) * 64;
-  const int nb = mb0 + 32 < L.rp ? 2 : (mb0 < L.rp ? 1 : 0);   // uniform per wave
+  const int nkg = ap_nkg(L.rp);
   if (full) {
-    if (nb == 2) proj_left<true, 2>(D, L, local, ldsT, sred);
-    else if (nb == 1) proj_left<true, 1>(D, L, local, ldsT, sred);
-    else proj_left<true, 0>(D, L, local, ldsT, sred);
+    if (nkg == 4) proj_left_nb<true, 4>(D, L, local, ldsT, sred);
+    else if (nkg == 2) proj_left_nb<true, 2>(D, L, local, ldsT, sred);
+    else proj_left_nb<true, 1>(D, L, local, ldsT, sred);
   } else {
-    if (nb == 2) proj_left<false, 2>(D, L, local, ldsT, sred);
-    else if (nb == 1) proj_left<false, 1>(D, L, local, ldsT, sred);
-    else proj_left<false, 0>(D, L, local, ldsT, sred);
+    if (nkg == 4) proj_left_nb<false, 4>(D, L, local, ldsT, sred);
+    else if (nkg == 2) proj_left_nb<false, 2>(D, L, local, ldsT, sred);
+    else proj_left_nb<false, 1>(D, L, local, ldsT, sred);
   }
 }
 
@@ -2028,6 +2109,13 @@ static int apollo_run(int phase, int dtype, int stochastic, const a8_apollo_tens
   if (stochastic && (dtype == A8_F32 || dtype == A8_F64)) stochastic = 0;
   std::vector<ApDesc> tab((size_t)n);
   std::vector<int32_t> first((size_t)6 * n);
+  // few right-side tiles of 96 rows: two workgroups per CU are not reached, so the rows of
+  // a P fragment matter less than the number of workgroups
+  int64_t nr96 = 0;
+  for (int i = 0; i < n; ++i)
+    if (ts[i].rows >= ts[i].cols && ts[i].rank > 0)
+      nr96 += (ts[i].rows + kApTileR - 1) / kApTileR * ((ts[i].rank + kApPass - 1) / kApPass);
+  const bool few = nr96 < 512;
   int64_t nrt = 0, nlt = 0, nwt = 0, nunit = 0, nsc = 0, napp = 0;
   for (int i = 0; i < n; ++i) {
     const a8_apollo_tensor& t = ts[i];
@@ -2043,7 +2131,7 @@ static int apollo_run(int phase, int dtype, int stochastic, const a8_apollo_tens
       return set_error(A8_ERR_ARG, "APOLLO with step_scalars needs each record's proj_state and proj_gap > 0");
     if (!aligned16(t.param) || !aligned16(t.grad) || !aligned16(t.workspace))
       return set_error(A8_ERR_ALIGN, "APOLLO param, grad and workspace must be 16-byte aligned");
-    const int64_t trows = ap_tile(dtype == A8_BF16, t.rows, t.cols, t.rank);
+    const int64_t trows = ap_tile(dtype == A8_BF16, t.rows, t.cols, t.rank, few);
     const ApL L = ap_layout(t.rows, t.cols, t.rank, trows);
     ApDesc& D = tab[(size_t)i];
     D.grad = t.grad; D.param = t.param; D.ws = t.workspace; D.proj_t = t.proj_t;
@@ -2124,7 +2212,8 @@ static int apollo_run(int phase, int dtype, int stochastic, const a8_apollo_tens
     // g_low = G P^T / P^T G with the channel norms of G: bf16 G as it is, fp32 G in three terms
     const bool g16 = dtype == A8_BF16;
     if (nrt > 0) {
-      if (g16) hipLaunchKernelGGL(k_ap_proj_r, dim3((unsigned)nrt), dim3(256), 0, st, one, dtab, n);
+      if (g16 && few) hipLaunchKernelGGL(k_ap_proj_r<1>, dim3((unsigned)nrt), dim3(256), 0, st, one, dtab, n);
+      else if (g16) hipLaunchKernelGGL(k_ap_proj_r<kApRB>, dim3((unsigned)nrt), dim3(256), 0, st, one, dtab, n);
       else hipLaunchKernelGGL(k_ap_proj_r32, dim3((unsigned)nrt), dim3(256), 0, st, one, dtab, n);
       if ((rc = check_launch("k_ap_proj_r"))) return rc;
     }
@@ -2205,13 +2294,8 @@ extern "C" {
 int64_t a8_apollo_workspace_floats(int64_t rows, int64_t cols, int64_t rank, int channel) {
   (void)channel;
   if (rows <= 0 || cols <= 0 || rank <= 0) return 0;
-  // either tile height (the dtype is not known here): the larger workspace
-  int64_t m = 0;
-  for (int g16 = 0; g16 < 2; ++g16) {
-    const int64_t a = ap_layout(rows, cols, rank, ap_tile(g16 != 0, rows, cols, rank)).total;
-    m = a > m ? a : m;
-  }
-  return m;
+  // the lowest tiles (neither the dtype nor the group is known here): the largest workspace
+  return ap_layout(rows, cols, rank, kApTileS).total;
 }
 
 int64_t a8_apollo_table_bytes(int ntensors) { return ntensors > 0 ? table_bytes(ntensors) : 0; }
