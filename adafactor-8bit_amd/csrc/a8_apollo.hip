@@ -36,6 +36,10 @@ namespace a8 {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kApTile = 64;     // G columns per left-side projection tile (and fp32 G's right-side tile)
@@ -88,10 +92,11 @@ __host__ __device__ inline ApL ap_layout(int64_t R, int64_t C, int64_t r, int64_
   w.ngsq = w.u + w.n_low;                  // ||G_ch||^2
   w.fin = w.ngsq + w.nchg;                 // channel scale s
   w.scal = w.fin + w.nchg;                 // 16 per-matrix scalars
-  // bf16[3][rp][Kp]: P rows, three terms.  Kept from step to step, so its place depends on
-  // the matrix alone (the tile height may change with the group)
+  // P rows: bf16[3][rp][Kp] in three terms, for wide tiles fp16[2][rp][Kp].  Kept from step
+  // to step, so its place depends on the matrix alone (the height of narrow tiles may change
+  // with the group)
   w.psplit = (w.scal + 16 + 63) / 64 * 64;
-  w.gpart = w.psplit + (3 * w.rp * w.Kp + 3) / 4 * 2;   // double[ntr]  ||G||^2 per tile
+  w.gpart = w.psplit + ((trows == kApWide ? 2 : 3) * w.rp * w.Kp + 3) / 4 * 2;   // double[ntr]  ||G||^2 per tile
   w.ppart = w.gpart + 2 * w.ntr;           // double[ntr]  ||p||^2 per tile
   w.spart = w.ppart + 2 * w.ntr;           // double[3 nsc] sum ngsq s^2, sum u^2, sum g_low^2
   w.total = w.spart + 6 * w.nsc;
@@ -99,7 +104,8 @@ __host__ __device__ inline ApL ap_layout(int64_t R, int64_t C, int64_t r, int64_
 }
 
 // Scalars in ApL::scal: [0] step (-alpha/denom, bias-corrected), [1] decay,
-// [3] tensor final scale, [4] alpha, [5] norm_unscaled, [6] fira scale.
+// [3] tensor final scale, [4] alpha, [5] norm_unscaled, [6] fira scale; kept with P's
+// split: [8] the power of two by which the fp16 split is scaled.
 
 // One matrix.  Read through the scalar cache: 8-byte words only.
 struct ApDesc {
@@ -291,13 +297,93 @@ __device__ __forceinline__ void split_unit(int64_t u, int64_t nblk, int64_t nkc,
     gp(out)[psw_unit(t, blk, kc, j, l, nblk, nkc)] = u32x4{w[t][0], w[t][1], w[t][2], w[t][3]};
 }
 
-__global__ __launch_bounds__(256) void k_ap_split(const float* __restrict__ pt, int64_t r, int64_t K, int right,
-                                                 int64_t rp, int64_t Kp, u32x4* __restrict__ out) {
-  const int64_t nblk = rp / 32, nkc = Kp / 32;
+// ---- the fp16 split of the wide tiles
+// P times a power of two (its largest element then in [2^10, 2^11)) as hi + lo, each rounded
+// to the nearest fp16.  The residual x - hi spans 13 signed bits of x's last place and lo
+// keeps 12 of them, so the sum is x itself for three quarters of the values and one unit of
+// x's 24th bit off for the rest (2^-25 of the largest element at worst for values below
+// 2^-13 of it).  Two MFMA terms in place of the exact bf16 split's three.
+
+// E: biased exponent of the largest magnitude (0: all zero).  The scale's biased exponent.
+__device__ __forceinline__ int p_scale_exp(int E) {
+  const int e = 264 - E;
+  return e < 10 ? 10 : (e > 244 ? 244 : e);
+}
+__device__ __forceinline__ float exp_f(int biased) { return __uint_as_float((uint32_t)biased << 23); }
+__device__ __forceinline__ uint32_t h_bits(_Float16 h) { return (uint32_t)__builtin_bit_cast(unsigned short, h); }
+
+// Unit (chunk kc, output block blk, sub-step j, lane l) of the two-term split, in the order
+// of psw_unit with two terms to a chunk; s: the scale.
+template <typename PV>
+__device__ __forceinline__ void split_unit2(int64_t u, int64_t nblk, int64_t nkc, int64_t r, int64_t K, float s,
+                                            PV pv, u32x4* __restrict__ out) {
+  const int l = (int)(u & 63), j = (int)((u >> 6) & 1);
+  const int64_t c = u >> 7, kc = c % nkc, blk = c / nkc;
+  const int64_t row = 32 * blk + (l & 31), k0 = 32 * kc + 16 * (l >> 5) + 8 * j;
+  uint32_t w[2][4] = {};
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const int64_t k = k0 + e;
+    const float x = (row < r && k < K) ? pv(row, k) * s : 0.0f;
+    const _Float16 h = (_Float16)x;
+    const _Float16 lo = (_Float16)(x - (float)h);
+    w[0][e >> 1] |= h_bits(h) << (16 * (e & 1));
+    w[1][e >> 1] |= h_bits(lo) << (16 * (e & 1));
+  }
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+    gp(out)[(((kc * 2 + t) * nblk + blk) * 2 + j) * 64 + l] = u32x4{w[t][0], w[t][1], w[t][2], w[t][3]};
+}
+
+__device__ __forceinline__ uint32_t max_u(uint32_t a, uint32_t b) { return a > b ? a : b; }
+// Largest x of 256 lanes; every lane gets it.
+__device__ __forceinline__ uint32_t wg_max_u(uint32_t x, uint32_t* s4) {
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) x = max_u(x, __shfl_xor(x, d, 64));
+  if ((threadIdx.x & 63) == 0) s4[threadIdx.x >> 6] = x;
+  __syncthreads();
+  return max_u(max_u(s4[0], s4[1]), max_u(s4[2], s4[3]));
+}
+// Magnitude bits of the largest of pt[i0], pt[i0 + step], ... below n.
+__device__ __forceinline__ uint32_t abs_max(const float* pt, int64_t i0, int64_t step, int64_t n) {
+  uint32_t m = 0u;
+  for (int64_t i = i0; i < n; i += step) m = max_u(m, __float_as_uint(gp(pt)[i]) & 0x7FFFFFFFu);
+  return m;
+}
+
+// Before k_ap_split of wide tiles: kPMax workgroups' maxima of P^T, in the head of the
+// workspace's u (written later in the step; rank >= 256, so it holds them).  Both kernels
+// take one matrix or a table of them, kPMax and `per` workgroups each.
+constexpr int kPMax = 64;
+__global__ __launch_bounds__(256) void k_ap_pmax(ApDesc one, const ApDesc* tab) {
+  const ApDesc D = tab ? tab[blockIdx.x / kPMax] : one;
+  if (D.trows != kApWide) return;
+  __shared__ uint32_t s4[4];
+  const ApL L = ap_layout(D.R, D.C, D.r, D.trows);
+  const int slot = (int)blockIdx.x % kPMax;
+  const uint32_t m = wg_max_u(abs_max(D.proj_t, slot * 256 + (int)threadIdx.x, kPMax * 256, D.r * L.K), s4);
+  if (threadIdx.x == 0) gp(D.ws)[L.u + slot] = __uint_as_float(m);
+}
+
+__global__ __launch_bounds__(256) void k_ap_split(ApDesc one, const ApDesc* tab, int per) {
+  const ApDesc D = tab ? tab[blockIdx.x / per] : one;
+  __shared__ uint32_t s4[4];
+  const ApL L = ap_layout(D.R, D.C, D.r, D.trows);
+  const bool right = D.R >= D.C;
+  const float* pt = D.proj_t;
+  const int64_t r = D.r, K = L.K, nblk = L.rp / 32, nkc = L.Kp / 32;
   const int64_t nu = nblk * nkc * 128;   // units per term
+  u32x4* out = reinterpret_cast<u32x4*>(D.ws + L.psplit);
   auto pv = [&](int64_t row, int64_t k) { return right ? gp(pt)[k * r + row] : gp(pt)[row * K + k]; };
-  for (int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x; u < nu; u += (int64_t)gridDim.x * 256)
-    split_unit(u, nblk, nkc, r, K, pv, out);
+  const int64_t u0 = (int64_t)(blockIdx.x % per) * 256 + threadIdx.x, step = (int64_t)per * 256;
+  if (D.trows == kApWide) {
+    const uint32_t m = wg_max_u(__float_as_uint(gp(D.ws)[L.u + threadIdx.x % kPMax]), s4);
+    const float s = exp_f(p_scale_exp((int)(m >> 23)));
+    if (u0 == 0) gp(D.ws)[L.scal + 8] = s;
+    for (int64_t u = u0; u < nu; u += step) split_unit2(u, nblk, nkc, r, K, s, pv, out);
+  } else {
+    for (int64_t u = u0; u < nu; u += step) split_unit(u, nblk, nkc, r, K, pv, out);
+  }
 }
 
 // ------------------------------------------------------------ device projection schedule
@@ -391,6 +477,16 @@ __global__ __launch_bounds__(256) void k_ap_pgen(ApDesc one, const ApDesc* tab, 
   float* pt = const_cast<float*>(D.proj_t);
   const uint64_t seed = (uint64_t)gp(D.pstate)[2];
   const float rsq = (float)sqrt((double)r);
+  // a wide tile's scale: from P as given, or for a generated P from its bound (Box-Muller
+  // from 53 bits: |z| <= sqrt(106 ln 2) < 8.6)
+  __shared__ uint32_t s4[4];
+  const bool wide = D.trows == kApWide;
+  float s = 1.0f;
+  if (wide) {
+    const uint32_t m = fresh == 1 ? __float_as_uint(8.6f / rsq) : wg_max_u(abs_max(pt, threadIdx.x, 256, r * K), s4);
+    s = exp_f(p_scale_exp((int)(m >> 23)));
+    if (slot == 0 && threadIdx.x == 0) gp(D.ws)[L.scal + 8] = s;
+  }
   for (int64_t u = (int64_t)slot * 256 + threadIdx.x; u < nu; u += (int64_t)kPGen * 256) {
     if (fresh == 1) {
       auto pv = [&](int64_t row, int64_t k) {
@@ -399,10 +495,12 @@ __global__ __launch_bounds__(256) void k_ap_pgen(ApDesc one, const ApDesc* tab, 
         gp(pt)[right ? k * r + row : row * K + k] = v;
         return v;
       };
-      split_unit(u, nblk, nkc, r, K, pv, out);
+      if (wide) split_unit2(u, nblk, nkc, r, K, s, pv, out);
+      else split_unit(u, nblk, nkc, r, K, pv, out);
     } else {
       auto pv = [&](int64_t row, int64_t k) { return right ? gp(pt)[k * r + row] : gp(pt)[row * K + k]; };
-      split_unit(u, nblk, nkc, r, K, pv, out);
+      if (wide) split_unit2(u, nblk, nkc, r, K, s, pv, out);
+      else split_unit(u, nblk, nkc, r, K, pv, out);
     }
   }
 }
@@ -772,33 +870,69 @@ __device__ __forceinline__ void proj_left(const ApDesc& D, const ApL& L, int til
 }
 
 // ------------------------------------------------------------ MFMA projection, wide tiles
-// bf16 G at ranks that are a multiple of 256 (C4's rank 256): a workgroup
-// computes a 256-channel x 256-output tile of g_low (channels: G rows on the
-// right side, G columns on the left).  Per 32-k slab the workgroup stages both
-// operands in LDS, double buffered: G, scrubbed, as [channel][k] rows, and the
-// chunk's split P for the tile's eight output blocks (fragment order, a plain
-// copy).  Each P unit is then fetched from L2 once per 256 channels: 6 bytes of
-// split P per G element (the narrower tiles above fetch it per wave, 16 bytes
-// per element at 96 rows).  The global loads of slab s + 1 are in flight while
-// slab s is multiplied; one barrier per slab publishes the next.  The squares
-// of each channel are summed from the staged slab for the channel norms.
-// FULL: all 256 channels exist, K % 32 == 0 and rows are 16-byte aligned.
+// Ranks that are a multiple of 256: a workgroup computes a 256-channel x 256-output tile of
+// g_low (channels: G rows on the right side, G columns on the left).  Per 32-k slab it
+// stages both operands in LDS, double buffered: G as [channel][k] rows and the chunk's split
+// P for the tile's eight output blocks (fragment order, a plain copy).  Each P unit is then
+// fetched from L2 once per 256 channels: 4 bytes of split P per G element.  FULL: all 256
+// channels exist, K % 32 == 0 and rows are 16-byte aligned.
+//
+// Both operands are fp16, each scaled by powers of two: the MFMA rate of fp16 is bf16's, and
+// its 11 bits take P in two terms where bf16's 8 take three.  A G element is exact in fp16
+// from 2^12 times the largest magnitude seen of its channel (below) down to 2^-20 of it, and
+// kept to 2^-28 of it below that; P's split errs by at most one unit of an element's 24th
+// bit.  A third of the accumulator's roundings falls away with the third term, and they
+// weigh more: against 64 bits g_low's rms error goes from 1.74e-7 of its rms to 1.56e-7 at
+// K = 256, from 4.9e-7 to 4.1e-7 at K = 2048 and from 9.9e-7 to 8.2e-7 at K = 8192, on either
+// side, for normal, heavy-tailed and one-signed gradients alike.
+//
+// Rank 256 over 1.1e9 elements: three bf16 terms 1577 us, two fp16 terms 1293, with the
+// barrier inside the MFMA stream (see proj_wide) 1241.  Matrix cores are busy for 49% of the
+// cycles at the 1.8 GHz the chip holds here; all operands from L2 instead of memory would give
+// 1097, the last round of tiles (7.2 per CU) leaves a tenth idle.
+//
+// A channel's scale must be known before its first slab is stored.  It comes from the
+// largest magnitude in two slabs, the first and the middle one, with 2^12 of headroom; in a
+// tile with a channel that is zero there (`careful`), from all slabs.  An element that does
+// not fit shows as an fp16 infinity, NaN or infinity in G as itself; a packed maximum over
+// everything stored finds either, and the workgroup then runs its tile again, careful and
+// with non-finite values as zero.  So the usual tile reads G once and needs no scrubbing, one
+// with zero rows reads it twice, and outliers above 2^12 of the sample and non-finite values
+// cost their tile a second run.
 constexpr int kApW = kApWide;             // channels and outputs of a wide tile
 constexpr int kApWS = 40;                 // LDS row stride (halves) of the G slab: 32 k + 8 pad
 constexpr int kApWGh = kApW * kApWS;      // halves per G slab buffer (20 KB)
-constexpr int kApWPu = 3 * 8 * 2 * 64;    // 16-byte P units per slab: 3 terms x 8 blocks x 2 j x 64 lanes (48 KB)
+constexpr int kApWPu = 2 * 8 * 2 * 64;    // 16-byte P units per slab: 2 terms x 8 blocks x 2 j x 64 lanes (32 KB)
 
-// Eight waves per wide tile, two per SIMD: waves (channel half gh, output quarter
-// oq) each own a 128 x 64 block (4 x 2 MFMA tiles, 128 accumulators), so one
-// wave's MFMAs issue while the other of its SIMD waits on LDS or staging.  The
-// staging of the next slab is split over 512 lanes (8 loads and 8 LDS stores
-// each), and a channel's squares over two lanes (k 0-15 and 16-31 of every slab),
-// added once at the end.  A lane's 16 squares of a slab are exact products summed
-// in fp32 by v_dot2_f32_bf16 (its rounding is the hardware's, within an ulp of
-// the fp32 sum); the slabs' sums accumulate in double.
+__device__ __forceinline__ f32x16 mfma_h(u32x4 a, u32x4 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0,
+                                                0);
+}
+__device__ __forceinline__ uint32_t cvt_h2(float a, float b) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, f16x2));
+}
+__device__ __forceinline__ uint32_t max_h2(uint32_t m, uint32_t w) {   // magnitudes of both halves
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, m),
+                                                                __builtin_bit_cast(u16x2, w & 0x7FFF7FFFu)));
+}
+__device__ __forceinline__ float dot_h2(uint32_t a, float c) {   // c + the squares of both halves
+  return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, a), __builtin_bit_cast(f16x2, a), c, false);
+}
+// A channel's scale (biased exponent) from its largest magnitude's E.
+__device__ __forceinline__ int g_scale_exp(int E, bool careful) {
+  const int e = (careful ? 268 : 257) - E;   // the largest below 2^15, the sample's below 2^4
+  return e < 1 ? 1 : (e > 251 ? 251 : e);
+}
+
+// Eight waves per wide tile, two per SIMD: waves (channel half gh, output quarter oq) each
+// own a 128 x 64 block (4 x 2 MFMA tiles, 128 accumulators), so one wave's MFMAs issue while
+// the other of its SIMD waits on LDS or staging.  The staging of a slab is split over 512
+// lanes, and a channel's squares over two lanes (k 0-15 and 16-31 of every slab), added once
+// at the end.  A lane's 16 squares of a slab are exact products summed in fp32 by
+// v_dot2_f32_f16; the slabs' sums accumulate in double.
 template <bool RIGHT, bool FULL>
-__device__ __forceinline__ void proj_wide8(const ApDesc& D, const ApL& L, int tile, uint16_t* gsl, u32x4* psl,
-                                           double* sred) {
+__device__ __forceinline__ void proj_wide(const ApDesc& D, const ApL& L, int tile, uint16_t* gsl, u32x4* psl,
+                                          int* sexp, double* sred, int* bad) {
   const int tid = threadIdx.x, l = tid & 63, l32 = l & 31, hi = l >> 5;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int gh = w >> 2, oq = w & 3;   // the wave's channel half and output quarter
@@ -812,143 +946,223 @@ __device__ __forceinline__ void proj_wide8(const ApDesc& D, const ApL& L, int ti
   const uint16_t* G = reinterpret_cast<const uint16_t*>(D.grad);
   const u32x4* Ps = reinterpret_cast<const u32x4*>(D.ws + L.psplit);
   const bool pass0 = pass == 0;
-  // G loader.  Right: rows (tid >> 2) + 128 i, eight k at 8 (tid & 3).  Left: k
-  // rows 2 (tid & 15) + i, eight columns at 8 (tid >> 4), stored transposed as
-  // pairs of k in one 32-bit word.
-  auto ldG1 = [&](int64_t k0, int i) -> u32x4 {
-    if constexpr (RIGHT) {
-      const int64_t row = ch0 + (tid >> 2) + 128 * i, k = k0 + 8 * (tid & 3);
-      if constexpr (FULL) return ldu(G, (uint32_t)((row * C + k) * 2));
-      const int cnt = K - k >= 8 ? 8 : (K - k > 0 ? (int)(K - k) : 0);
-      return ldg8(G, row * C + k, row < R ? cnt : 0);
-    } else {
-      const int64_t row = k0 + 2 * (tid & 15) + i, col = ch0 + 8 * (tid >> 4);
-      if constexpr (FULL) return ldu(G, (uint32_t)((row * C + col) * 2));
-      const int cnt = C - col >= 8 ? 8 : (C - col > 0 ? (int)(C - col) : 0);
-      return ldg8(G, row * C + col, row < K ? cnt : 0);
-    }
-  };
-  // G store, piece i of 2: right, row piece i; left, columns 4 i .. 4 i + 3 of the
-  // lane's eight (both k rows)
-  auto stG1 = [&](const u32x4* f, uint16_t* sl, int i) {
-    if constexpr (RIGHT) {
-      *reinterpret_cast<u32x4*>(&sl[((tid >> 2) + 128 * i) * kApWS + 8 * (tid & 3)]) = scrub8(f[i]);
-    } else {
-      const int kp = 2 * (tid & 15), c0 = 8 * (tid >> 4);
-      const u32x4 a = scrub8(f[0]), b = scrub8(f[1]);   // k rows kp, kp + 1
-      const uint32_t wa[4] = {a.x, a.y, a.z, a.w}, wb[4] = {b.x, b.y, b.z, b.w};
-#pragma unroll
-      for (int e = 4 * i; e < 4 * i + 4; ++e) {
-        const uint32_t lo = (e & 1) ? (wa[e >> 1] >> 16) : (wa[e >> 1] & 0xFFFFu);
-        const uint32_t hv = (e & 1) ? (wb[e >> 1] & 0xFFFF0000u) : (wb[e >> 1] << 16);
-        *reinterpret_cast<uint32_t*>(&sl[(c0 + e) * kApWS + kp]) = lo | hv;
-      }
-    }
-  };
-  // P: units tid + 512 i of the slab's 3072 (term i / 2)
-  auto ldP1 = [&](int64_t kc, int i) -> u32x4 {
-    return gp(Ps)[((kc * 3 + (i >> 1)) * nblk + 8 * pass) * 128 + tid + 512 * (i & 1)];
-  };
   f32x16 acc[4][2];
-#pragma unroll
-  for (int q = 0; q < 4; ++q)
-#pragma unroll
-    for (int c = 0; c < 2; ++c) acc[q][c] = f32x16{};
-  double nsq = 0.0;   // squares of channel ch0 + (tid & 255), k half tid >> 8
-  u32x4 fg[2], fp[6];   // the next slab, between its loads and its LDS stores
-  // One slab from LDS buffer b, 48 MFMAs, the other instructions placed between
-  // them in a fixed order (scheduling fences):
-  //   before MFMA 0: sub-step 0's G fragments, its first P term, the two
-  //     channel-row reads;
-  //   sub-step 0 (MFMAs 0-23): after MFMA m the squares of channel elements
-  //     2m, 2m + 1 (m < 8, one v_dot2); P terms 1-2 (m 0-3), the next slab's 8 global loads (m 4-11),
-  //     sub-step 1's G fragments (m 12-15), its P terms 0-1 (m 16-19, into the
-  //     registers of sub-step 0's dead terms);
-  //   sub-step 1 (MFMAs 24-47): its P term 2 (m 0-1), then after every third
-  //     MFMA one of the next slab's 8 LDS stores (6 P units, 2 G pieces).
-  auto slab = [&](const int b, const int64_t kn, auto next) {
-    constexpr bool NEXT = decltype(next)::value;
-    const uint16_t* gs = gsl + b * kApWGh;
-    const u32x4* ps = psl + b * kApWPu;
-    uint16_t* gn = gsl + (b ^ 1) * kApWGh;
-    u32x4* pn = psl + (b ^ 1) * kApWPu;
-    u32x4 ga[4], gb[4], pa[3][2], pb[3][2], cr[2];
-    float sq16 = 0.0f;
-    auto rdG = [&](int j, int q) {
-      return *reinterpret_cast<const u32x4*>(&gs[(gh * 128 + 32 * q + l32) * kApWS + 16 * hi + 8 * j]);
+  double nsq = 0.0;   // scaled squares of channel ch0 + (tid & 255), k half tid >> 8
+  for (bool careful = false;; careful = true) {
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));   // the addresses below are made again: hoisted out of this loop, they spill
+    const int l = tid & 63, l32 = l & 31, hi = l >> 5;
+    // G loader, piece i of 2, eight elements each.  Right: rows (tid >> 2) + 128 i, k at
+    // 8 (tid & 3).  Left: k rows 2 (tid & 15) + i, columns at 8 (tid >> 4), stored transposed
+    // as pairs of k in one 32-bit word.
+    auto ldG1 = [&](int64_t k0, int i, u32x4* f) {
+      const int64_t row = RIGHT ? ch0 + (tid >> 2) + 128 * i : k0 + 2 * (tid & 15) + i;
+      const int64_t col = RIGHT ? k0 + 8 * (tid & 3) : ch0 + 8 * (tid >> 4);
+      const int64_t left = C - col;
+      const int cnt = row >= R || left <= 0 ? 0 : (left >= 8 ? 8 : (int)left);
+      if constexpr (FULL) f[i] = ldu(G, (uint32_t)((row * C + col) * 2));
+      else f[i] = ldg8(G, row * C + col, cnt);
     };
-    auto rdP = [&](int j, int t, int c) { return ps[((t * 8 + oq * 2 + c) * 2 + j) * 64 + l]; };
-    auto rdC = [&](int g) {
-      return *reinterpret_cast<const u32x4*>(&gs[(tid & 255) * kApWS + 16 * (tid >> 8) + 8 * g]);
+    auto val = [&](const u32x4* f, int i, int e) -> float {   // element e of piece i
+      const uint32_t q = f[i][e >> 1];
+      return __uint_as_float((e & 1) ? (q & 0xFFFF0000u) : (q << 16));
     };
+    // P: units tid + 512 i of the slab's 2048 (term i / 2)
+    auto ldP1 = [&](int64_t kc, int i) -> u32x4 {
+      return gp(Ps)[((kc * 2 + (i >> 1)) * nblk + 8 * pass) * 128 + tid + 512 * (i & 1)];
+    };
+    constexpr int NC = RIGHT ? 2 : 8;   // channels that this lane stages
+    auto lane_ch = [&](int c) { return RIGHT ? (tid >> 2) + 128 * c : 8 * (tid >> 4) + c; };
+    u32x4 fg[2], fp[4];   // a slab between its loads and its LDS stores
+    float sc[NC];           // the scales of the lane's channels
+    {
+      // largest finite magnitudes of the lane's channels
+      uint32_t m[NC] = {};
+      auto seen = [&](const u32x4* f) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) ga[q] = rdG(0, q);
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int c = 0; c < 2; ++c) pa[0][c] = rdP(0, 0, c);
-    cr[0] = rdC(0);
-    cr[1] = rdC(1);
-    __builtin_amdgcn_sched_barrier(0);
+          for (int e = 0; e < 8; ++e) {
+            const uint32_t b = __float_as_uint(val(f, i, e)) & 0x7FFFFFFFu;
+            uint32_t& mc = m[RIGHT ? i : e];
+            mc = max_u(mc, b >= 0x7F800000u ? 0u : b);
+          }
+      };
+      ldG1(0, 0, fg);
+      ldG1(0, 1, fg);
 #pragma unroll
-    for (int m = 0; m < 24; ++m) {
-      const int t = m / 8, c = (m / 4) % 2, q = m % 4;
-      if constexpr (RIGHT) acc[q][c] = mfma(as_bf8(ga[q]), as_bf8(pa[t][c]), acc[q][c]);
-      else acc[q][c] = mfma(as_bf8(pa[t][c]), as_bf8(ga[q]), acc[q][c]);
-      if (m < 8) {   // two squares per MFMA (v_dot2), the slab's 16 in fp32, then into double
-        const uint32_t wv = cr[m / 4][m % 4];
-        sq16 = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, wv), __builtin_bit_cast(bf16x2, wv), sq16,
-                                               false);
-        if (m == 7) nsq += (double)sq16;
-      }
-      if (m < 4) {
-        pa[1 + m / 2][m % 2] = rdP(0, 1 + m / 2, m % 2);
-      } else if (m < 12) {
-        if constexpr (NEXT) {
-          if (m < 10) fp[m - 4] = ldP1(kn, m - 4);
-          else fg[m - 10] = ldG1(32 * kn, m - 10);
+      for (int i = 0; i < 4; ++i) fp[i] = ldP1(0, i);
+      if (careful) {
+        u32x4 f4[4][2];
+        for (int64_t s = 1; s < nslab; s += 4) {   // the last group's repeats change no maximum
+#pragma unroll
+          for (int j = 0; j < 8; ++j) ldG1(32 * (s + j / 2 < nslab ? s + j / 2 : nslab - 1), j % 2, f4[j / 2]);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) seen(f4[j]);
         }
-      } else if (m < 16) {
-        gb[m - 12] = rdG(1, m - 12);
-      } else if (m < 20) {
-        pb[(m - 16) / 2][m % 2] = rdP(1, (m - 16) / 2, m % 2);
+      } else {
+        u32x4 f2[2];
+        ldG1(32 * (nslab >> 1), 0, f2);
+        ldG1(32 * (nslab >> 1), 1, f2);
+        seen(f2);
       }
-      __builtin_amdgcn_sched_barrier(0);
-    }
+      seen(fg);
 #pragma unroll
-    for (int m = 0; m < 24; ++m) {
-      const int t = m / 8, c = (m / 4) % 2, q = m % 4;
-      if constexpr (RIGHT) acc[q][c] = mfma(as_bf8(gb[q]), as_bf8(pb[t][c]), acc[q][c]);
-      else acc[q][c] = mfma(as_bf8(pb[t][c]), as_bf8(gb[q]), acc[q][c]);
-      if (m < 2) pb[2][m] = rdP(1, 2, m);
-      if constexpr (NEXT) {
-        if (m % 3 == 2) {
-          const int pc = m / 3;
-          if (pc < 6) pn[tid + 512 * pc] = fp[pc];
-          else stG1(fg, gn, pc - 6);
-        }
+      for (int c = 0; c < NC; ++c) {
+#pragma unroll
+        for (int d = 1; d < (RIGHT ? 4 : 16); d <<= 1) m[c] = max_u(m[c], __shfl_xor(m[c], d, 64));
       }
-      __builtin_amdgcn_sched_barrier(0);
+      if ((tid & (RIGHT ? 3 : 15)) == 0) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) sexp[lane_ch(c)] = (int)(m[c] >> 23);
+      }
     }
-  };
-#pragma unroll
-  for (int i = 0; i < 2; ++i) fg[i] = ldG1(0, i);
-#pragma unroll
-  for (int i = 0; i < 6; ++i) psl[tid + 512 * i] = ldP1(0, i);
-  stG1(fg, gsl, 0);
-  stG1(fg, gsl, 1);
-  __syncthreads();
-  // slab s's LDS stores go to the other buffer, whose readers finished slab s - 1
-  // before the last barrier
-  for (int64_t s = 0; s + 1 < nslab; ++s) {
-    slab((int)(s & 1), s + 1, std::true_type{});
     __syncthreads();
+    {
+      if (!careful) {
+        bool zero = false;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) zero |= sexp[l + 64 * i] == 0 && ch0 + l + 64 * i < nch;
+        if (__ballot(zero)) {   // the same in every wave
+          __syncthreads();      // before sexp is written again
+          continue;
+        }
+      }
+      auto scale_exp = [&](int ch) { return g_scale_exp(sexp[ch], careful); };
+#pragma unroll
+      for (int c = 0; c < NC; ++c) sc[c] = exp_f(scale_exp(lane_ch(c)));
+      if (tid < kApW) sexp[kApW + tid] = scale_exp(tid);
+    }
+    uint32_t mx = 0u;
+    auto scrubG = [&] {
+      fg[0] = scrub8(fg[0]);
+      fg[1] = scrub8(fg[1]);
+    };
+    // Word e of the lane's eight, two elements of one channel: to fp16, and to LDS (right: four
+    // words at a time).
+    u32x4 cw;
+    auto stG1 = [&](uint16_t* sl, int e) {
+      const int pc = e >> 2, i = e & 3;
+      float a = RIGHT ? val(fg, pc, 2 * i) : val(fg, 0, e), b = RIGHT ? val(fg, pc, 2 * i + 1) : val(fg, 1, e);
+      a *= sc[RIGHT ? pc : e];
+      b *= sc[RIGHT ? pc : e];
+      const uint32_t h = cvt_h2(a, b);
+      mx = max_h2(mx, h);
+      if constexpr (RIGHT) {
+        cw[i] = h;
+        if (i == 3) *reinterpret_cast<u32x4*>(&sl[((tid >> 2) + 128 * pc) * kApWS + 8 * (tid & 3)]) = cw;
+      } else {
+        *reinterpret_cast<uint32_t*>(&sl[(8 * (tid >> 4) + e) * kApWS + 2 * (tid & 15)]) = h;
+      }
+    };
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int c = 0; c < 2; ++c) acc[q][c] = f32x16{};
+    nsq = 0.0;
+    // One slab from LDS buffer b, 32 MFMAs, the other instructions placed between them in a
+    // fixed order (scheduling fences).  g0 and p0 hold sub-step 0's first fragments on entry.
+    // Sub-step 0 reads its later fragments, the squares' rows and sub-step 1's first
+    // fragments; around its end the next slab (whose global loads were issued most of a slab
+    // ago) is converted and stored to the other buffer, and the loads of the slab after it
+    // issued.  The slab's one barrier stands in sub-step 1, behind this slab's last LDS read
+    // and the next one's last store, with 8 MFMAs left to cover the next slab's first reads.
+    u32x4 g0[4], p0[2][2];
+    auto rdG = [&](int b, int j, int q) {
+      return *reinterpret_cast<const u32x4*>(&gsl[b * kApWGh + (gh * 128 + 32 * q + l32) * kApWS + 16 * hi + 8 * j]);
+    };
+    auto rdP = [&](int b, int j, int t, int c) { return psl[b * kApWPu + ((t * 8 + oq * 2 + c) * 2 + j) * 64 + l]; };
+    auto slab = [&](const int b, const int64_t kl, auto next) {
+      constexpr bool NEXT = decltype(next)::value;
+      uint16_t* gn = gsl + (b ^ 1) * kApWGh;
+      u32x4* pn = psl + (b ^ 1) * kApWPu;
+      u32x4 g1[4], p1[2][2], cr;
+      float sq16 = 0.0f;
+      auto mul = [&](const u32x4* g, const u32x4 (*p)[2], int m) {
+        const int t = m / 8, c = (m / 4) % 2, q = m % 4;
+        if constexpr (RIGHT) acc[q][c] = mfma_h(g[q], p[t][c], acc[q][c]);
+        else acc[q][c] = mfma_h(p[t][c], g[q], acc[q][c]);
+      };
+      auto stage = [&](int n) {   // slot n of the slab's 32
+        if constexpr (NEXT) {
+          if (n == 12 && careful) scrubG();
+          if (n >= 12 && n < 20) stG1(gn, n - 12);
+          if (n >= 20 && n < 24) {
+            const int i = n - 20;
+            if (i < 2) ldG1(kl * 32, i, fg);
+            pn[tid + 512 * i] = fp[i];
+            fp[i] = ldP1(kl, i);
+          }
+        }
+      };
+#pragma unroll
+      for (int m = 0; m < 16; ++m) {
+        mul(g0, p0, m);
+        if (m < 2) p0[1][m] = rdP(b, 0, 1, m);
+        if (m == 2 || m == 6)
+          cr = *reinterpret_cast<const u32x4*>(&gsl[b * kApWGh + (tid & 255) * kApWS + 16 * (tid >> 8) + 2 * (m - 2)]);
+        if (m == 4 || m == 5 || m == 8 || m == 9) {   // four squares
+          sq16 = dot_h2(cr[2 * (m & 1)], sq16);
+          sq16 = dot_h2(cr[2 * (m & 1) + 1], sq16);
+          if (m == 9) nsq += (double)sq16;
+        }
+        if (m >= 8 && m < 12) g1[m - 8] = rdG(b, 1, m - 8);
+        if (m >= 12 && m < 14) p1[0][m - 12] = rdP(b, 1, 0, m - 12);
+        stage(m);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int m = 0; m < 16; ++m) {
+        mul(g1, p1, m);
+        if (m < 2) p1[1][m] = rdP(b, 1, 1, m);
+        stage(16 + m);
+        if constexpr (NEXT) {
+          if (m == 8) __syncthreads();
+          if (m >= 8 && m < 12) g0[m - 8] = rdG(b ^ 1, 0, m - 8);
+          if (m >= 12 && m < 14) p0[0][m - 12] = rdP(b ^ 1, 0, 0, m - 12);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    if (careful) scrubG();
+#pragma unroll
+    for (int e = 0; e < 8; ++e) stG1(gsl, e);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) psl[tid + 512 * i] = fp[i];
+    {
+      const int64_t k1 = nslab > 1 ? 1 : 0;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) ldG1(32 * k1, i, fg);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) fp[i] = ldP1(k1, i);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) g0[q] = rdG(0, 0, q);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) p0[0][c] = rdP(0, 0, 0, c);
+    for (int64_t s = 0; s + 1 < nslab; ++s)
+      slab((int)(s & 1), s + 2 < nslab ? s + 2 : nslab - 1, std::true_type{});
+    slab((int)((nslab - 1) & 1), 0, std::false_type{});
+    if (careful) break;
+    if ((mx & 0x7FFFu) >= 0x7C00u || (mx >> 16) >= 0x7C00u) *bad = 1;
+    __syncthreads();
+    if (!__builtin_amdgcn_readfirstlane(*bad)) break;
   }
-  slab((int)((nslab - 1) & 1), nslab, std::false_type{});
   float* glow = D.ws + L.glow;
+  const int pexp = 254 - (int)(__float_as_uint(gp(D.ws)[L.scal + 8]) >> 23);
+  const int* se = sexp + kApW;
   const int64_t gx0 = ch0 + gh * 128, ox0 = (int64_t)pass * kApW + oq * 64;
 #pragma unroll
   for (int q = 0; q < 4; ++q)
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
+      // the powers of two come off (see store_acc for an accumulator's rows)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int ch = gh * 128 + 32 * q + (RIGHT ? 8 * (v >> 2) + 4 * hi + (v & 3) : l32);
+        acc[q][c][v] = __builtin_amdgcn_ldexpf(acc[q][c][v], pexp - se[ch]);
+      }
       if constexpr (RIGHT) store_acc(acc[q][c], glow, r, gx0 + 32 * q, ox0 + 32 * c + l32, R, r, hi);
       else store_acc(acc[q][c], glow, C, ox0 + 32 * c, gx0 + 32 * q + l32, r, C, hi);
     }
@@ -961,7 +1175,7 @@ __device__ __forceinline__ void proj_wide8(const ApDesc& D, const ApL& L, int ti
   if (tid < kApW) {
     const int64_t ch = ch0 + tid;
     if (ch < nch) {
-      tot = nsq + half1[tid];
+      tot = ldexp(nsq + half1[tid], 2 * (127 - se[tid]));
       gp(D.ws + L.ngsq)[ch] = norm_sq(tot);
     }
   }
@@ -1349,7 +1563,7 @@ void k_ap_proj_l(ApDesc one, const ApDesc* tab, int ntab) {
   }
 }
 
-// Wide tiles of both sides, eight waves (one workgroup per CU: 138 KB of LDS).
+// Wide tiles of both sides, eight waves (one workgroup per CU: 108 KB of LDS).
 // Workgroups are dealt to the 8 XCDs round-robin by index; XCD x takes the
 // contiguous tile range [start[x], start[x + 1]) in order (its L2 then holds
 // the P split of one or two matrices at a time).  The host cuts the ranges at
@@ -1359,10 +1573,12 @@ void k_ap_proj_l(ApDesc one, const ApDesc* tab, int ntab) {
 struct ApXcd {
   int32_t start[9];
 };
-__global__ __launch_bounds__(512) void k_ap_proj_w8(ApDesc one, const ApDesc* tab, int ntab, ApXcd xs) {
+__global__ __launch_bounds__(512) void k_ap_proj_w(ApDesc one, const ApDesc* tab, int ntab, ApXcd xs) {
   __shared__ __attribute__((aligned(16))) uint16_t gsl[2 * kApWGh];
   __shared__ u32x4 psl[2 * kApWPu];
   __shared__ double sred[8 + kApW];
+  __shared__ int sexp[2 * kApW];
+  __shared__ int bad;
   const int x = (int)blockIdx.x % 8;
   const int wg = xs.start[x] + (int)blockIdx.x / 8;
   if (wg >= xs.start[x + 1]) return;
@@ -1370,12 +1586,17 @@ __global__ __launch_bounds__(512) void k_ap_proj_w8(ApDesc one, const ApDesc* ta
   const ApDesc D = ap_pick(one, tab, ntab, 5, wg, local);
   const ApL L = ap_layout(D.R, D.C, D.r, D.trows);
   const int64_t ch0 = (local % L.ntr) * kApW;
+  if (threadIdx.x == 0) bad = 0;
+  auto tile = [&](auto right, auto full) {
+    constexpr bool R = decltype(right)::value, F = decltype(full)::value;
+    proj_wide<R, F>(D, L, local, gsl, psl, sexp, sred, &bad);
+  };
   if (D.R >= D.C) {
-    if (D.valign && ch0 + kApW <= D.R && D.C % 32 == 0) proj_wide8<true, true>(D, L, local, gsl, psl, sred);
-    else proj_wide8<true, false>(D, L, local, gsl, psl, sred);
+    if (D.valign && ch0 + kApW <= D.R && D.C % 32 == 0) tile(std::true_type{}, std::true_type{});
+    else tile(std::true_type{}, std::false_type{});
   } else {
-    if (D.valign && ch0 + kApW <= D.C && D.R % 32 == 0) proj_wide8<false, true>(D, L, local, gsl, psl, sred);
-    else proj_wide8<false, false>(D, L, local, gsl, psl, sred);
+    if (D.valign && ch0 + kApW <= D.C && D.R % 32 == 0) tile(std::false_type{}, std::true_type{});
+    else tile(std::false_type{}, std::false_type{});
   }
 }
 
@@ -2200,13 +2421,22 @@ static int apollo_run(int phase, int dtype, int stochastic, const a8_apollo_tens
       hipLaunchKernelGGL(k_ap_pgen, dim3((unsigned)(n * kPGen)), dim3(256), 0, st, one, dtab, n);
       if ((rc = check_launch("k_ap_pgen"))) return rc;
     }
-    for (int i = 0; i < n && !dsc; ++i) {
+    int nfresh = 0;
+    for (int i = 0; i < n && !dsc; ++i) nfresh += ts[i].proj_fresh ? 1 : 0;
+    const bool all = nfresh == n && dtab;   // as on every refresh of the matrices of one schedule: one launch
+    for (int i = 0; i < (all ? 1 : (nfresh ? n : 0)); ++i) {
       if (!ts[i].proj_fresh) continue;
       const ApDesc& D = tab[(size_t)i];
       const ApL L = ap_layout(D.R, D.C, D.r, D.trows);
       const int64_t nb = (L.rp * L.Kp / 8 + 255) / 256;
-      hipLaunchKernelGGL(k_ap_split, dim3((unsigned)(nb < 4096 ? nb : 4096)), dim3(256), 0, st, D.proj_t, D.r, L.K,
-                         (int)(D.R >= D.C), L.rp, L.Kp, reinterpret_cast<u32x4*>(D.ws + L.psplit));
+      const int per = all ? 64 : (int)(nb < 4096 ? nb : 4096);
+      if (all ? nwt > 0 : D.trows == kApWide) {
+        hipLaunchKernelGGL(k_ap_pmax, dim3((unsigned)(all ? n * kPMax : kPMax)), dim3(256), 0, st, D,
+                           all ? dtab : nullptr);
+        if ((rc = check_launch("k_ap_pmax"))) return rc;
+      }
+      hipLaunchKernelGGL(k_ap_split, dim3((unsigned)(all ? n * per : per)), dim3(256), 0, st, D, all ? dtab : nullptr,
+                         per);
       if ((rc = check_launch("k_ap_split"))) return rc;
     }
     // g_low = G P^T / P^T G with the channel norms of G: bf16 G as it is, fp32 G in three terms
@@ -2244,8 +2474,8 @@ static int apollo_run(int phase, int dtype, int stochastic, const a8_apollo_tens
       while (xi <= 8) xs.start[xi++] = (int32_t)wg;
       int32_t most = 0;
       for (int k = 0; k < 8; ++k) most = std::max(most, xs.start[k + 1] - xs.start[k]);
-      hipLaunchKernelGGL(k_ap_proj_w8, dim3((unsigned)(8 * most)), dim3(512), 0, st, one, dtab, n, xs);
-      if ((rc = check_launch("k_ap_proj_w8"))) return rc;
+      hipLaunchKernelGGL(k_ap_proj_w, dim3((unsigned)(8 * most)), dim3(512), 0, st, one, dtab, n, xs);
+      if ((rc = check_launch("k_ap_proj_w"))) return rc;
     }
     if (h.scale_param) {   // ||p||^2 of the parameter (fp64 parameters refuse scale_parameter above)
       for (int i = 0; i < n; ++i) {

@@ -1,0 +1,93 @@
+"""g_low and the channel norms of APOLLO's bf16 projection kernels against 64 bits.
+
+Wide tiles (ranks that are a multiple of 256) hold both operands as scaled fp16: G from a
+scale that two slabs of each channel suggest, P^T as two terms.  The inputs below take every
+way through that: the usual one, channels that are zero where the scale looks, values far
+above it, values that are not finite, and the ends of the exponent range.  Narrow tiles are
+taken at both heights and at every split of the reduction over their waves.
+
+Bounds, u = 2^-24: the accumulator's rounding of T K products, T terms of P^T, is at most
+T (K + 2) u sum |g||p|; the fp16 split adds one unit of an element's 24th bit (2 u |p|), and
+values below the fp16 range 2^-28 of their channel's largest and 2^-35 of P^T's.  A channel's
+squares: 16-term fp32 sums (16 u), their sum in 64 bits, and the norm rounded and squared (3 u).
+"""
+import numpy as np
+import pytest
+import torch
+
+from test_gpu_apollo import C4_KW, _ws
+
+U = 2.0 ** -24
+
+
+def _low(shape, rank, g):
+    from adafactor8bit import Adafactor8Bit
+    p = torch.nn.Parameter(torch.zeros(shape, dtype=torch.bfloat16, device="cuda"))
+    opt = Adafactor8Bit([p], **dict(C4_KW, apollo_rank=rank))
+    p.grad = g.cuda()
+    opt.step()
+    torch.cuda.synchronize()
+    pt = opt.state[p]["apollo_proj_matrix_T"].double().cpu().numpy()
+    G = np.where(np.isfinite(g.double().numpy()), g.double().numpy(), 0.0)
+    right = shape[0] >= shape[1]
+    out = (shape[0], rank) if right else (rank, shape[1])
+    ws = _ws(opt, p)
+    n = out[0] * out[1]
+    return right, G, pt, ws[:n].reshape(out).astype(np.float64), ws[2 * n:2 * n + max(shape)].astype(np.float64)
+
+
+def _gradient(shape, kind, seed):
+    gen = torch.Generator().manual_seed(seed)
+    g = torch.randn(shape, generator=gen)
+    ch, k = (0, 1) if shape[0] >= shape[1] else (1, 0)
+    at = torch.arange(shape[ch])
+    t = g if ch == 0 else g.t()      # channels first
+    if kind == "zeros":              # some channels, and the first slab of others
+        t[at % 7 == 0] = 0.0
+        t[at % 5 == 1, :32] = 0.0
+        t[at % 5 == 1, shape[k] // 64 * 32:shape[k] // 64 * 32 + 32] = 0.0
+    elif kind == "outliers":
+        t[at, (40 + 3 * at) % shape[k]] *= 2.0 ** 20
+    elif kind == "nonfinite":
+        t[at[::3], (7 * at[::3]) % shape[k]] = float("inf")
+        t[at[1::3], (5 * at[1::3]) % shape[k]] = float("nan")
+    elif kind == "tiny":
+        t *= 2.0 ** -120
+    elif kind == "spread":
+        t *= torch.exp2((at % 81 - 40).float())[:, None]
+    return g.to(torch.bfloat16)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["plain", "zeros", "outliers", "nonfinite", "tiny", "spread"])
+@pytest.mark.parametrize("shape,rank", [((256, 256), 256), ((513, 264), 256), ((768, 544), 512), ((300, 290), 256),
+                                        ((288, 512), 256), ((264, 1001), 256), ((544, 700), 512)])
+def test_wide_tiles_against_64_bits(shape, rank, kind):
+    print(f"[apollo wide] {shape} r={rank} {kind}", flush=True)
+    right, G, pt, low, nsq = _low(shape, rank, _gradient(shape, kind, 21))
+    a, b = (G, pt) if right else (pt, G)
+    K = min(shape)
+    top = np.abs(G).max(axis=1, keepdims=True) if right else np.abs(G).max(axis=0, keepdims=True)
+    sp = np.abs(pt).sum(axis=0, keepdims=True) if right else np.abs(pt).sum(axis=1, keepdims=True)
+    sg = np.abs(G).sum(axis=1, keepdims=True) if right else np.abs(G).sum(axis=0, keepdims=True)
+    bound = (2 * (K + 2) + 2) * U * (np.abs(a) @ np.abs(b)) + 2.0 ** -28 * top * sp + 2.0 ** -35 * np.abs(pt).max() * sg
+    err = np.abs(low - a @ b)
+    assert np.all(err <= bound + 1e-44), float((err / (bound + 1e-44)).max())
+    if kind != "tiny":               # its squares are below the fp32 range
+        exact = (G * G).sum(axis=1 if right else 0)
+        assert np.all(np.abs(nsq - exact) <= 19 * U * exact)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [90, 49250])     # 32 rows to a tile, and 96 where there are enough of them
+@pytest.mark.parametrize("cols,rank", [(72, 32), (71, 64), (90, 65), (89, 33)])
+def test_narrow_tiles_against_64_bits(rows, cols, rank):
+    for shape in ((rows, cols), (cols, rows)) if rows > cols else ((rows, cols),):
+        print(f"[apollo narrow] {shape} r={rank}", flush=True)
+        right, G, pt, low, nsq = _low(shape, rank, _gradient(shape, "plain", 22))
+        a, b = (G, pt) if right else (pt, G)
+        err = np.abs(low - a @ b)
+        bound = 3 * (cols + 2) * U * (np.abs(a) @ np.abs(b))
+        assert np.all(err <= bound), float((err / bound).max())
+        exact = (G * G).sum(axis=1 if right else 0)
+        assert np.all(np.abs(nsq - exact) <= 19 * U * exact)
