@@ -200,6 +200,7 @@ __device__ __forceinline__ double ap_wg_sum(double x, double* s4) {
 // type says so, and global loads need no more), element loads otherwise (cnt in 0..8, the
 // rest zero).
 typedef u32x4 u32x4_e2 __attribute__((aligned(2)));
+typedef u32x2 u32x2_e1 __attribute__((aligned(1)));
 typedef f32x4 f32x4_e4 __attribute__((aligned(4)));
 __device__ __forceinline__ u32x4 ldg8(const uint16_t* base, int64_t off, int cnt) {
   if (cnt == 8) return *((const A8_G u32x4_e2*)(base + off));
@@ -1709,16 +1710,21 @@ __device__ __forceinline__ void ap_low_unit(const ApDesc& D, const ApL& L, int u
   }
   // The code streams are loaded here, before the AL8 decode table and its
   // barrier, so that their latency overlaps the table build.
-  uint32_t cw[2] = {0u, 0u};   // AL8 codes (table path)
-  if constexpr (VB == 8) {
-    if (!first && VL >= 64) {
-      if constexpr (FULL) {
-        const u32x2 q = *gp(reinterpret_cast<const u32x2*>(reinterpret_cast<const uint8_t*>(D.v_q) + e0));
-        cw[0] = q.x; cw[1] = q.y;
-      } else if (v_ok) {
+  uint32_t cw[VB == 16 ? 4 : 2] = {};   // V codes
+  if (VB != 0 && !first) {
+    if constexpr (FULL && VB == 8) {
+      const u32x2 q = *((const A8_G u32x2_e1*)(reinterpret_cast<const uint8_t*>(D.v_q) + e0));
+      cw[0] = q.x; cw[1] = q.y;
+    } else if constexpr (FULL && VB == 16) {
+      const u32x4 q = *((const A8_G u32x4_e2*)(reinterpret_cast<const uint16_t*>(D.v_q) + e0));
+      cw[0] = q.x; cw[1] = q.y; cw[2] = q.z; cw[3] = q.w;
+    } else if (v_ok) {
 #pragma unroll
-        for (int k = 0; k < 8; ++k)
+      for (int k = 0; k < 8; ++k) {
+        if constexpr (VB == 8)
           cw[k >> 2] |= (uint32_t)gp(reinterpret_cast<const uint8_t*>(D.v_q))[e0 + k] << (8 * (k & 3));
+        else if constexpr (VB == 16)
+          cw[k >> 1] |= (uint32_t)gp(reinterpret_cast<const uint16_t*>(D.v_q))[e0 + k] << (16 * (k & 1));
       }
     }
   }
@@ -1740,27 +1746,29 @@ __device__ __forceinline__ void ap_low_unit(const ApDesc& D, const ApL& L, int u
 #pragma unroll
       for (int k = 0; k < 8; ++k)
         if (k < cnt) vo[k] = gp(D.v_fp32)[e0 + k];
-    } else if (VB == 8 && VL >= 64) {
-      // one block per VL lanes (VL / 64 waves); its 255 decoded values into LDS
+    } else if (VB == 8 && VL > 64) {
+      // blocks of 1024 and more, one per VL lanes (VL / 64 waves): their 255 decoded values
+      // into LDS, one or two powers per lane.  With four or more blocks to the unit a table
+      // takes four powers per lane and more, an LDS store to each and eight LDS reads;
+      // decoding the eight codes in place takes eight powers and neither.  Rank 256 over
+      // 1.1e9 bf16 elements: a step with blocks of 256 took 175 us more than one with blocks
+      // of 2048, now 8; 3.1e8 fp32 elements, 16-bit codes: 2019 -> 1913 us; 8-bit codes in
+      // blocks of 512: 1885 -> 1873 us.
       const int bw = lane / VL;   // block of this unit
       const int64_t vbb = (int64_t)unit * (kApUnit >> lbv) + bw;
       const bool bok = vbb < nvb;   // a tail unit may end before its last block slot
       const float s_old = bok ? gp(D.v_scale)[vbb] : 0.0f, lm_old = bok ? gp(D.v_min_log)[vbb] : 0.0f;
-      for (int c = lane % VL; c < 256; c += VL)
-        dtab[bw * 256 + c] = c ? exp2_exact(((float)(c - 1) * s_old) / 254.0f + lm_old) : 0.0f;
+      for (int c = lane % VL; c < 256; c += VL) dtab[bw * 256 + c] = al_decode<254>((uint32_t)c, s_old, lm_old, false);
       __syncthreads();
 #pragma unroll
       for (int k = 0; k < 8; ++k) vo[k] = dtab[bw * 256 + ((cw[k >> 2] >> (8 * (k & 3))) & 0xFFu)];
     } else if (v_ok) {
-      const float s_old = gp(D.v_scale)[vb], lm_old = gp(D.v_min_log)[vb];
+      uint32_t c[8];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        uint32_t c;
-        if constexpr (VB == 8) c = gp(reinterpret_cast<const uint8_t*>(D.v_q))[e0 + k];
-        else c = gp(reinterpret_cast<const uint16_t*>(D.v_q))[e0 + k];
-        const float lm2 = VB == 8 ? 254.0f : 65534.0f;
-        vo[k] = c ? exp2_exact(((float)(c - 1) * s_old) / lm2 + lm_old) : 0.0f;
-      }
+      for (int k = 0; k < 8; ++k)
+        c[k] = VB == 8 ? (cw[k >> 2] >> (8 * (k & 3))) & 0xFFu
+                       : (cw[(k >> 1) % (VB == 16 ? 4 : 2)] >> (16 * (k & 1))) & 0xFFFFu;
+      al_decode<VB == 16 ? 65534 : 254, 8>(c, gp(D.v_scale)[vb], gp(D.v_min_log)[vb], false, vo);
     }
   }
 #pragma unroll
@@ -1939,7 +1947,7 @@ __device__ __forceinline__ void ap_low_unit(const ApDesc& D, const ApL& L, int u
 template <int VB, int MK>
 __global__ __launch_bounds__(256) void k_ap_low(ApDesc one, const ApDesc* tab, int ntab, ApHyp h) {
   __shared__ float xw[16];
-  __shared__ float dtab[4 * 256];
+  __shared__ float dtab[2 * 256];
   int unit;
   const ApDesc D = ap_pick(one, tab, ntab, 2, (int)blockIdx.x, unit);
   const ApL L = ap_layout(D.R, D.C, D.r, D.trows);

@@ -4,7 +4,8 @@ Wide tiles (ranks that are a multiple of 256) hold both operands as scaled fp16:
 scale that two slabs of each channel suggest, P^T as two terms.  The inputs below take every
 way through that: the usual one, channels that are zero where the scale looks, values far
 above it, values that are not finite, and the ends of the exponent range.  Narrow tiles are
-taken at both heights and at every split of the reduction over their waves.
+taken at both heights and at every split of the reduction over their waves.  The low-rank
+second moment is decoded through a table or directly, by its block size.
 
 Bounds, u = 2^-24: the accumulator's rounding of T K products, T terms of P^T, is at most
 T (K + 2) u sum |g||p|; the fp16 split adds one unit of an element's 24th bit (2 u |p|), and
@@ -91,3 +92,41 @@ def test_narrow_tiles_against_64_bits(rows, cols, rank):
         assert np.all(err <= bound), float((err / bound).max())
         exact = (G * G).sum(axis=1 if right else 0)
         assert np.all(np.abs(nsq - exact) <= 19 * U * exact)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("quant,top", [("al8", 255), ("al16", 65535)])
+@pytest.mark.parametrize("block", [256, 512, 1024, 2048])
+def test_low_rank_second_moment_decode(quant, top, block):
+    """The second step's V from the first one's codes, in units of 2048 elements and a part of one:
+    the block's range to fp32 rounding of its logarithms (below 64: 2^-18, twice), the codes to a tie."""
+    print(f"[apollo v] {quant} {block}", flush=True)
+    from adafactor8bit import Adafactor8Bit
+    shape, rank = (1001, 40), 37
+    gen = torch.Generator().manual_seed(block)
+    p = torch.nn.Parameter(torch.zeros(shape, device="cuda"))
+    opt = Adafactor8Bit([p], **dict(C4_KW, apollo_rank=rank, block_size=block, v_quant_type=quant))
+    v = None
+    for _ in range(2):
+        p.grad = (torch.randn(shape, generator=gen) * 1e-3).cuda()
+        opt.step()
+        torch.cuda.synchronize()
+        st = opt.state[p]
+        q = st["v_low_q"].cpu().numpy().reshape(-1).view(np.uint8 if top == 255 else np.uint16).astype(np.float64)
+        sc, lo = (st[k].cpu().numpy().astype(np.float32).repeat(block) for k in ("v_low_scale", "v_low_min_log"))
+        n = shape[0] * rank
+        if v is None:
+            x = (q.astype(np.float32) - np.float32(1)) * sc / np.float32(top - 1) + lo
+            v = np.where(q == 0, 0.0, np.exp2(x.astype(np.float64)).astype(np.float32))[:n].astype(np.float64)
+    g = _ws(opt, p)[:n]
+    w = np.float64(np.float32(1.0 - 0.999))
+    v = np.pad(v + w * ((g * g).astype(np.float32) - v.astype(np.float32)), (0, q.size - n))
+    logs = np.log2(np.where(v > 0, v, 1.0)).reshape(-1, block)
+    nz = (v > 0).reshape(-1, block)
+    least = np.maximum(np.where(nz, logs, np.inf).min(1), 2 * np.log2(1e-6))
+    most = np.where(nz, logs, -np.inf).max(1)
+    assert np.abs(lo[::block] - least).max() <= 2.0 ** -17
+    assert np.abs(sc[::block] - (most - least)).max() <= 2.0 ** -17
+    want = np.clip(np.rint((logs - lo[::block, None]) / sc[::block, None] * (top - 1)) + 1, 1, top)
+    off = np.abs(q - np.where(nz, want, 0).reshape(-1))
+    assert off.max() <= 1 and (off > 0).mean() <= (1e-4 if top == 255 else 0.02)
