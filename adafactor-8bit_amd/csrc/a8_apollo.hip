@@ -564,8 +564,14 @@ constexpr int kApTS = 40;   // LDS row stride (halves) of the left side's transp
 // to each 64 outputs of a 256-output pass; for ranks up to 128, NKG = 2 waves, and up to 64,
 // all four, take the same 64 outputs on different parts of every k slab (a 32-k chunk, or
 // one 16-k sub-step of one), and add their accumulators through LDS at the end in a fixed
-// order.  Without the split three of four waves had no MFMAs at rank 64.
-__device__ __forceinline__ int ap_nkg(int64_t rp) { return rp <= 64 ? 4 : (rp <= 128 ? 2 : 1); }
+// order.  Without the split three of four waves had no MFMAs at rank 64: five uneven
+// matrices, k_ap_proj_l 80 -> 41 us, k_ap_proj_r (with lower tiles) 153 -> 33.
+// A K of at most 128 (two slabs of the right side) leaves too little to share: a step over
+// 16384 x 128 at rank 64 takes 42.0 us split and 41.6 not, over 128 x 16384 43.4 and 43.9,
+// and such shapes keep the reduction in one wave, the order of an unsplit sum.
+__device__ __forceinline__ int ap_nkg(int64_t rp, int64_t K) {
+  return K <= 128 || rp > 128 ? 1 : (rp <= 64 ? 4 : 2);
+}
 
 // acc += the accumulators of the group's other waves (kg > 0), in wave order; every wave
 // of the workgroup calls it the same number of times.  og: the wave's output group.
@@ -1520,7 +1526,7 @@ void k_ap_proj_r(ApDesc one, const ApDesc* tab, int ntab) {
   const ApL L = ap_layout(D.R, D.C, D.r, D.trows);
   const int64_t row0 = (local % L.ntr) * (32 * RB);
   const bool full = D.valign && row0 + 32 * RB <= D.R && D.C % 64 == 0;
-  const int nkg = ap_nkg(L.rp);
+  const int nkg = ap_nkg(L.rp, L.K);
   if (full) {
     if (nkg == 4) proj_right_nb<true, 4, RB>(D, L, local, lds, sred);
     else if (nkg == 2) proj_right_nb<true, 2, RB>(D, L, local, lds, sred);
@@ -1552,7 +1558,7 @@ void k_ap_proj_l(ApDesc one, const ApDesc* tab, int ntab) {
   const ApL L = ap_layout(D.R, D.C, D.r, D.trows);
   const int64_t n0 = (local % L.ntr) * kApTile;
   const bool full = D.valign && n0 + kApTile <= D.C && D.R % 32 == 0;
-  const int nkg = ap_nkg(L.rp);
+  const int nkg = ap_nkg(L.rp, L.K);
   if (full) {
     if (nkg == 4) proj_left_nb<true, 4>(D, L, local, ldsT, sred);
     else if (nkg == 2) proj_left_nb<true, 2>(D, L, local, ldsT, sred);

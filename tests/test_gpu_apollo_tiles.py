@@ -80,10 +80,10 @@ def test_wide_tiles_against_64_bits(shape, rank, kind):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows", [90, 49250])     # 32 rows to a tile, and 96 where there are enough of them
-@pytest.mark.parametrize("cols,rank", [(72, 32), (71, 64), (90, 65), (89, 33)])
+@pytest.mark.parametrize("rows", [200, 49250])    # 32 rows to a tile, and 96 where there are enough of them
+@pytest.mark.parametrize("cols,rank", [(72, 32), (136, 32), (135, 64), (154, 65), (153, 33), (130, 130)])
 def test_narrow_tiles_against_64_bits(rows, cols, rank):
-    for shape in ((rows, cols), (cols, rows)) if rows > cols else ((rows, cols),):
+    for shape in ((rows, cols), (cols, rows)):
         print(f"[apollo narrow] {shape} r={rank}", flush=True)
         right, G, pt, low, nsq = _low(shape, rank, _gradient(shape, "plain", 22))
         a, b = (G, pt) if right else (pt, G)
