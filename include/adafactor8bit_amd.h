@@ -398,7 +398,7 @@ typedef struct a8_apollo_tensor {
   uint64_t sr_seed;
   /* per-step fields, read by a8_apollo_step_multi (a8_apollo_step takes them as arguments) */
   int first_step;          /* V initialised as g_low^2 * beta_val (no low-rank state yet) */
-  int proj_fresh;          /* P^T changed since the last call for this workspace */
+  int proj_fresh;          /* P^T, or whether the dtype is bf16, changed since the last call for this workspace */
   uint64_t step;           /* optimizer step (stochastic-rounding stream) */
   float bias_factor;       /* see bias_mode */
   /* device projection schedule (with step_scalars; NULL otherwise): int64[4] =
@@ -414,7 +414,7 @@ typedef struct a8_apollo_tensor {
  * torch.matmul at optimizer.py:2678-2681).  first_step: V initialised as
  * g_low^2 * beta_val (AL floor -126); later steps lerp with floor log_floor
  * (log2(max(apollo_eps^2, FLT_MIN))).  proj_fresh: P^T changed since the last
- * call for this workspace (its bf16 split is recomputed).  has_m: beta1 is set;
+ * call for this workspace (its split is recomputed).  has_m: beta1 is set;
  * m_fp32 selects fp32 m_low.  channel: apollo_scale_type "channel" (else
  * "tensor").  bias_mode 0/1/2: none / step *= bias_factor / step /= bias_factor.
  * wd_mode 0/1/2: none / decay uses alpha / decay uses lr.  V block_size and

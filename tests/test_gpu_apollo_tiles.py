@@ -130,3 +130,26 @@ def test_low_rank_second_moment_decode(quant, top, block):
     want = np.clip(np.rint((logs - lo[::block, None]) / sc[::block, None] * (top - 1)) + 1, 1, top)
     off = np.abs(q - np.where(nz, want, 0).reshape(-1))
     assert off.max() <= 1 and (off > 0).mean() <= (1e-4 if top == 255 else 0.02)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("capturable", [False, True])
+@pytest.mark.parametrize("order", [(torch.bfloat16, torch.float32), (torch.float32, torch.bfloat16)])
+def test_projection_split_follows_the_dtype(order, capturable):
+    """A parameter that changes between bf16 and fp32 has P^T split anew: the two kernels read
+    different forms of it.  Bound: the accumulator's, six products to an element at most."""
+    print(f"[apollo dtype] {order} {capturable}", flush=True)
+    from adafactor8bit import Adafactor8Bit
+    p = torch.nn.Parameter(torch.zeros((384, 256), device="cuda", dtype=order[0]))
+    opt = Adafactor8Bit([p], **dict(C4_KW, capturable=capturable))
+    for t, dt in enumerate(order + order):
+        p.grad = None
+        p.data = p.data.to(dt)
+        g = torch.randn((384, 256), generator=torch.Generator().manual_seed(t)).to(dt)
+        p.grad = g.cuda()
+        opt.step()
+        torch.cuda.synchronize()
+        pt = opt.state[p]["apollo_proj_matrix_T"].double().cpu().numpy()
+        G = g.double().numpy()
+        low = _ws(opt, p)[:384 * 256].reshape(384, 256).astype(np.float64)
+        assert np.all(np.abs(low - G @ pt) <= 6 * 258 * U * (np.abs(G) @ np.abs(pt)))
