@@ -82,7 +82,7 @@ constexpr int kSplit = 32;
 // Rows of the statistics tiles of a group of `total` elements: the tallest tiles that
 // still make about 2048 of them, eight workgroups for each of the 256 CUs.  256 rows from
 // 512 M elements on; a 44 M-parameter layer had 176 tiles of 256 rows, less than one
-// workgroup per CU, and takes 32 (k_fstats 64 -> 21 us, k_came1 144 -> 38).
+// workgroup per CU, and takes 32 (k_fstats 64 -> 24 us, k_came1 144 -> 52).
 static int64_t group_tile_rows(int64_t total) {
   int64_t tr = kTR;
   while (tr < kTRS && tr * kTC * 2048 < total) tr *= 2;

@@ -106,7 +106,7 @@ __device__ __forceinline__ Desc1D load_desc(const Desc1D* tab, int n, int wg) {
 // from the same old codes and gradient -- the same bits -- and re-encodes both states in
 // its one pass.  A clipped step then moves 6 + 16 bytes per fp32 parameter instead of
 // 11 + 19 with V' written and read back in fp32, and the 4 bytes of v_buf per parameter
-// are not allocated: 137.5 M parameters 267 + 437 -> 131 + 395 us.
+// are not allocated: 137.5 M parameters 267 + 437 -> 130 + 370 us.
 //
 // Lane t of a workgroup holds elements j*1024 + 4t + i of its 2048-element
 // unit (half j = 0, 1; i = 0..3), at register index k = 4j + i: every
