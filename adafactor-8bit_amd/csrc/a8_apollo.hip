@@ -900,12 +900,15 @@ __device__ __forceinline__ void proj_left(const ApDesc& D, const ApL& L, int til
 //
 // A channel's scale must be known before its first slab is stored.  It comes from the
 // largest magnitude in two slabs, the first and the middle one, with 2^12 of headroom; in a
-// tile with a channel that is zero there (`careful`), from all slabs.  An element that does
-// not fit shows as an fp16 infinity, NaN or infinity in G as itself; a packed maximum over
-// everything stored finds either, and the workgroup then runs its tile again, careful and
-// with non-finite values as zero.  So the usual tile reads G once and needs no scrubbing, one
-// with zero rows reads it twice, and outliers above 2^12 of the sample and non-finite values
-// cost their tile a second run.
+// tile with a channel that is zero there, from seven more.  A channel that is zero there too
+// takes a scale of 2^124, which any element from 2^-108 on leaves.  An element that does not
+// fit shows as an fp16 infinity, NaN or infinity in G as itself; a packed maximum over
+// everything stored finds either, and the workgroup then runs its tile again with the largest
+// magnitudes of all slabs and non-finite values as zero (`careful`).  So the usual tile reads
+// G once and needs no scrubbing, also with rows of zeros among its own, and outliers above
+// 2^12 of the sample and non-finite values cost their tile a second run: four matrices of
+// 32000 x 2048 step in 618 us (676 with three bf16 terms), with nine tenths of the rows zero
+// in 595 (640), with such an outlier in every row in 907 (676).
 constexpr int kApW = kApWide;             // channels and outputs of a wide tile
 constexpr int kApWS = 40;                 // LDS row stride (halves) of the G slab: 32 k + 8 pad
 constexpr int kApWGh = kApW * kApWS;      // halves per G slab buffer (20 KB)
@@ -955,7 +958,8 @@ __device__ __forceinline__ void proj_wide(const ApDesc& D, const ApL& L, int til
   const bool pass0 = pass == 0;
   f32x16 acc[4][2];
   double nsq = 0.0;   // scaled squares of channel ch0 + (tid & 255), k half tid >> 8
-  for (bool careful = false;; careful = true) {
+  for (int round = 0;;) {   // 0: two slabs sampled, 1: nine, 2: all
+    const bool careful = round == 2;
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));   // the addresses below are made again: hoisted out of this loop, they spill
     const int l = tid & 63, l32 = l & 31, hi = l >> 5;
@@ -999,11 +1003,15 @@ __device__ __forceinline__ void proj_wide(const ApDesc& D, const ApL& L, int til
       ldG1(0, 1, fg);
 #pragma unroll
       for (int i = 0; i < 4; ++i) fp[i] = ldP1(0, i);
-      if (careful) {
+      if (round) {
         u32x4 f4[4][2];
-        for (int64_t s = 1; s < nslab; s += 4) {   // the last group's repeats change no maximum
+        const int64_t step = careful || nslab < 8 ? 1 : nslab >> 3;
+        for (int64_t s = step; s < nslab; s += 4 * step) {   // the last group's repeats change no maximum
 #pragma unroll
-          for (int j = 0; j < 8; ++j) ldG1(32 * (s + j / 2 < nslab ? s + j / 2 : nslab - 1), j % 2, f4[j / 2]);
+          for (int j = 0; j < 8; ++j) {
+            const int64_t sj = s + (j / 2) * step;
+            ldG1(32 * (sj < nslab ? sj : nslab - 1), j % 2, f4[j / 2]);
+          }
 #pragma unroll
           for (int j = 0; j < 4; ++j) seen(f4[j]);
         }
@@ -1026,12 +1034,13 @@ __device__ __forceinline__ void proj_wide(const ApDesc& D, const ApL& L, int til
     }
     __syncthreads();
     {
-      if (!careful) {
+      if (round == 0) {
         bool zero = false;
 #pragma unroll
         for (int i = 0; i < 4; ++i) zero |= sexp[l + 64 * i] == 0 && ch0 + l + 64 * i < nch;
         if (__ballot(zero)) {   // the same in every wave
           __syncthreads();      // before sexp is written again
+          round = 1;
           continue;
         }
       }
@@ -1155,6 +1164,7 @@ __device__ __forceinline__ void proj_wide(const ApDesc& D, const ApL& L, int til
     if ((mx & 0x7FFFu) >= 0x7C00u || (mx >> 16) >= 0x7C00u) *bad = 1;
     __syncthreads();
     if (!__builtin_amdgcn_readfirstlane(*bad)) break;
+    round = 2;
   }
   float* glow = D.ws + L.glow;
   const int pexp = 254 - (int)(__float_as_uint(gp(D.ws)[L.scal + 8]) >> 23);

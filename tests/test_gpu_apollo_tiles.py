@@ -47,6 +47,8 @@ def _gradient(shape, kind, seed):
         t[at % 7 == 0] = 0.0
         t[at % 5 == 1, :32] = 0.0
         t[at % 5 == 1, shape[k] // 64 * 32:shape[k] // 64 * 32 + 32] = 0.0
+        t[at % 11 == 3] = 0.0        # zero but for one element, off the looked-at slabs where K allows it
+        t[at % 11 == 3, 101] = 1.0
     elif kind == "outliers":
         t[at, (40 + 3 * at) % shape[k]] *= 2.0 ** 20
     elif kind == "nonfinite":
