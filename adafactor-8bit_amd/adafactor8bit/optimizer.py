@@ -1707,14 +1707,9 @@ def _apollo_prep(opt, p, grad, st, group, dsc=None):
     key = (dev, "apollo", id(p))
     ent = opt._ws.get(key)
     nws = int(nat.lib().a8_apollo_workspace_floats(R, C, rank, 1))
-    half_split = p.dtype == torch.bfloat16 and rank % 256 == 0   # the form in which the workspace keeps P^T's split
     if ent is None or ent["ws"].numel() < nws:
-        ent = {"ws": torch.empty(nws, dtype=torch.float32, device=dev), "proj": None, "half": half_split}
+        ent = {"ws": torch.empty(nws, dtype=torch.float32, device=dev), "proj": None}
         opt._ws[key] = ent
-    elif ent["half"] != half_split:   # the parameter changed its dtype: split P^T anew
-        ent["proj"], ent["half"] = None, half_split
-        if pstate is not None:
-            pstate[3:].fill_(2)
     if dsc is None and (ent["proj"] is None or ent["proj"] != (proj_T.data_ptr(), proj_T._version)):
         fresh = True
     ent["proj"] = (proj_T.data_ptr(), proj_T._version)

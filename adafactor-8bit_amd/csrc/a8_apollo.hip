@@ -67,7 +67,7 @@ __host__ __device__ inline int64_t ap_tile(bool g16, int64_t R, int64_t C, int64
 // Workspace of one matrix (offsets in floats; partial arrays hold doubles).
 struct ApL {
   int64_t n_low, nchg, K, Kp, rp, ntr, npass, ntile, nunit, nsc, napp;
-  int64_t glow, u, ngsq, fin, scal, gpart, ppart, spart, psplit, total;
+  int64_t glow, u, ngsq, fin, scal, gpart, ppart, spart, psplit, phalf, total;
 };
 
 // trows: G channels (rows on the right side, columns on the left) per projection
@@ -92,11 +92,12 @@ __host__ __device__ inline ApL ap_layout(int64_t R, int64_t C, int64_t r, int64_
   w.ngsq = w.u + w.n_low;                  // ||G_ch||^2
   w.fin = w.ngsq + w.nchg;                 // channel scale s
   w.scal = w.fin + w.nchg;                 // 16 per-matrix scalars
-  // P rows: bf16[3][rp][Kp] in three terms, for wide tiles fp16[2][rp][Kp].  Kept from step
-  // to step, so its place depends on the matrix alone (the height of narrow tiles may change
-  // with the group)
+  // P rows: bf16[3][rp][Kp] in three terms, and at the ranks of the wide tiles also
+  // fp16[2][rp][Kp].  Kept from step to step, so their places depend on the matrix alone (the
+  // tiles change with G's type and with the group)
   w.psplit = (w.scal + 16 + 63) / 64 * 64;
-  w.gpart = w.psplit + ((trows == kApWide ? 2 : 3) * w.rp * w.Kp + 3) / 4 * 2;   // double[ntr]  ||G||^2 per tile
+  w.phalf = w.psplit + 3 * w.rp * w.Kp / 2;   // rp % 32 == 0 and Kp % 64 == 0: 16-byte aligned
+  w.gpart = w.phalf + (r % kApWide == 0 ? w.rp * w.Kp : 0);   // double[ntr]  ||G||^2 per tile
   w.ppart = w.gpart + 2 * w.ntr;           // double[ntr]  ||p||^2 per tile
   w.spart = w.ppart + 2 * w.ntr;           // double[3 nsc] sum ngsq s^2, sum u^2, sum g_low^2
   w.total = w.spart + 6 * w.nsc;
@@ -269,35 +270,6 @@ __device__ __forceinline__ int64_t psw_unit(int64_t t, int64_t blk, int64_t kc, 
   return (((kc * 3 + t) * nblk + blk) * 2 + j) * 64 + l;
 }
 
-// One 16-byte unit u of the split (three terms), from P^T values pv(row, k).
-template <typename PV>
-__device__ __forceinline__ void split_unit(int64_t u, int64_t nblk, int64_t nkc, int64_t r, int64_t K,
-                                           PV pv, u32x4* __restrict__ out) {
-  const int l = (int)(u & 63), j = (int)((u >> 6) & 1);
-  const int64_t c = u >> 7, kc = c % nkc, blk = c / nkc;
-  const int64_t row = 32 * blk + (l & 31), k0 = 32 * kc + 16 * (l >> 5) + 8 * j;
-  uint32_t w[3][4] = {};
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const int64_t k = k0 + e;
-    const float x = (row < r && k < K) ? pv(row, k) : 0.0f;
-    const __hip_bfloat16 h = __float2bfloat16(x);
-    const float r1 = x - __bfloat162float(h);
-    const __hip_bfloat16 m = __float2bfloat16(r1);
-    const __hip_bfloat16 lo = __float2bfloat16(r1 - __bfloat162float(m));
-    uint16_t bh, bm, bl;
-    __builtin_memcpy(&bh, &h, 2);
-    __builtin_memcpy(&bm, &m, 2);
-    __builtin_memcpy(&bl, &lo, 2);
-    w[0][e >> 1] |= (uint32_t)bh << (16 * (e & 1));
-    w[1][e >> 1] |= (uint32_t)bm << (16 * (e & 1));
-    w[2][e >> 1] |= (uint32_t)bl << (16 * (e & 1));
-  }
-#pragma unroll
-  for (int t = 0; t < 3; ++t)
-    gp(out)[psw_unit(t, blk, kc, j, l, nblk, nkc)] = u32x4{w[t][0], w[t][1], w[t][2], w[t][3]};
-}
-
 // ---- the fp16 split of the wide tiles
 // P times a power of two (its largest element then in [2^10, 2^11)) as hi + lo, each rounded
 // to the nearest fp16.  The residual x - hi spans 13 signed bits of x's last place and lo
@@ -313,27 +285,43 @@ __device__ __forceinline__ int p_scale_exp(int E) {
 __device__ __forceinline__ float exp_f(int biased) { return __uint_as_float((uint32_t)biased << 23); }
 __device__ __forceinline__ uint32_t h_bits(_Float16 h) { return (uint32_t)__builtin_bit_cast(unsigned short, h); }
 
-// Unit (chunk kc, output block blk, sub-step j, lane l) of the two-term split, in the order
-// of psw_unit with two terms to a chunk; s: the scale.
+// One 16-byte unit u of each split, from P^T values pv(row, k): three bf16 terms to out, and if
+// half is set two fp16 terms of s times the value there, in the same order with two terms to
+// a chunk.
 template <typename PV>
-__device__ __forceinline__ void split_unit2(int64_t u, int64_t nblk, int64_t nkc, int64_t r, int64_t K, float s,
-                                            PV pv, u32x4* __restrict__ out) {
+__device__ __forceinline__ void split_unit(int64_t u, int64_t nblk, int64_t nkc, int64_t r, int64_t K, PV pv,
+                                           u32x4* __restrict__ out, u32x4* __restrict__ half, float s) {
   const int l = (int)(u & 63), j = (int)((u >> 6) & 1);
   const int64_t c = u >> 7, kc = c % nkc, blk = c / nkc;
   const int64_t row = 32 * blk + (l & 31), k0 = 32 * kc + 16 * (l >> 5) + 8 * j;
-  uint32_t w[2][4] = {};
+  uint32_t w[3][4] = {}, v[2][4] = {};
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     const int64_t k = k0 + e;
-    const float x = (row < r && k < K) ? pv(row, k) * s : 0.0f;
-    const _Float16 h = (_Float16)x;
-    const _Float16 lo = (_Float16)(x - (float)h);
-    w[0][e >> 1] |= h_bits(h) << (16 * (e & 1));
-    w[1][e >> 1] |= h_bits(lo) << (16 * (e & 1));
+    const float x = (row < r && k < K) ? pv(row, k) : 0.0f;
+    const __hip_bfloat16 h = __float2bfloat16(x);
+    const float r1 = x - __bfloat162float(h);
+    const __hip_bfloat16 m = __float2bfloat16(r1);
+    const __hip_bfloat16 lo = __float2bfloat16(r1 - __bfloat162float(m));
+    uint16_t bh, bm, bl;
+    __builtin_memcpy(&bh, &h, 2);
+    __builtin_memcpy(&bm, &m, 2);
+    __builtin_memcpy(&bl, &lo, 2);
+    w[0][e >> 1] |= (uint32_t)bh << (16 * (e & 1));
+    w[1][e >> 1] |= (uint32_t)bm << (16 * (e & 1));
+    w[2][e >> 1] |= (uint32_t)bl << (16 * (e & 1));
+    const float xs = x * s;
+    const _Float16 xh = (_Float16)xs;
+    v[0][e >> 1] |= h_bits(xh) << (16 * (e & 1));
+    v[1][e >> 1] |= h_bits((_Float16)(xs - (float)xh)) << (16 * (e & 1));
   }
 #pragma unroll
+  for (int t = 0; t < 3; ++t)
+    gp(out)[psw_unit(t, blk, kc, j, l, nblk, nkc)] = u32x4{w[t][0], w[t][1], w[t][2], w[t][3]};
+  if (!half) return;
+#pragma unroll
   for (int t = 0; t < 2; ++t)
-    gp(out)[(((kc * 2 + t) * nblk + blk) * 2 + j) * 64 + l] = u32x4{w[t][0], w[t][1], w[t][2], w[t][3]};
+    gp(half)[(((kc * 2 + t) * nblk + blk) * 2 + j) * 64 + l] = u32x4{v[t][0], v[t][1], v[t][2], v[t][3]};
 }
 
 __device__ __forceinline__ uint32_t max_u(uint32_t a, uint32_t b) { return a > b ? a : b; }
@@ -352,13 +340,13 @@ __device__ __forceinline__ uint32_t abs_max(const float* pt, int64_t i0, int64_t
   return m;
 }
 
-// Before k_ap_split of wide tiles: kPMax workgroups' maxima of P^T, in the head of the
-// workspace's u (written later in the step; rank >= 256, so it holds them).  Both kernels
-// take one matrix or a table of them, kPMax and `per` workgroups each.
+// Before k_ap_split at the ranks of wide tiles: kPMax workgroups' maxima of P^T, in the head
+// of the workspace's u (written later in the step; rank >= 256, so it holds them).  Both
+// kernels take one matrix or a table of them, kPMax and `per` workgroups each.
 constexpr int kPMax = 64;
 __global__ __launch_bounds__(256) void k_ap_pmax(ApDesc one, const ApDesc* tab) {
   const ApDesc D = tab ? tab[blockIdx.x / kPMax] : one;
-  if (D.trows != kApWide) return;
+  if (D.r % kApWide != 0) return;
   __shared__ uint32_t s4[4];
   const ApL L = ap_layout(D.R, D.C, D.r, D.trows);
   const int slot = (int)blockIdx.x % kPMax;
@@ -377,14 +365,15 @@ __global__ __launch_bounds__(256) void k_ap_split(ApDesc one, const ApDesc* tab,
   u32x4* out = reinterpret_cast<u32x4*>(D.ws + L.psplit);
   auto pv = [&](int64_t row, int64_t k) { return right ? gp(pt)[k * r + row] : gp(pt)[row * K + k]; };
   const int64_t u0 = (int64_t)(blockIdx.x % per) * 256 + threadIdx.x, step = (int64_t)per * 256;
-  if (D.trows == kApWide) {
+  float s = 1.0f;
+  u32x4* half = nullptr;
+  if (r % kApWide == 0) {
     const uint32_t m = wg_max_u(__float_as_uint(gp(D.ws)[L.u + threadIdx.x % kPMax]), s4);
-    const float s = exp_f(p_scale_exp((int)(m >> 23)));
+    s = exp_f(p_scale_exp((int)(m >> 23)));
     if (u0 == 0) gp(D.ws)[L.scal + 8] = s;
-    for (int64_t u = u0; u < nu; u += step) split_unit2(u, nblk, nkc, r, K, s, pv, out);
-  } else {
-    for (int64_t u = u0; u < nu; u += step) split_unit(u, nblk, nkc, r, K, pv, out);
+    half = reinterpret_cast<u32x4*>(D.ws + L.phalf);
   }
+  for (int64_t u = u0; u < nu; u += step) split_unit(u, nblk, nkc, r, K, pv, out, half, s);
 }
 
 // ------------------------------------------------------------ device projection schedule
@@ -481,12 +470,13 @@ __global__ __launch_bounds__(256) void k_ap_pgen(ApDesc one, const ApDesc* tab, 
   // a wide tile's scale: from P as given, or for a generated P from its bound (Box-Muller
   // from 53 bits: |z| <= sqrt(106 ln 2) < 8.6)
   __shared__ uint32_t s4[4];
-  const bool wide = D.trows == kApWide;
   float s = 1.0f;
-  if (wide) {
+  u32x4* half = nullptr;
+  if (r % kApWide == 0) {
     const uint32_t m = fresh == 1 ? __float_as_uint(8.6f / rsq) : wg_max_u(abs_max(pt, threadIdx.x, 256, r * K), s4);
     s = exp_f(p_scale_exp((int)(m >> 23)));
     if (slot == 0 && threadIdx.x == 0) gp(D.ws)[L.scal + 8] = s;
+    half = reinterpret_cast<u32x4*>(D.ws + L.phalf);
   }
   for (int64_t u = (int64_t)slot * 256 + threadIdx.x; u < nu; u += (int64_t)kPGen * 256) {
     if (fresh == 1) {
@@ -496,12 +486,10 @@ __global__ __launch_bounds__(256) void k_ap_pgen(ApDesc one, const ApDesc* tab, 
         gp(pt)[right ? k * r + row : row * K + k] = v;
         return v;
       };
-      if (wide) split_unit2(u, nblk, nkc, r, K, s, pv, out);
-      else split_unit(u, nblk, nkc, r, K, pv, out);
+      split_unit(u, nblk, nkc, r, K, pv, out, half, s);
     } else {
       auto pv = [&](int64_t row, int64_t k) { return right ? gp(pt)[k * r + row] : gp(pt)[row * K + k]; };
-      if (wide) split_unit2(u, nblk, nkc, r, K, s, pv, out);
-      else split_unit(u, nblk, nkc, r, K, pv, out);
+      split_unit(u, nblk, nkc, r, K, pv, out, half, s);
     }
   }
 }
@@ -954,7 +942,7 @@ __device__ __forceinline__ void proj_wide(const ApDesc& D, const ApL& L, int til
   const int64_t nblk = L.rp / 32;
   const int64_t nslab = (K + 31) / 32;
   const uint16_t* G = reinterpret_cast<const uint16_t*>(D.grad);
-  const u32x4* Ps = reinterpret_cast<const u32x4*>(D.ws + L.psplit);
+  const u32x4* Ps = reinterpret_cast<const u32x4*>(D.ws + L.phalf);
   const bool pass0 = pass == 0;
   f32x16 acc[4][2];
   double nsq = 0.0;   // scaled squares of channel ch0 + (tid & 255), k half tid >> 8
@@ -2445,8 +2433,11 @@ static int apollo_run(int phase, int dtype, int stochastic, const a8_apollo_tens
       hipLaunchKernelGGL(k_ap_pgen, dim3((unsigned)(n * kPGen)), dim3(256), 0, st, one, dtab, n);
       if ((rc = check_launch("k_ap_pgen"))) return rc;
     }
-    int nfresh = 0;
-    for (int i = 0; i < n && !dsc; ++i) nfresh += ts[i].proj_fresh ? 1 : 0;
+    int nfresh = 0, nhalf = 0;
+    for (int i = 0; i < n && !dsc; ++i) {
+      nfresh += ts[i].proj_fresh ? 1 : 0;
+      nhalf += ts[i].rank % kApWide == 0 ? 1 : 0;
+    }
     const bool all = nfresh == n && dtab;   // as on every refresh of the matrices of one schedule: one launch
     for (int i = 0; i < (all ? 1 : (nfresh ? n : 0)); ++i) {
       if (!ts[i].proj_fresh) continue;
@@ -2454,7 +2445,7 @@ static int apollo_run(int phase, int dtype, int stochastic, const a8_apollo_tens
       const ApL L = ap_layout(D.R, D.C, D.r, D.trows);
       const int64_t nb = (L.rp * L.Kp / 8 + 255) / 256;
       const int per = all ? 64 : (int)(nb < 4096 ? nb : 4096);
-      if (all ? nwt > 0 : D.trows == kApWide) {
+      if (all ? nhalf > 0 : D.r % kApWide == 0) {
         hipLaunchKernelGGL(k_ap_pmax, dim3((unsigned)(all ? n * kPMax : kPMax)), dim3(256), 0, st, D,
                            all ? dtab : nullptr);
         if ((rc = check_launch("k_ap_pmax"))) return rc;

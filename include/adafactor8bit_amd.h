@@ -398,7 +398,7 @@ typedef struct a8_apollo_tensor {
   uint64_t sr_seed;
   /* per-step fields, read by a8_apollo_step_multi (a8_apollo_step takes them as arguments) */
   int first_step;          /* V initialised as g_low^2 * beta_val (no low-rank state yet) */
-  int proj_fresh;          /* P^T, or whether the dtype is bf16, changed since the last call for this workspace */
+  int proj_fresh;          /* P^T changed since the last call for this workspace */
   uint64_t step;           /* optimizer step (stochastic-rounding stream) */
   float bias_factor;       /* see bias_mode */
   /* device projection schedule (with step_scalars; NULL otherwise): int64[4] =
