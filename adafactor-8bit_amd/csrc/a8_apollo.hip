@@ -869,38 +869,31 @@ __device__ __forceinline__ void proj_left(const ApDesc& D, const ApL& L, int til
 // g_low (channels: G rows on the right side, G columns on the left).  Per 32-k slab it
 // stages both operands in LDS, double buffered: G as [channel][k] rows and the chunk's split
 // P for the tile's eight output blocks (fragment order, a plain copy).  Each P unit is then
-// fetched from L2 once per 256 channels: 4 bytes of split P per G element.  FULL: all 256
-// channels exist, K % 32 == 0 and rows are 16-byte aligned.
+// fetched from L2 once per 256 channels.  FULL: all 256 channels exist, K % 32 == 0 and rows
+// are 16-byte aligned.
 //
-// Both operands are fp16, each scaled by powers of two: the MFMA rate of fp16 is bf16's, and
-// its 11 bits take P in two terms where bf16's 8 take three.  A G element is exact in fp16
-// from 2^12 times the largest magnitude seen of its channel (below) down to 2^-20 of it, and
-// kept to 2^-28 of it below that; P's split errs by at most one unit of an element's 24th
-// bit.  A third of the accumulator's roundings falls away with the third term, and they
-// weigh more: against 64 bits g_low's rms error goes from 1.74e-7 of its rms to 1.56e-7 at
-// K = 256, from 4.9e-7 to 4.1e-7 at K = 2048 and from 9.9e-7 to 8.2e-7 at K = 8192, on either
-// side, for normal, heavy-tailed and one-signed gradients alike.
-//
-// Rank 256 over 1.1e9 elements: three bf16 terms 1577 us, two fp16 terms 1293, with the
-// barrier inside the MFMA stream (see proj_wide) 1241.  Matrix cores are busy for 49% of the
-// cycles at the 1.8 GHz the chip holds here; all operands from L2 instead of memory would give
-// 1097, the last round of tiles (7.2 per CU) leaves a tenth idle.
+// wide_half takes both operands as fp16, each scaled by powers of two: the MFMA rate of fp16
+// is bf16's, and its 11 bits take P in two terms where bf16's 8 take three.  A G element is
+// exact in fp16 from 2^12 times the largest magnitude seen of its channel (below) down to
+// 2^-20 of it, and kept to 2^-28 of it below that.
 //
 // A channel's scale must be known before its first slab is stored.  It comes from the
 // largest magnitude in two slabs, the first and the middle one, with 2^12 of headroom; in a
-// tile with a channel that is zero there, from seven more.  A channel that is zero there too
-// takes a scale of 2^124, which any element from 2^-108 on leaves.  An element that does not
-// fit shows as an fp16 infinity, NaN or infinity in G as itself; a packed maximum over
-// everything stored finds either, and the workgroup then runs its tile again with the largest
-// magnitudes of all slabs and non-finite values as zero (`careful`).  So the usual tile reads
-// G once and needs no scrubbing, also with rows of zeros among its own, and outliers above
-// 2^12 of the sample and non-finite values cost their tile a second run: four matrices of
-// 32000 x 2048 step in 618 us (676 with three bf16 terms), with nine tenths of the rows zero
-// in 595 (640), with such an outlier in every row in 907 (676).
+// tile with a channel that is zero there, from three more.  A channel that is zero there too
+// takes a scale of 2^124, which any element from 2^-108 on leaves.  An element that does not fit shows as an fp16 infinity, NaN or infinity in G as
+// itself, and a packed maximum over everything stored finds either before the slab is
+// multiplied.  The slab is then stored again scrubbed, as all later ones of the tile are;
+// if that does not fit, wide_exact takes the tile from this slab on: G as it is, scrubbed,
+// against P in three exact bf16 terms.
+//
+// Four matrices of 32000 x 2048 at rank 256, a step (in brackets with three bf16 terms from
+// the first slab on): normal gradients 761 us (836), nine tenths of the rows zero 713 (780),
+// an element in ten of each row 667 (745), one in a hundred 752 (734), a value above 2^12 of
+// the sample in every row 831 (825), one to a tile 757 (773), an infinity to a tile 688 (764).
 constexpr int kApW = kApWide;             // channels and outputs of a wide tile
 constexpr int kApWS = 40;                 // LDS row stride (halves) of the G slab: 32 k + 8 pad
 constexpr int kApWGh = kApW * kApWS;      // halves per G slab buffer (20 KB)
-constexpr int kApWPu = 2 * 8 * 2 * 64;    // 16-byte P units per slab: 2 terms x 8 blocks x 2 j x 64 lanes (32 KB)
+constexpr int kApWPu = 8 * 2 * 64;        // 16-byte P units per slab and term: 8 blocks x 2 j x 64 lanes (16 KB)
 
 __device__ __forceinline__ f32x16 mfma_h(u32x4 a, u32x4 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0,
@@ -916,100 +909,92 @@ __device__ __forceinline__ uint32_t max_h2(uint32_t m, uint32_t w) {   // magnit
 __device__ __forceinline__ float dot_h2(uint32_t a, float c) {   // c + the squares of both halves
   return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, a), __builtin_bit_cast(f16x2, a), c, false);
 }
-// A channel's scale (biased exponent) from its largest magnitude's E.
-__device__ __forceinline__ int g_scale_exp(int E, bool careful) {
-  const int e = (careful ? 268 : 257) - E;   // the largest below 2^15, the sample's below 2^4
-  return e < 1 ? 1 : (e > 251 ? 251 : e);
-}
+// A channel's scale (biased exponent) from the biased exponent of its sample's largest
+// magnitude, which lands below 2^4.
+__device__ __forceinline__ int g_scale_exp(int E) { return E < 6 ? 251 : 257 - E; }
 
 // Eight waves per wide tile, two per SIMD: waves (channel half gh, output quarter oq) each
 // own a 128 x 64 block (4 x 2 MFMA tiles, 128 accumulators), so one wave's MFMAs issue while
 // the other of its SIMD waits on LDS or staging.  The staging of a slab is split over 512
 // lanes, and a channel's squares over two lanes (k 0-15 and 16-31 of every slab), added once
-// at the end.  A lane's 16 squares of a slab are exact products summed in fp32 by
-// v_dot2_f32_f16; the slabs' sums accumulate in double.
+// at the end.  A lane's 16 squares of a slab are exact products summed in fp32 by a dot
+// instruction; the slabs' sums accumulate in double.
 template <bool RIGHT, bool FULL>
-__device__ __forceinline__ void proj_wide(const ApDesc& D, const ApL& L, int tile, uint16_t* gsl, u32x4* psl,
-                                          int* sexp, double* sred, int* bad) {
-  const int tid = threadIdx.x, l = tid & 63, l32 = l & 31, hi = l >> 5;
+struct Wide {
+  const uint16_t* G;
+  int64_t R, C, nch, ch0, nblk, nslab;
+  int pass;
+  uint16_t* gsl;   // LDS: two G slabs
+  u32x4* psl;      // LDS: two P slabs
+
+  // Piece i of 2 of the slab at k0, eight elements each.  Right: rows (tid >> 2) + 128 i, k
+  // at 8 (tid & 3).  Left: k rows 2 (tid & 15) + i, columns at 8 (tid >> 4), stored
+  // transposed as pairs of k in one 32-bit word.
+  __device__ __forceinline__ u32x4 ldG(int tid, int64_t k0, int i) const {
+    const int64_t row = RIGHT ? ch0 + (tid >> 2) + 128 * i : k0 + 2 * (tid & 15) + i;
+    const int64_t col = RIGHT ? k0 + 8 * (tid & 3) : ch0 + 8 * (tid >> 4);
+    if constexpr (FULL) return ldu(G, (uint32_t)((row * C + col) * 2));
+    const int64_t left = C - col;
+    return ldg8(G, row * C + col, row >= R || left <= 0 ? 0 : (left >= 8 ? 8 : (int)left));
+  }
+  // A wave's G fragment: sub-step j, channels 32 q + l % 32 of its half.
+  __device__ __forceinline__ u32x4 rdG(int b, int ch, int j, int hi) const {
+    return *reinterpret_cast<const u32x4*>(&gsl[b * kApWGh + ch * kApWS + 16 * hi + 8 * j]);
+  }
+  // Eight elements of a channel's row for its squares.
+  __device__ __forceinline__ u32x4 rdC(int b, int tid, int g) const {
+    return *reinterpret_cast<const u32x4*>(&gsl[b * kApWGh + (tid & 255) * kApWS + 16 * (tid >> 8) + 8 * g]);
+  }
+};
+
+__device__ __forceinline__ float bf_val(u32x4 f, int e) {   // element e of eight bf16
+  const uint32_t q = f[e >> 1];
+  return __uint_as_float((e & 1) ? (q & 0xFFFF0000u) : (q << 16));
+}
+
+// The tile's slabs in fp16, from the first until one that does not fit; returns how many were
+// multiplied.  acc and nsq are in G's and P's own units on return.  sexp: int[2 kApW] of
+// LDS; bad: int[2], zero on entry (a barrier ago or not yet written).
+template <bool RIGHT, bool FULL>
+__device__ __forceinline__ int64_t wide_half(const Wide<RIGHT, FULL>& W, const u32x4* Ps, int pexp, int* sexp, int* bad,
+                                             f32x16 (&acc)[4][2], double& nsq) {
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));   // addresses shared with wide_exact's would spill
+  const int l = tid & 63, l32 = l & 31, hi = l >> 5;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int gh = w >> 2, oq = w & 3;   // the wave's channel half and output quarter
-  const int pass = (int)(tile / L.ntr);
-  const int64_t gt = tile - (int64_t)pass * L.ntr;
-  const int64_t R = D.R, C = D.C, r = D.r;
-  const int64_t K = RIGHT ? C : R, nch = RIGHT ? R : C;
-  const int64_t ch0 = gt * kApW;
-  const int64_t nblk = L.rp / 32;
-  const int64_t nslab = (K + 31) / 32;
-  const uint16_t* G = reinterpret_cast<const uint16_t*>(D.grad);
-  const u32x4* Ps = reinterpret_cast<const u32x4*>(D.ws + L.phalf);
-  const bool pass0 = pass == 0;
-  f32x16 acc[4][2];
-  double nsq = 0.0;   // scaled squares of channel ch0 + (tid & 255), k half tid >> 8
-  for (int round = 0;;) {   // 0: two slabs sampled, 1: nine, 2: all
-    const bool careful = round == 2;
-    int tid = threadIdx.x;
-    asm volatile("" : "+v"(tid));   // the addresses below are made again: hoisted out of this loop, they spill
-    const int l = tid & 63, l32 = l & 31, hi = l >> 5;
-    // G loader, piece i of 2, eight elements each.  Right: rows (tid >> 2) + 128 i, k at
-    // 8 (tid & 3).  Left: k rows 2 (tid & 15) + i, columns at 8 (tid >> 4), stored transposed
-    // as pairs of k in one 32-bit word.
-    auto ldG1 = [&](int64_t k0, int i, u32x4* f) {
-      const int64_t row = RIGHT ? ch0 + (tid >> 2) + 128 * i : k0 + 2 * (tid & 15) + i;
-      const int64_t col = RIGHT ? k0 + 8 * (tid & 3) : ch0 + 8 * (tid >> 4);
-      const int64_t left = C - col;
-      const int cnt = row >= R || left <= 0 ? 0 : (left >= 8 ? 8 : (int)left);
-      if constexpr (FULL) f[i] = ldu(G, (uint32_t)((row * C + col) * 2));
-      else f[i] = ldg8(G, row * C + col, cnt);
-    };
-    auto val = [&](const u32x4* f, int i, int e) -> float {   // element e of piece i
-      const uint32_t q = f[i][e >> 1];
-      return __uint_as_float((e & 1) ? (q & 0xFFFF0000u) : (q << 16));
-    };
-    // P: units tid + 512 i of the slab's 2048 (term i / 2)
-    auto ldP1 = [&](int64_t kc, int i) -> u32x4 {
-      return gp(Ps)[((kc * 2 + (i >> 1)) * nblk + 8 * pass) * 128 + tid + 512 * (i & 1)];
-    };
-    constexpr int NC = RIGHT ? 2 : 8;   // channels that this lane stages
-    auto lane_ch = [&](int c) { return RIGHT ? (tid >> 2) + 128 * c : 8 * (tid >> 4) + c; };
-    u32x4 fg[2], fp[4];   // a slab between its loads and its LDS stores
-    float sc[NC];           // the scales of the lane's channels
-    {
-      // largest finite magnitudes of the lane's channels
-      uint32_t m[NC] = {};
-      auto seen = [&](const u32x4* f) {
+  const int64_t nslab = W.nslab;
+  // P: units tid + 512 i of the slab's 2048 (term i / 2)
+  auto ldP1 = [&](int64_t kc, int i) -> u32x4 {
+    return gp(Ps)[((kc * 2 + (i >> 1)) * W.nblk + 8 * W.pass) * 128 + tid + 512 * (i & 1)];
+  };
+  constexpr int NC = RIGHT ? 2 : 8;   // channels that this lane stages
+  auto lane_ch = [&](int c) { return RIGHT ? (tid >> 2) + 128 * c : 8 * (tid >> 4) + c; };
+  u32x4 fg[2], fp[4];   // a slab between its loads and its LDS stores
+  float sc[NC];         // the scales of the lane's channels
+  {
+    // largest finite magnitudes of the lane's channels
+    uint32_t m[NC] = {};
+    auto seen = [&](const u32x4* f) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < 2; ++i)
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const uint32_t b = __float_as_uint(val(f, i, e)) & 0x7FFFFFFFu;
-            uint32_t& mc = m[RIGHT ? i : e];
-            mc = max_u(mc, b >= 0x7F800000u ? 0u : b);
-          }
-      };
-      ldG1(0, 0, fg);
-      ldG1(0, 1, fg);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) fp[i] = ldP1(0, i);
-      if (round) {
-        u32x4 f4[4][2];
-        const int64_t step = careful || nslab < 8 ? 1 : nslab >> 3;
-        for (int64_t s = step; s < nslab; s += 4 * step) {   // the last group's repeats change no maximum
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const int64_t sj = s + (j / 2) * step;
-            ldG1(32 * (sj < nslab ? sj : nslab - 1), j % 2, f4[j / 2]);
-          }
-#pragma unroll
-          for (int j = 0; j < 4; ++j) seen(f4[j]);
+        for (int e = 0; e < 8; ++e) {
+          const uint32_t b = __float_as_uint(bf_val(f[i], e)) & 0x7FFFFFFFu;
+          uint32_t& mc = m[RIGHT ? i : e];
+          mc = max_u(mc, b >= 0x7F800000u ? 0u : b);
         }
-      } else {
-        u32x4 f2[2];
-        ldG1(32 * (nslab >> 1), 0, f2);
-        ldG1(32 * (nslab >> 1), 1, f2);
-        seen(f2);
-      }
-      seen(fg);
+    };
+    u32x4 f2[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) fg[i] = W.ldG(tid, 0, i);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) fp[i] = ldP1(0, i);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) f2[i] = W.ldG(tid, 32 * (nslab >> 1), i);
+    seen(f2);
+    seen(fg);
+    auto publish = [&] {
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
 #pragma unroll
@@ -1019,159 +1004,327 @@ __device__ __forceinline__ void proj_wide(const ApDesc& D, const ApL& L, int til
 #pragma unroll
         for (int c = 0; c < NC; ++c) sexp[lane_ch(c)] = (int)(m[c] >> 23);
       }
+      __syncthreads();
+    };
+    publish();
+    bool zero = false;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) zero |= sexp[l + 64 * i] == 0 && W.ch0 + l + 64 * i < W.nch;
+    if (__ballot(zero)) {   // the same in every wave
+      u32x4 f3[3][2];
+#pragma unroll
+      for (int j = 0; j < 6; ++j) f3[j / 2][j % 2] = W.ldG(tid, 32 * ((nslab - 1) * (j / 2 < 2 ? 2 * (j / 2) + 1 : 4) / 4), j % 2);
+#pragma unroll
+      for (int j = 0; j < 3; ++j) seen(f3[j]);
+      __syncthreads();   // before sexp is written again
+      publish();
     }
-    __syncthreads();
-    {
-      if (round == 0) {
-        bool zero = false;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) zero |= sexp[l + 64 * i] == 0 && ch0 + l + 64 * i < nch;
-        if (__ballot(zero)) {   // the same in every wave
-          __syncthreads();      // before sexp is written again
-          round = 1;
-          continue;
-        }
-      }
-      auto scale_exp = [&](int ch) { return g_scale_exp(sexp[ch], careful); };
-#pragma unroll
-      for (int c = 0; c < NC; ++c) sc[c] = exp_f(scale_exp(lane_ch(c)));
-      if (tid < kApW) sexp[kApW + tid] = scale_exp(tid);
-    }
-    uint32_t mx = 0u;
-    auto scrubG = [&] {
-      fg[0] = scrub8(fg[0]);
-      fg[1] = scrub8(fg[1]);
-    };
-    // Word e of the lane's eight, two elements of one channel: to fp16, and to LDS (right: four
-    // words at a time).
-    u32x4 cw;
-    auto stG1 = [&](uint16_t* sl, int e) {
-      const int pc = e >> 2, i = e & 3;
-      float a = RIGHT ? val(fg, pc, 2 * i) : val(fg, 0, e), b = RIGHT ? val(fg, pc, 2 * i + 1) : val(fg, 1, e);
-      a *= sc[RIGHT ? pc : e];
-      b *= sc[RIGHT ? pc : e];
-      const uint32_t h = cvt_h2(a, b);
-      mx = max_h2(mx, h);
-      if constexpr (RIGHT) {
-        cw[i] = h;
-        if (i == 3) *reinterpret_cast<u32x4*>(&sl[((tid >> 2) + 128 * pc) * kApWS + 8 * (tid & 3)]) = cw;
-      } else {
-        *reinterpret_cast<uint32_t*>(&sl[(8 * (tid >> 4) + e) * kApWS + 2 * (tid & 15)]) = h;
-      }
-    };
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-      for (int c = 0; c < 2; ++c) acc[q][c] = f32x16{};
-    nsq = 0.0;
-    // One slab from LDS buffer b, 32 MFMAs, the other instructions placed between them in a
-    // fixed order (scheduling fences).  g0 and p0 hold sub-step 0's first fragments on entry.
-    // Sub-step 0 reads its later fragments, the squares' rows and sub-step 1's first
-    // fragments; around its end the next slab (whose global loads were issued most of a slab
-    // ago) is converted and stored to the other buffer, and the loads of the slab after it
-    // issued.  The slab's one barrier stands in sub-step 1, behind this slab's last LDS read
-    // and the next one's last store, with 8 MFMAs left to cover the next slab's first reads.
-    u32x4 g0[4], p0[2][2];
-    auto rdG = [&](int b, int j, int q) {
-      return *reinterpret_cast<const u32x4*>(&gsl[b * kApWGh + (gh * 128 + 32 * q + l32) * kApWS + 16 * hi + 8 * j]);
-    };
-    auto rdP = [&](int b, int j, int t, int c) { return psl[b * kApWPu + ((t * 8 + oq * 2 + c) * 2 + j) * 64 + l]; };
-    auto slab = [&](const int b, const int64_t kl, auto next) {
-      constexpr bool NEXT = decltype(next)::value;
-      uint16_t* gn = gsl + (b ^ 1) * kApWGh;
-      u32x4* pn = psl + (b ^ 1) * kApWPu;
-      u32x4 g1[4], p1[2][2], cr;
-      float sq16 = 0.0f;
-      auto mul = [&](const u32x4* g, const u32x4 (*p)[2], int m) {
-        const int t = m / 8, c = (m / 4) % 2, q = m % 4;
-        if constexpr (RIGHT) acc[q][c] = mfma_h(g[q], p[t][c], acc[q][c]);
-        else acc[q][c] = mfma_h(p[t][c], g[q], acc[q][c]);
-      };
-      auto stage = [&](int n) {   // slot n of the slab's 32
-        if constexpr (NEXT) {
-          if (n == 12 && careful) scrubG();
-          if (n >= 12 && n < 20) stG1(gn, n - 12);
-          if (n >= 20 && n < 24) {
-            const int i = n - 20;
-            if (i < 2) ldG1(kl * 32, i, fg);
-            pn[tid + 512 * i] = fp[i];
-            fp[i] = ldP1(kl, i);
-          }
-        }
-      };
-#pragma unroll
-      for (int m = 0; m < 16; ++m) {
-        mul(g0, p0, m);
-        if (m < 2) p0[1][m] = rdP(b, 0, 1, m);
-        if (m == 2 || m == 6)
-          cr = *reinterpret_cast<const u32x4*>(&gsl[b * kApWGh + (tid & 255) * kApWS + 16 * (tid >> 8) + 2 * (m - 2)]);
-        if (m == 4 || m == 5 || m == 8 || m == 9) {   // four squares
-          sq16 = dot_h2(cr[2 * (m & 1)], sq16);
-          sq16 = dot_h2(cr[2 * (m & 1) + 1], sq16);
-          if (m == 9) nsq += (double)sq16;
-        }
-        if (m >= 8 && m < 12) g1[m - 8] = rdG(b, 1, m - 8);
-        if (m >= 12 && m < 14) p1[0][m - 12] = rdP(b, 1, 0, m - 12);
-        stage(m);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-#pragma unroll
-      for (int m = 0; m < 16; ++m) {
-        mul(g1, p1, m);
-        if (m < 2) p1[1][m] = rdP(b, 1, 1, m);
-        stage(16 + m);
-        if constexpr (NEXT) {
-          if (m == 8) __syncthreads();
-          if (m >= 8 && m < 12) g0[m - 8] = rdG(b ^ 1, 0, m - 8);
-          if (m >= 12 && m < 14) p0[0][m - 12] = rdP(b ^ 1, 0, 0, m - 12);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    };
-    if (careful) scrubG();
-#pragma unroll
-    for (int e = 0; e < 8; ++e) stG1(gsl, e);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) psl[tid + 512 * i] = fp[i];
-    {
-      const int64_t k1 = nslab > 1 ? 1 : 0;
-#pragma unroll
-      for (int i = 0; i < 2; ++i) ldG1(32 * k1, i, fg);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) fp[i] = ldP1(k1, i);
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < 4; ++q) g0[q] = rdG(0, 0, q);
-#pragma unroll
-    for (int c = 0; c < 2; ++c) p0[0][c] = rdP(0, 0, 0, c);
-    for (int64_t s = 0; s + 1 < nslab; ++s)
-      slab((int)(s & 1), s + 2 < nslab ? s + 2 : nslab - 1, std::true_type{});
-    slab((int)((nslab - 1) & 1), 0, std::false_type{});
-    if (careful) break;
-    if ((mx & 0x7FFFu) >= 0x7C00u || (mx >> 16) >= 0x7C00u) *bad = 1;
-    __syncthreads();
-    if (!__builtin_amdgcn_readfirstlane(*bad)) break;
-    round = 2;
   }
-  float* glow = D.ws + L.glow;
-  const int pexp = 254 - (int)(__float_as_uint(gp(D.ws)[L.scal + 8]) >> 23);
-  const int* se = sexp + kApW;
-  const int64_t gx0 = ch0 + gh * 128, ox0 = (int64_t)pass * kApW + oq * 64;
+#pragma unroll
+  for (int c = 0; c < NC; ++c) sc[c] = exp_f(g_scale_exp(sexp[lane_ch(c)]));
+  if (tid < kApW) sexp[kApW + tid] = g_scale_exp(sexp[tid]);
+  uint32_t mx = 0u;
 #pragma unroll
   for (int q = 0; q < 4; ++q)
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      // the powers of two come off (see store_acc for an accumulator's rows)
+    for (int c = 0; c < 2; ++c) acc[q][c] = f32x16{};
+  nsq = 0.0;
+  // Word e of the lane's eight, two elements of one channel: to fp16, and to LDS (right: four
+  // words at a time).
+  u32x4 cw;
+  auto stG1 = [&](uint16_t* sl, const u32x4* f, int e) {
+    const int pc = e >> 2, i = e & 3;
+    float a = RIGHT ? bf_val(f[pc], 2 * i) : bf_val(f[0], e), b = RIGHT ? bf_val(f[pc], 2 * i + 1) : bf_val(f[1], e);
+    a *= sc[RIGHT ? pc : e];
+    b *= sc[RIGHT ? pc : e];
+    const uint32_t h = cvt_h2(a, b);
+    mx = max_h2(mx, h);
+    if constexpr (RIGHT) {
+      cw[i] = h;
+      if (i == 3) *reinterpret_cast<u32x4*>(&sl[((tid >> 2) + 128 * pc) * kApWS + 8 * (tid & 3)]) = cw;
+    } else {
+      *reinterpret_cast<uint32_t*>(&sl[(8 * (tid >> 4) + e) * kApWS + 2 * (tid & 15)]) = h;
+    }
+  };
+  // An fp16 exponent of all ones in either half: everything stored so far is in mx.
+  auto misfit = [&] { return ((mx + 0x04000400u) & 0x80008000u) != 0u; };
+  bool careful = false;   // G is scrubbed
+  // Slab s, whose bad[b] was set, anew; returns whether it fits without its non-finite values.
+  auto restage = [&](const int b, const int64_t s) -> bool {
+    u32x4 f[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) f[i] = scrub8(W.ldG(tid, 32 * s, i));
+    __syncthreads();   // every wave has read the slab's first fragments and bad
+    if (tid == 0) bad[b] = 0;
+    careful = true;
+    mx = 0u;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) stG1(W.gsl + b * kApWGh, f, e);
+    __syncthreads();
+    if (misfit()) bad[b] = 1;
+    __syncthreads();
+    return !__builtin_amdgcn_readfirstlane(bad[b]);
+  };
+  // One slab from LDS buffer b, 32 MFMAs, the other instructions placed between them in a
+  // fixed order (scheduling fences).  g0 and p0 hold sub-step 0's first fragments on entry.
+  // Sub-step 0 reads its later fragments, the squares' rows and sub-step 1's first
+  // fragments; around its end the next slab (whose global loads were issued most of a slab
+  // ago) is converted and stored to the other buffer, and the loads of the slab after it
+  // issued.  The slab's one barrier stands in sub-step 1, behind this slab's last LDS read
+  // and the next one's last store, with 8 MFMAs left to cover the next slab's first reads.
+  // Returns whether the next slab fits.  bad[b ^ 1] is written before the barrier and read
+  // behind it; the next slab's writers take the other word, and the slab after that stands
+  // behind another barrier, so every wave reads the same value.
+  u32x4 g0[4], p0[2][2];
+  auto rdP = [&](int b, int j, int t, int c) {
+    return W.psl[b * 2 * kApWPu + ((t * 8 + oq * 2 + c) * 2 + j) * 64 + l];
+  };
+  auto rdG = [&](int b, int j, int q) { return W.rdG(b, gh * 128 + 32 * q + l32, j, hi); };
+  auto slab = [&](const int b, const int64_t kl, auto next) -> bool {
+    constexpr bool NEXT = decltype(next)::value;
+    uint16_t* gn = W.gsl + (b ^ 1) * kApWGh;
+    u32x4* pn = W.psl + (b ^ 1) * 2 * kApWPu;
+    u32x4 g1[4], p1[2][2], cr;
+    float sq16 = 0.0f;
+    int odd = 0;
+    auto mul = [&](const u32x4* g, const u32x4 (*p)[2], int m) {
+      const int t = m / 8, c = (m / 4) % 2, q = m % 4;
+      if constexpr (RIGHT) acc[q][c] = mfma_h(g[q], p[t][c], acc[q][c]);
+      else acc[q][c] = mfma_h(p[t][c], g[q], acc[q][c]);
+    };
+    auto stage = [&](int n) {   // slot n of the slab's 32
+      if constexpr (NEXT) {
+        if (n == 12 && careful) {
+          fg[0] = scrub8(fg[0]);
+          fg[1] = scrub8(fg[1]);
+        }
+        if (n >= 12 && n < 20) stG1(gn, fg, n - 12);
+        if (n >= 20 && n < 24) {
+          const int i = n - 20;
+          if (i == 0 && misfit()) bad[b ^ 1] = 1;
+          if (i < 2) fg[i] = W.ldG(tid, kl * 32, i);
+          pn[tid + 512 * i] = fp[i];
+          fp[i] = ldP1(kl, i);
+        }
+      }
+    };
+#pragma unroll
+    for (int m = 0; m < 16; ++m) {
+      mul(g0, p0, m);
+      if (m < 2) p0[1][m] = rdP(b, 0, 1, m);
+      if (m == 2 || m == 6) cr = W.rdC(b, tid, (m - 2) / 4);
+      if (m == 4 || m == 5 || m == 8 || m == 9) {   // four squares
+        sq16 = dot_h2(cr[2 * (m & 1)], sq16);
+        sq16 = dot_h2(cr[2 * (m & 1) + 1], sq16);
+        if (m == 9) nsq += (double)sq16;
+      }
+      if (m >= 8 && m < 12) g1[m - 8] = rdG(b, 1, m - 8);
+      if (m >= 12 && m < 14) p1[0][m - 12] = rdP(b, 1, 0, m - 12);
+      stage(m);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int m = 0; m < 16; ++m) {
+      mul(g1, p1, m);
+      if (m < 2) p1[1][m] = rdP(b, 1, 1, m);
+      stage(16 + m);
+      if constexpr (NEXT) {
+        if (m == 8) {
+          __syncthreads();
+          odd = bad[b ^ 1];
+        }
+        if (m >= 8 && m < 12) g0[m - 8] = rdG(b ^ 1, 0, m - 8);
+        if (m >= 12 && m < 14) p0[0][m - 12] = rdP(b ^ 1, 0, 0, m - 12);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    return !__builtin_amdgcn_readfirstlane(odd);
+  };
+#pragma unroll
+  for (int e = 0; e < 8; ++e) stG1(W.gsl, fg, e);
+  if (misfit()) bad[0] = 1;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) W.psl[tid + 512 * i] = fp[i];
+  {
+    const int64_t k1 = nslab > 1 ? 1 : 0;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) fg[i] = W.ldG(tid, 32 * k1, i);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) fp[i] = ldP1(k1, i);
+  }
+  __syncthreads();
+  // the loop has one exit: with two, the accumulators are copied and spill
+  int64_t s = 0, end = nslab;
+  if (__builtin_amdgcn_readfirstlane(bad[0]) && !restage(0, 0)) end = 0;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) g0[q] = rdG(0, 0, q);
+#pragma unroll
+  for (int c = 0; c < 2; ++c) p0[0][c] = rdP(0, 0, 0, c);
+  for (; s + 1 < end; ++s) {
+    const int b = (int)(s & 1);
+    if (!slab(b, s + 2 < nslab ? s + 2 : nslab - 1, std::true_type{})) {
+      if (!restage(b ^ 1, s + 1)) end = s + 1;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) g0[q] = rdG(b ^ 1, 0, q);
+    }
+  }
+  if (end == nslab) {
+    slab((int)(s & 1), 0, std::false_type{});
+    s = nslab;
+  }
+  // the powers of two come off (see store_acc for an accumulator's rows)
+  const int* se = sexp + kApW;
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         const int ch = gh * 128 + 32 * q + (RIGHT ? 8 * (v >> 2) + 4 * hi + (v & 3) : l32);
         acc[q][c][v] = __builtin_amdgcn_ldexpf(acc[q][c][v], pexp - se[ch]);
       }
+  nsq = ldexp(nsq, 2 * (127 - se[tid & 255]));
+  return s;
+}
+
+// The tile's slabs from s0 on (any of them) added to acc and nsq: bf16 G, scrubbed, against the
+// three bf16 terms of P, which hold it exactly.
+template <bool RIGHT, bool FULL>
+__device__ __forceinline__ void wide_exact(const Wide<RIGHT, FULL>& W, const u32x4* Ps, int64_t s0, f32x16 (&acc)[4][2],
+                                           double& nsq) {
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));   // addresses shared with wide_half's would spill
+  const int l = tid & 63, l32 = l & 31, hi = l >> 5;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int gh = w >> 2, oq = w & 3;
+  // P: units tid + 512 i of the slab's 3072 (term i / 2)
+  auto ldP1 = [&](int64_t kc, int i) -> u32x4 {
+    return gp(Ps)[((kc * 3 + (i >> 1)) * W.nblk + 8 * W.pass) * 128 + tid + 512 * (i & 1)];
+  };
+  u32x4 fg[2], fp[6];   // the next slab, between its loads and its LDS stores
+  // G store, piece i of 2: right, row piece i; left, columns 4 i .. 4 i + 3 of the lane's
+  // eight (both k rows)
+  auto stG1 = [&](uint16_t* sl, int i) {
+    if constexpr (RIGHT) {
+      *reinterpret_cast<u32x4*>(&sl[((tid >> 2) + 128 * i) * kApWS + 8 * (tid & 3)]) = scrub8(fg[i]);
+    } else {
+      const u32x4 a = scrub8(fg[0]), b = scrub8(fg[1]);   // two k rows
+#pragma unroll
+      for (int e = 4 * i; e < 4 * i + 4; ++e) {
+        const uint32_t lo = (e & 1) ? (a[e >> 1] >> 16) : (a[e >> 1] & 0xFFFFu);
+        const uint32_t hv = (e & 1) ? (b[e >> 1] & 0xFFFF0000u) : (b[e >> 1] << 16);
+        *reinterpret_cast<uint32_t*>(&sl[(8 * (tid >> 4) + e) * kApWS + 2 * (tid & 15)]) = lo | hv;
+      }
+    }
+  };
+  // One slab from LDS buffer b, 48 MFMAs, the other instructions placed between them:
+  //   before MFMA 0: sub-step 0's G fragments, its first P term, the channel-row reads;
+  //   sub-step 0 (MFMAs 0-23): the squares (m < 8), P terms 1-2 (m 0-3), the next slab's 8
+  //     global loads (m 4-11), sub-step 1's G fragments (m 12-15) and P terms 0-1 (m 16-19);
+  //   sub-step 1 (MFMAs 24-47): its P term 2 (m 0-1), then after every third MFMA one of the
+  //     next slab's 8 LDS stores (6 P units, 2 G pieces).
+  auto slab = [&](const int b, const int64_t kn, auto next) {
+    constexpr bool NEXT = decltype(next)::value;
+    uint16_t* gn = W.gsl + (b ^ 1) * kApWGh;
+    u32x4* pn = W.psl + (b ^ 1) * 3 * kApWPu;
+    u32x4 ga[4], gb[4], pa[3][2], pb[3][2], cr[2];
+    float sq16 = 0.0f;
+    auto rdG = [&](int j, int q) { return W.rdG(b, gh * 128 + 32 * q + l32, j, hi); };
+    auto rdP = [&](int j, int t, int c) {
+      return W.psl[b * 3 * kApWPu + ((t * 8 + oq * 2 + c) * 2 + j) * 64 + l];
+    };
+    auto mul = [&](const u32x4* g, const u32x4 (*p)[2], int m) {
+      const int t = m / 8, c = (m / 4) % 2, q = m % 4;
+      if constexpr (RIGHT) acc[q][c] = mfma(as_bf8(g[q]), as_bf8(p[t][c]), acc[q][c]);
+      else acc[q][c] = mfma(as_bf8(p[t][c]), as_bf8(g[q]), acc[q][c]);
+    };
+#pragma unroll
+    for (int q = 0; q < 4; ++q) ga[q] = rdG(0, q);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) pa[0][c] = rdP(0, 0, c);
+    cr[0] = W.rdC(b, tid, 0);
+    cr[1] = W.rdC(b, tid, 1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int m = 0; m < 24; ++m) {
+      mul(ga, pa, m);
+      if (m < 8) {   // two squares per MFMA, the slab's 16 in fp32, then into double
+        const bf16x2 c2 = __builtin_bit_cast(bf16x2, (uint32_t)cr[m / 4][m % 4]);
+        sq16 = __builtin_amdgcn_fdot2_f32_bf16(c2, c2, sq16, false);
+        if (m == 7) nsq += (double)sq16;
+      }
+      if (m < 4) {
+        pa[1 + m / 2][m % 2] = rdP(0, 1 + m / 2, m % 2);
+      } else if (m < 12) {
+        if constexpr (NEXT) {
+          if (m < 10) fp[m - 4] = ldP1(kn, m - 4);
+          else fg[m - 10] = W.ldG(tid, 32 * kn, m - 10);
+        }
+      } else if (m < 16) {
+        gb[m - 12] = rdG(1, m - 12);
+      } else if (m < 20) {
+        pb[(m - 16) / 2][m % 2] = rdP(1, (m - 16) / 2, m % 2);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int m = 0; m < 24; ++m) {
+      mul(gb, pb, m);
+      if (m < 2) pb[2][m] = rdP(1, 2, m);
+      if constexpr (NEXT) {
+        if (m % 3 == 2) {
+          const int pc = m / 3;
+          if (pc < 6) pn[tid + 512 * pc] = fp[pc];
+          else stG1(gn, pc - 6);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  __syncthreads();   // wide_half's last LDS reads
+#pragma unroll
+  for (int i = 0; i < 2; ++i) fg[i] = W.ldG(tid, 32 * s0, i);
+#pragma unroll
+  for (int i = 0; i < 6; ++i) W.psl[tid + 512 * i] = ldP1(s0, i);
+  stG1(W.gsl, 0);
+  stG1(W.gsl, 1);
+  __syncthreads();
+  // a slab's LDS stores go to the other buffer, whose readers finished before the last barrier
+  int b = 0;
+  for (int64_t s = s0; s + 1 < W.nslab; ++s, b ^= 1) {
+    slab(b, s + 1, std::true_type{});
+    __syncthreads();
+  }
+  slab(b, 0, std::false_type{});
+}
+
+template <bool RIGHT, bool FULL>
+__device__ __forceinline__ void proj_wide(const ApDesc& D, const ApL& L, int tile, uint16_t* gsl, u32x4* psl,
+                                          int* sexp, double* sred, int* bad) {
+  const int tid = threadIdx.x, l = tid & 63, l32 = l & 31, hi = l >> 5;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int gh = w >> 2, oq = w & 3;
+  const int pass = (int)(tile / L.ntr);
+  const int64_t gt = tile - (int64_t)pass * L.ntr;
+  const int64_t R = D.R, C = D.C, r = D.r;
+  const int64_t ch0 = gt * kApW, nch = RIGHT ? R : C;
+  const Wide<RIGHT, FULL> W{reinterpret_cast<const uint16_t*>(D.grad), R, C, nch, ch0, L.rp / 32,
+                            ((RIGHT ? C : R) + 31) / 32, pass, gsl, psl};
+  f32x16 acc[4][2];
+  double nsq;   // squares of channel ch0 + (tid & 255), k half tid >> 8
+  const int pexp = 254 - (int)(__float_as_uint(gp(D.ws)[L.scal + 8]) >> 23);
+  const int64_t s = wide_half(W, reinterpret_cast<const u32x4*>(D.ws + L.phalf), pexp, sexp, bad, acc, nsq);
+  if (s < W.nslab) wide_exact(W, reinterpret_cast<const u32x4*>(D.ws + L.psplit), s, acc, nsq);
+  float* glow = D.ws + L.glow;
+  const int64_t gx0 = ch0 + gh * 128, ox0 = (int64_t)pass * kApW + oq * 64;
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
       if constexpr (RIGHT) store_acc(acc[q][c], glow, r, gx0 + 32 * q, ox0 + 32 * c + l32, R, r, hi);
       else store_acc(acc[q][c], glow, C, ox0 + 32 * c, gx0 + 32 * q + l32, r, C, hi);
     }
-  if (!pass0) return;
+  if (pass != 0) return;
   // a channel's two k halves, then the tile's channels in the order of four waves
   double* half1 = sred + 8;
   if (tid >= kApW) half1[tid - kApW] = nsq;
@@ -1180,7 +1333,7 @@ __device__ __forceinline__ void proj_wide(const ApDesc& D, const ApL& L, int til
   if (tid < kApW) {
     const int64_t ch = ch0 + tid;
     if (ch < nch) {
-      tot = ldexp(nsq + half1[tid], 2 * (127 - se[tid]));
+      tot = nsq + half1[tid];
       gp(D.ws + L.ngsq)[ch] = norm_sq(tot);
     }
   }
@@ -1568,7 +1721,7 @@ void k_ap_proj_l(ApDesc one, const ApDesc* tab, int ntab) {
   }
 }
 
-// Wide tiles of both sides, eight waves (one workgroup per CU: 108 KB of LDS).
+// Wide tiles of both sides, eight waves (one workgroup per CU: 140 KB of LDS).
 // Workgroups are dealt to the 8 XCDs round-robin by index; XCD x takes the
 // contiguous tile range [start[x], start[x + 1]) in order (its L2 then holds
 // the P split of one or two matrices at a time).  The host cuts the ranges at
@@ -1580,10 +1733,10 @@ struct ApXcd {
 };
 __global__ __launch_bounds__(512) void k_ap_proj_w(ApDesc one, const ApDesc* tab, int ntab, ApXcd xs) {
   __shared__ __attribute__((aligned(16))) uint16_t gsl[2 * kApWGh];
-  __shared__ u32x4 psl[2 * kApWPu];
+  __shared__ u32x4 psl[2 * 3 * kApWPu];
   __shared__ double sred[8 + kApW];
   __shared__ int sexp[2 * kApW];
-  __shared__ int bad;
+  __shared__ int bad[2];
   const int x = (int)blockIdx.x % 8;
   const int wg = xs.start[x] + (int)blockIdx.x / 8;
   if (wg >= xs.start[x + 1]) return;
@@ -1591,10 +1744,10 @@ __global__ __launch_bounds__(512) void k_ap_proj_w(ApDesc one, const ApDesc* tab
   const ApDesc D = ap_pick(one, tab, ntab, 5, wg, local);
   const ApL L = ap_layout(D.R, D.C, D.r, D.trows);
   const int64_t ch0 = (local % L.ntr) * kApW;
-  if (threadIdx.x == 0) bad = 0;
+  if (threadIdx.x < 2) bad[threadIdx.x] = 0;
   auto tile = [&](auto right, auto full) {
     constexpr bool R = decltype(right)::value, F = decltype(full)::value;
-    proj_wide<R, F>(D, L, local, gsl, psl, sexp, sred, &bad);
+    proj_wide<R, F>(D, L, local, gsl, psl, sexp, sred, bad);
   };
   if (D.R >= D.C) {
     if (D.valign && ch0 + kApW <= D.R && D.C % 32 == 0) tile(std::true_type{}, std::true_type{});
