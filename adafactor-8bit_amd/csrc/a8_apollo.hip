@@ -54,6 +54,7 @@ constexpr int kApRuns = 2;      // runs of eight elements per k_ap_apply lane (4
 constexpr int kApApp = 2048 * kApRuns;   // matrix elements per k_ap_apply workgroup
 
 constexpr int kApWide = 256;     // channels per wide projection tile (bf16 G, rank % 256 == 0)
+constexpr int kPMax = 64;        // workgroups that split one P^T for wide tiles, at most (their maxima: ApL::pmax)
 static_assert(kApWide == kApPass, "a wide tile covers one output pass");
 
 // G channels per projection tile of a matrix: wide tiles for bf16 G at ranks
@@ -67,7 +68,7 @@ __host__ __device__ inline int64_t ap_tile(bool g16, int64_t R, int64_t C, int64
 // Workspace of one matrix (offsets in floats; partial arrays hold doubles).
 struct ApL {
   int64_t n_low, nchg, K, Kp, rp, ntr, npass, ntile, nunit, nsc, napp;
-  int64_t glow, u, ngsq, fin, scal, gpart, ppart, spart, psplit, phalf, total;
+  int64_t glow, u, ngsq, fin, scal, gpart, ppart, spart, psplit, phalf, pmax, total;
 };
 
 // trows: G channels (rows on the right side, columns on the left) per projection
@@ -97,7 +98,9 @@ __host__ __device__ inline ApL ap_layout(int64_t R, int64_t C, int64_t r, int64_
   // tiles change with G's type and with the group)
   w.psplit = (w.scal + 16 + 63) / 64 * 64;
   w.phalf = w.psplit + 3 * w.rp * w.Kp / 2;   // rp % 32 == 0 and Kp % 64 == 0: 16-byte aligned
-  w.gpart = w.phalf + (r % kApWide == 0 ? w.rp * w.Kp : 0);   // double[ntr]  ||G||^2 per tile
+  const bool half = r % kApWide == 0;
+  w.pmax = w.phalf + (half ? w.rp * w.Kp : 0);   // P's largest magnitude, in kPMax parts
+  w.gpart = w.pmax + (half ? kPMax : 0);   // double[ntr]  ||G||^2 per tile
   w.ppart = w.gpart + 2 * w.ntr;           // double[ntr]  ||p||^2 per tile
   w.spart = w.ppart + 2 * w.ntr;           // double[3 nsc] sum ngsq s^2, sum u^2, sum g_low^2
   w.total = w.spart + 6 * w.nsc;
@@ -105,8 +108,7 @@ __host__ __device__ inline ApL ap_layout(int64_t R, int64_t C, int64_t r, int64_
 }
 
 // Scalars in ApL::scal: [0] step (-alpha/denom, bias-corrected), [1] decay,
-// [3] tensor final scale, [4] alpha, [5] norm_unscaled, [6] fira scale; kept with P's
-// split: [8] the power of two by which the fp16 split is scaled.
+// [3] tensor final scale, [4] alpha, [5] norm_unscaled, [6] fira scale.
 
 // One matrix.  Read through the scalar cache: 8-byte words only.
 struct ApDesc {
@@ -271,34 +273,39 @@ __device__ __forceinline__ int64_t psw_unit(int64_t t, int64_t blk, int64_t kc, 
 }
 
 // ---- the fp16 split of the wide tiles
-// P times a power of two (its largest element then in [2^10, 2^11)) as hi + lo, each rounded
-// to the nearest fp16.  The residual x - hi spans 13 signed bits of x's last place and lo
-// keeps 12 of them, so the sum is x itself for three quarters of the values and one unit of
-// x's 24th bit off for the rest (2^-25 of the largest element at worst for values below
-// 2^-13 of it).  Two MFMA terms in place of the exact bf16 split's three.
-
-// E: biased exponent of the largest magnitude (0: all zero).  The scale's biased exponent.
-__device__ __forceinline__ int p_scale_exp(int E) {
-  const int e = 264 - E;
-  return e < 10 ? 10 : (e > 244 ? 244 : e);
+// P times a power of two as hi + lo, each rounded to the nearest fp16.  The residual x - hi
+// spans 13 signed bits of x's last place and lo keeps 12 of them, so the sum is x itself for
+// three quarters of the values and one unit of x's 24th bit off for the rest (2^-25 where
+// the scaled value is below 2^-2).  Two MFMA terms in place of the exact bf16 split's three.
+//
+// The power depends on the rank alone, so that a split depends on P^T alone, however it got
+// here (drawn on the device, given by the host, read from a checkpoint): it takes the
+// generator's largest value, |z| <= sqrt(106 ln 2) < 8.6 (Box-Muller from 53 bits) over
+// sqrt(r), to [2^14, 2^15).  A P^T whose largest element lands outside [2^10, 65504] (no
+// Gaussian of 256 values and more does) is taken by its three bf16 terms.
+__device__ __forceinline__ int p_scale_exp(int64_t r) {   // biased exponent
+  return 268 - (int)(__float_as_uint(8.6f / (float)sqrt((double)r)) >> 23);
 }
 __device__ __forceinline__ float exp_f(int biased) { return __uint_as_float((uint32_t)biased << 23); }
 __device__ __forceinline__ uint32_t h_bits(_Float16 h) { return (uint32_t)__builtin_bit_cast(unsigned short, h); }
 
+__device__ __forceinline__ uint32_t max_u(uint32_t a, uint32_t b) { return a > b ? a : b; }
+
 // One 16-byte unit u of each split, from P^T values pv(row, k): three bf16 terms to out, and if
 // half is set two fp16 terms of s times the value there, in the same order with two terms to
-// a chunk.
+// a chunk.  Returns the bits of the unit's largest magnitude.
 template <typename PV>
-__device__ __forceinline__ void split_unit(int64_t u, int64_t nblk, int64_t nkc, int64_t r, int64_t K, PV pv,
+__device__ __forceinline__ uint32_t split_unit(int64_t u, int64_t nblk, int64_t nkc, int64_t r, int64_t K, PV pv,
                                            u32x4* __restrict__ out, u32x4* __restrict__ half, float s) {
   const int l = (int)(u & 63), j = (int)((u >> 6) & 1);
   const int64_t c = u >> 7, kc = c % nkc, blk = c / nkc;
   const int64_t row = 32 * blk + (l & 31), k0 = 32 * kc + 16 * (l >> 5) + 8 * j;
-  uint32_t w[3][4] = {}, v[2][4] = {};
+  uint32_t w[3][4] = {}, v[2][4] = {}, mx = 0u;
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     const int64_t k = k0 + e;
     const float x = (row < r && k < K) ? pv(row, k) : 0.0f;
+    mx = max_u(mx, __float_as_uint(x) & 0x7FFFFFFFu);
     const __hip_bfloat16 h = __float2bfloat16(x);
     const float r1 = x - __bfloat162float(h);
     const __hip_bfloat16 m = __float2bfloat16(r1);
@@ -318,13 +325,14 @@ __device__ __forceinline__ void split_unit(int64_t u, int64_t nblk, int64_t nkc,
 #pragma unroll
   for (int t = 0; t < 3; ++t)
     gp(out)[psw_unit(t, blk, kc, j, l, nblk, nkc)] = u32x4{w[t][0], w[t][1], w[t][2], w[t][3]};
-  if (!half) return;
+  if (half) {
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
-    gp(half)[(((kc * 2 + t) * nblk + blk) * 2 + j) * 64 + l] = u32x4{v[t][0], v[t][1], v[t][2], v[t][3]};
+    for (int t = 0; t < 2; ++t)
+      gp(half)[(((kc * 2 + t) * nblk + blk) * 2 + j) * 64 + l] = u32x4{v[t][0], v[t][1], v[t][2], v[t][3]};
+  }
+  return mx;
 }
 
-__device__ __forceinline__ uint32_t max_u(uint32_t a, uint32_t b) { return a > b ? a : b; }
 // Largest x of 256 lanes; every lane gets it.
 __device__ __forceinline__ uint32_t wg_max_u(uint32_t x, uint32_t* s4) {
 #pragma unroll
@@ -333,27 +341,22 @@ __device__ __forceinline__ uint32_t wg_max_u(uint32_t x, uint32_t* s4) {
   __syncthreads();
   return max_u(max_u(s4[0], s4[1]), max_u(s4[2], s4[3]));
 }
-// Magnitude bits of the largest of pt[i0], pt[i0 + step], ... below n.
-__device__ __forceinline__ uint32_t abs_max(const float* pt, int64_t i0, int64_t step, int64_t n) {
-  uint32_t m = 0u;
-  for (int64_t i = i0; i < n; i += step) m = max_u(m, __float_as_uint(gp(pt)[i]) & 0x7FFFFFFFu);
-  return m;
+// Workgroup slot of per (at most kPMax) leaves its part's largest magnitude.
+__device__ __forceinline__ void put_pmax(float* ws, const ApL& L, int slot, int per, uint32_t m, uint32_t* s4) {
+  m = wg_max_u(m, s4);
+  if (threadIdx.x == 0)
+    for (int i = slot; i < kPMax; i += per) gp(ws)[L.pmax + i] = __uint_as_float(m);
+}
+// Whether P^T's fp16 split holds it (every lane of a wave calls it).
+__device__ __forceinline__ bool half_fits(const float* ws, const ApL& L, int pe) {
+  uint32_t m = __float_as_uint(gp(ws)[L.pmax + (threadIdx.x & 63)]);
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) m = max_u(m, __shfl_xor(m, d, 64));
+  const float x = __uint_as_float(m) * exp_f(pe);
+  return x >= 1024.0f && x <= 65504.0f;
 }
 
-// Before k_ap_split at the ranks of wide tiles: kPMax workgroups' maxima of P^T, in the head
-// of the workspace's u (written later in the step; rank >= 256, so it holds them).  Both
-// kernels take one matrix or a table of them, kPMax and `per` workgroups each.
-constexpr int kPMax = 64;
-__global__ __launch_bounds__(256) void k_ap_pmax(ApDesc one, const ApDesc* tab) {
-  const ApDesc D = tab ? tab[blockIdx.x / kPMax] : one;
-  if (D.r % kApWide != 0) return;
-  __shared__ uint32_t s4[4];
-  const ApL L = ap_layout(D.R, D.C, D.r, D.trows);
-  const int slot = (int)blockIdx.x % kPMax;
-  const uint32_t m = wg_max_u(abs_max(D.proj_t, slot * 256 + (int)threadIdx.x, kPMax * 256, D.r * L.K), s4);
-  if (threadIdx.x == 0) gp(D.ws)[L.u + slot] = __uint_as_float(m);
-}
-
+// One matrix or a table of them, `per` workgroups each.
 __global__ __launch_bounds__(256) void k_ap_split(ApDesc one, const ApDesc* tab, int per) {
   const ApDesc D = tab ? tab[blockIdx.x / per] : one;
   __shared__ uint32_t s4[4];
@@ -365,15 +368,12 @@ __global__ __launch_bounds__(256) void k_ap_split(ApDesc one, const ApDesc* tab,
   u32x4* out = reinterpret_cast<u32x4*>(D.ws + L.psplit);
   auto pv = [&](int64_t row, int64_t k) { return right ? gp(pt)[k * r + row] : gp(pt)[row * K + k]; };
   const int64_t u0 = (int64_t)(blockIdx.x % per) * 256 + threadIdx.x, step = (int64_t)per * 256;
-  float s = 1.0f;
-  u32x4* half = nullptr;
-  if (r % kApWide == 0) {
-    const uint32_t m = wg_max_u(__float_as_uint(gp(D.ws)[L.u + threadIdx.x % kPMax]), s4);
-    s = exp_f(p_scale_exp((int)(m >> 23)));
-    if (u0 == 0) gp(D.ws)[L.scal + 8] = s;
-    half = reinterpret_cast<u32x4*>(D.ws + L.phalf);
-  }
-  for (int64_t u = u0; u < nu; u += step) split_unit(u, nblk, nkc, r, K, pv, out, half, s);
+  const bool wide = r % kApWide == 0;
+  u32x4* half = wide ? reinterpret_cast<u32x4*>(D.ws + L.phalf) : nullptr;
+  const float s = exp_f(p_scale_exp(r));
+  uint32_t mx = 0u;
+  for (int64_t u = u0; u < nu; u += step) mx = max_u(mx, split_unit(u, nblk, nkc, r, K, pv, out, half, s));
+  if (wide) put_pmax(D.ws, L, (int)(blockIdx.x % per), per, mx, s4);
 }
 
 // ------------------------------------------------------------ device projection schedule
@@ -467,17 +467,11 @@ __global__ __launch_bounds__(256) void k_ap_pgen(ApDesc one, const ApDesc* tab, 
   float* pt = const_cast<float*>(D.proj_t);
   const uint64_t seed = (uint64_t)gp(D.pstate)[2];
   const float rsq = (float)sqrt((double)r);
-  // a wide tile's scale: from P as given, or for a generated P from its bound (Box-Muller
-  // from 53 bits: |z| <= sqrt(106 ln 2) < 8.6)
   __shared__ uint32_t s4[4];
-  float s = 1.0f;
-  u32x4* half = nullptr;
-  if (r % kApWide == 0) {
-    const uint32_t m = fresh == 1 ? __float_as_uint(8.6f / rsq) : wg_max_u(abs_max(pt, threadIdx.x, 256, r * K), s4);
-    s = exp_f(p_scale_exp((int)(m >> 23)));
-    if (slot == 0 && threadIdx.x == 0) gp(D.ws)[L.scal + 8] = s;
-    half = reinterpret_cast<u32x4*>(D.ws + L.phalf);
-  }
+  const bool wide = r % kApWide == 0;
+  u32x4* half = wide ? reinterpret_cast<u32x4*>(D.ws + L.phalf) : nullptr;
+  const float s = exp_f(p_scale_exp(r));
+  uint32_t mx = 0u;
   for (int64_t u = (int64_t)slot * 256 + threadIdx.x; u < nu; u += (int64_t)kPGen * 256) {
     if (fresh == 1) {
       auto pv = [&](int64_t row, int64_t k) {
@@ -486,12 +480,13 @@ __global__ __launch_bounds__(256) void k_ap_pgen(ApDesc one, const ApDesc* tab, 
         gp(pt)[right ? k * r + row : row * K + k] = v;
         return v;
       };
-      split_unit(u, nblk, nkc, r, K, pv, out, half, s);
+      mx = max_u(mx, split_unit(u, nblk, nkc, r, K, pv, out, half, s));
     } else {
       auto pv = [&](int64_t row, int64_t k) { return right ? gp(pt)[k * r + row] : gp(pt)[row * K + k]; };
-      split_unit(u, nblk, nkc, r, K, pv, out, half, s);
+      mx = max_u(mx, split_unit(u, nblk, nkc, r, K, pv, out, half, s));
     }
   }
+  if (wide) put_pmax(D.ws, L, slot, kPGen, mx, s4);
 }
 
 // a8_apollo_proj_gen: P^T of one matrix with the generator above.
@@ -886,6 +881,16 @@ __device__ __forceinline__ void proj_left(const ApDesc& D, const ApL& L, int til
 // if that does not fit, wide_exact takes the tile from this slab on: G as it is, scrubbed,
 // against P in three exact bf16 terms.
 //
+// P's fp16 split errs by at most a unit of an element's 24th bit, but a third of the
+// accumulator's roundings falls away with the third term, and from 48 products on they weigh
+// more: against 64 bits g_low's rms error is 1.06 times the bf16 terms' at K = 32, 1.00 at
+// 48, 0.98 at 64, 0.90 at 256 (1.55e-7 of g_low's rms), 0.84 at 2048 (4.1e-7) and 0.83 at
+// 8192, for normal, heavy-tailed, one-signed and log-uniform gradients on either side, so
+// wide_half takes K >= 48.  Exact zeros round nothing: a channel of a longer K with 9
+// non-zero products or more errs less as well (0.97), one with 5 errs 1.03 times as much
+// (7.5e-8), one with a single product 5.0e-8 in place of 3.3e-8 of its rms (a rounding to
+// fp32 alone: 2.6e-8 rms, 6.0e-8 at most).
+//
 // Four matrices of 32000 x 2048 at rank 256, a step (in brackets with three bf16 terms from
 // the first slab on): normal gradients 761 us (836), nine tenths of the rows zero 713 (780),
 // an element in ten of each row 667 (745), one in a hundred 752 (734), a value above 2^12 of
@@ -893,6 +898,7 @@ __device__ __forceinline__ void proj_left(const ApDesc& D, const ApL& L, int til
 constexpr int kApW = kApWide;             // channels and outputs of a wide tile
 constexpr int kApWS = 40;                 // LDS row stride (halves) of the G slab: 32 k + 8 pad
 constexpr int kApWGh = kApW * kApWS;      // halves per G slab buffer (20 KB)
+constexpr int kApHalfK = 48;              // shortest sums of wide_half
 constexpr int kApWPu = 8 * 2 * 64;        // 16-byte P units per slab and term: 8 blocks x 2 j x 64 lanes (16 KB)
 
 __device__ __forceinline__ f32x16 mfma_h(u32x4 a, u32x4 b, f32x16 c) {
@@ -954,9 +960,10 @@ __device__ __forceinline__ float bf_val(u32x4 f, int e) {   // element e of eigh
 
 // The tile's slabs in fp16, from the first until one that does not fit; returns how many were
 // multiplied.  acc and nsq are in G's and P's own units on return.  sexp: int[2 kApW] of
-// LDS; bad: int[2], zero on entry (a barrier ago or not yet written).
+// LDS; bad: int[4], set by the first wave: two words for slabs that do not fit (0), whether it
+// does not take P (its range or K), and the power of two of its split.
 template <bool RIGHT, bool FULL>
-__device__ __forceinline__ int64_t wide_half(const Wide<RIGHT, FULL>& W, const u32x4* Ps, int pexp, int* sexp, int* bad,
+__device__ __forceinline__ int64_t wide_half(const Wide<RIGHT, FULL>& W, const u32x4* Ps, int* sexp, int* bad,
                                              f32x16 (&acc)[4][2], double& nsq) {
   int tid = threadIdx.x;
   asm volatile("" : "+v"(tid));   // addresses shared with wide_exact's would spill
@@ -1156,6 +1163,7 @@ __device__ __forceinline__ int64_t wide_half(const Wide<RIGHT, FULL>& W, const u
   // the loop has one exit: with two, the accumulators are copied and spill
   int64_t s = 0, end = nslab;
   if (__builtin_amdgcn_readfirstlane(bad[0]) && !restage(0, 0)) end = 0;
+  if (__builtin_amdgcn_readfirstlane(bad[2])) end = 0;
 #pragma unroll
   for (int q = 0; q < 4; ++q) g0[q] = rdG(0, 0, q);
 #pragma unroll
@@ -1174,6 +1182,7 @@ __device__ __forceinline__ int64_t wide_half(const Wide<RIGHT, FULL>& W, const u
   }
   // the powers of two come off (see store_acc for an accumulator's rows)
   const int* se = sexp + kApW;
+  const int pexp = bad[3];
 #pragma unroll
   for (int q = 0; q < 4; ++q)
 #pragma unroll
@@ -1312,8 +1321,12 @@ __device__ __forceinline__ void proj_wide(const ApDesc& D, const ApL& L, int til
                             ((RIGHT ? C : R) + 31) / 32, pass, gsl, psl};
   f32x16 acc[4][2];
   double nsq;   // squares of channel ch0 + (tid & 255), k half tid >> 8
-  const int pexp = 254 - (int)(__float_as_uint(gp(D.ws)[L.scal + 8]) >> 23);
-  const int64_t s = wide_half(W, reinterpret_cast<const u32x4*>(D.ws + L.phalf), pexp, sexp, bad, acc, nsq);
+  if (tid < 64) {   // read behind wide_half's first barrier
+    const int pe = p_scale_exp(r);
+    const bool fits = half_fits(D.ws, L, pe) && (RIGHT ? C : R) >= kApHalfK;
+    if (tid < 4) bad[tid] = tid < 2 ? 0 : (tid == 2 ? (fits ? 0 : 1) : 254 - pe);
+  }
+  const int64_t s = wide_half(W, reinterpret_cast<const u32x4*>(D.ws + L.phalf), sexp, bad, acc, nsq);
   if (s < W.nslab) wide_exact(W, reinterpret_cast<const u32x4*>(D.ws + L.psplit), s, acc, nsq);
   float* glow = D.ws + L.glow;
   const int64_t gx0 = ch0 + gh * 128, ox0 = (int64_t)pass * kApW + oq * 64;
@@ -1736,7 +1749,7 @@ __global__ __launch_bounds__(512) void k_ap_proj_w(ApDesc one, const ApDesc* tab
   __shared__ u32x4 psl[2 * 3 * kApWPu];
   __shared__ double sred[8 + kApW];
   __shared__ int sexp[2 * kApW];
-  __shared__ int bad[2];
+  __shared__ int bad[4];
   const int x = (int)blockIdx.x % 8;
   const int wg = xs.start[x] + (int)blockIdx.x / 8;
   if (wg >= xs.start[x + 1]) return;
@@ -1744,7 +1757,6 @@ __global__ __launch_bounds__(512) void k_ap_proj_w(ApDesc one, const ApDesc* tab
   const ApDesc D = ap_pick(one, tab, ntab, 5, wg, local);
   const ApL L = ap_layout(D.R, D.C, D.r, D.trows);
   const int64_t ch0 = (local % L.ntr) * kApW;
-  if (threadIdx.x < 2) bad[threadIdx.x] = 0;
   auto tile = [&](auto right, auto full) {
     constexpr bool R = decltype(right)::value, F = decltype(full)::value;
     proj_wide<R, F>(D, L, local, gsl, psl, sexp, sred, bad);
@@ -2586,23 +2598,15 @@ static int apollo_run(int phase, int dtype, int stochastic, const a8_apollo_tens
       hipLaunchKernelGGL(k_ap_pgen, dim3((unsigned)(n * kPGen)), dim3(256), 0, st, one, dtab, n);
       if ((rc = check_launch("k_ap_pgen"))) return rc;
     }
-    int nfresh = 0, nhalf = 0;
-    for (int i = 0; i < n && !dsc; ++i) {
-      nfresh += ts[i].proj_fresh ? 1 : 0;
-      nhalf += ts[i].rank % kApWide == 0 ? 1 : 0;
-    }
+    int nfresh = 0;
+    for (int i = 0; i < n && !dsc; ++i) nfresh += ts[i].proj_fresh ? 1 : 0;
     const bool all = nfresh == n && dtab;   // as on every refresh of the matrices of one schedule: one launch
     for (int i = 0; i < (all ? 1 : (nfresh ? n : 0)); ++i) {
       if (!ts[i].proj_fresh) continue;
       const ApDesc& D = tab[(size_t)i];
       const ApL L = ap_layout(D.R, D.C, D.r, D.trows);
-      const int64_t nb = (L.rp * L.Kp / 8 + 255) / 256;
-      const int per = all ? 64 : (int)(nb < 4096 ? nb : 4096);
-      if (all ? nhalf > 0 : D.r % kApWide == 0) {
-        hipLaunchKernelGGL(k_ap_pmax, dim3((unsigned)(all ? n * kPMax : kPMax)), dim3(256), 0, st, D,
-                           all ? dtab : nullptr);
-        if ((rc = check_launch("k_ap_pmax"))) return rc;
-      }
+      const int64_t nb = (L.rp * L.Kp / 8 + 255) / 256, most = D.r % kApWide == 0 ? kPMax : 4096;
+      const int per = all ? kPMax : (int)(nb < most ? nb : most);
       hipLaunchKernelGGL(k_ap_split, dim3((unsigned)(all ? n * per : per)), dim3(256), 0, st, D, all ? dtab : nullptr,
                          per);
       if ((rc = check_launch("k_ap_split"))) return rc;
