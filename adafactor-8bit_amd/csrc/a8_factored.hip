@@ -4,8 +4,8 @@
 //   k_fstats   2-D tiles of up to kTRS rows x 1024 columns: row sums and column
 //              sums of g^2 (and sum p^2 for the relative step size), written as
 //              per-tile partials -- no atomics, so the result is deterministic;
-//   k_fcolsum  (tensors of more than kSplit row strips) the column partials
-//              summed over groups of kSplit strips, in parallel;
+//   k_fcolsum  (tensors of more than 1024 rows) the column partials summed over
+//              groups of strips, in parallel;
 //   k_fblock   one workgroup per AL block of each row/column vector: reduce the
 //              partials in a fixed order, EMA the second moment, refit and
 //              re-encode the block (columns: inv_col in place);
@@ -51,7 +51,7 @@ constexpr int kMkFp32 = 5;   // HyperF::mk of fp32 momentum (codecs are 1-4)
 struct FWs {
   int64_t rowpart;   // double [nchunk][B*R]       row partial sums
   int64_t colpart;   // double [B][nstrip][C]      column partial sums
-  int64_t colsum;    // double [B][nsplit][C]      column sums over groups of kSplit strips
+  int64_t colsum;    // double [B][nsplit][C]      column sums over groups of gss strips of kTRS rows
   int64_t p2;        // double [ntile]             partial sum p^2
   int64_t npart;     // double [max(nunit, nutile)] partial sums u^2 (per unit or per update tile)
   int64_t invr;      // [B*R]              new row V, then inv_row
@@ -63,31 +63,35 @@ struct FWs {
   int64_t nchunk, nstrip, ntile, nunit;
   int64_t nsplit;    // strip groups of the column reduction (1: k_fblock reads colpart)
   int64_t tr;        // rows per statistics tile
+  int64_t fold;      // strips per kTRS rows
+  int64_t nss, gss;  // strips of kTRS rows, and how many of them a k_fcolsum workgroup sums
   int64_t nustrip, nutile;   // update tiles: kTR rows x 1024 columns
 };
 
 // Tile geometry.  The update passes (k_fupdt) run on tiles of kTR = 32 rows x
 // 1024 columns, which stream best for them.  The statistics passes (k_fstats,
-// k_came1) take up to kTRS rows per tile: each tile ends with a write of its row
+// k_came1) take kTRS rows per tile in large groups: each tile ends with a write of its row
 // and column partials, and such writes spread through the read stream cost far
 // more bandwidth than their bytes, so fewer, taller tiles write less often.  The
-// column partials of tall matrices are reduced in parallel by k_fcolsum, kSplit
-// strips per workgroup, before k_fblock.
+// column partials of tall matrices are reduced in parallel by k_fcolsum before k_fblock.
+//
+// The order of every sum over rows (the columns' and sum p^2) is a function of the tensor
+// alone: rows in kTR at a time, those partials in turn over kTRS rows, and these over groups
+// of gss.  A tall tile adds its kTR-row partials itself; short tiles leave them to the
+// reductions.  So a matrix steps to the same bits alone and in any group.
 #ifndef A8_TRS
 #define A8_TRS 256
 #endif
 constexpr int kTRS = A8_TRS;
-constexpr int kSplit = 32;
+static_assert(kTRS % kTR == 0, "a tall tile holds whole short ones");
 
-// Rows of the statistics tiles of a group of `total` elements: the tallest tiles that
-// still make about 2048 of them, eight workgroups for each of the 256 CUs.  256 rows from
-// 512 M elements on; a 44 M-parameter layer had 176 tiles of 256 rows, less than one
-// workgroup per CU, and takes 32 (k_fstats 64 -> 24 us, k_came1 144 -> 52).
-static int64_t group_tile_rows(int64_t total) {
-  int64_t tr = kTR;
-  while (tr < kTRS && tr * kTC * 2048 < total) tr *= 2;
-  return tr;
-}
+// Rows of the statistics tiles of a group of `total` elements.  Tall tiles need about 900 of
+// them, three and a half workgroups for each of the 256 CUs: a 44 M-parameter layer had 176
+// tiles of 256 rows, less than one workgroup per CU (k_fstats 64 -> 24 us in tiles of 32
+// rows, k_came1 144 -> 52).  Steps, tiles of 32 / 256 rows: 141 M bf16 elements CAME 605 /
+// 663 us; 201 M Adafactor bf16 508 / 520, fp32 943 / 941, CAME bf16 821 / 850; 262 M
+// Adafactor bf16 674 / 636, fp32 1222 / 1127, CAME bf16 1013 / 977.
+static int64_t group_tile_rows(int64_t total) { return total > (int64_t)kTRS * kTC * 896 ? kTRS : kTR; }
 
 // A tensor's tile rows in such a group.
 static int64_t fws_tile_rows(int64_t R, int64_t group_rows) {
@@ -104,7 +108,12 @@ __host__ __device__ inline FWs fws_layout(int64_t B, int64_t R, int64_t C, int64
   w.nustrip = (R + kTR - 1) / kTR;
   w.nutile = B * w.nustrip * w.nchunk;
   w.nunit = (B * R * C + kUnit - 1) / kUnit;
-  w.nsplit = (w.nstrip > kSplit) ? (w.nstrip + kSplit - 1) / kSplit : 1;
+  w.fold = tr == kTR ? kTRS / kTR : 1;   // (fewer than kTRS rows make one tile, or are folded)
+  w.nss = (R + kTRS - 1) / kTRS;
+  int lg = 2;
+  while (w.nss > (int64_t)64 << lg) ++lg;
+  w.gss = (int64_t)1 << lg;
+  w.nsplit = (w.nss + w.gss - 1) >> lg;
   w.rowpart = 0;
   w.colpart = w.rowpart + 2 * w.nchunk * B * R;
   w.colsum = w.colpart + 2 * B * w.nstrip * C;
@@ -396,8 +405,8 @@ __device__ __forceinline__ void tile_rows_out(const double* s_row, double* rowpa
 
 // CUT: C cuts one of the wave's windows (C % 4 columns remain of it).  TINY: C < 4.
 template <typename T, bool PSQ, bool CUT, bool TINY>
-__device__ __forceinline__ void fstats_tile(const DescF& D, const TilePos& q, int64_t c0, double* acc,
-                                            double& psq, double* s_row) {
+__device__ __forceinline__ void fstats_tile(const DescF& D, const TilePos& q, int64_t c0, double* tot,
+                                            double* s_psq, double* s_row) {
   const T* G = reinterpret_cast<const T*>(D.grad);
   const T* P = reinterpret_cast<const T*>(D.param);
   const int64_t R = D.R, C = D.C;
@@ -422,7 +431,16 @@ __device__ __forceinline__ void fstats_tile(const DescF& D, const TilePos& q, in
       }
     }
   };
-  double rp[kRB];
+  double rp[kRB], acc[4] = {0.0, 0.0, 0.0, 0.0}, psq = 0.0;
+  auto fold = [&](int64_t r0) {   // the kTR rows before r0
+#pragma unroll
+    for (int e = 0; e < 4; ++e) { tot[256 * e] += acc[e]; acc[e] = 0.0; }
+    if constexpr (PSQ) {
+      psq = grp_sum_d(psq, 64);
+      if (wl == 0) s_psq[4 * ((r0 - q.r_lo - 1) / kTR)] = psq;
+      psq = 0.0;
+    }
+  };
   auto consume = [&]() {
 #pragma unroll
     for (int k = 0; k < kRB; ++k) {
@@ -462,10 +480,12 @@ __device__ __forceinline__ void fstats_tile(const DescF& D, const TilePos& q, in
     issue(r0);
     __builtin_amdgcn_sched_barrier(0);
     reduce(r0 - kRB);
+    if ((r0 - q.r_lo) % kTR == 0) fold(r0);
     __builtin_amdgcn_sched_barrier(0);
     consume();
   }
   reduce(r0 - kRB);
+  fold(r0);
 }
 
 // Row sums and column sums of g^2 (and sum p^2) as per-tile partials, accumulated
@@ -473,7 +493,7 @@ __device__ __forceinline__ void fstats_tile(const DescF& D, const TilePos& q, in
 template <typename T, bool PSQ>
 __global__ __launch_bounds__(256) void k_fstats(const DescF* __restrict__ table, int ntab) {
   __shared__ double s_row[4 * kTRS];
-  __shared__ double s4[4];
+  __shared__ double s_psq[4 * (kTRS / kTR)];   // [kTR rows][wave]
   const DescF D = *find_tile(table, ntab, (int64_t)blockIdx.x);
   const FWs W = fws_layout(D.B, D.R, D.C, D.tr);
   const TilePos q = tile_pos<false>(D, W);
@@ -481,24 +501,29 @@ __global__ __launch_bounds__(256) void k_fstats(const DescF* __restrict__ table,
   const int wave = __builtin_amdgcn_readfirstlane(lane >> 6);
   const int64_t C = D.C;
   const int64_t cw = q.c_base + 256 * wave, c0 = cw + 4 * wl;   // the wave's first column, the lane's
-  double acc[4] = {0.0, 0.0, 0.0, 0.0};
-  double psq = 0.0;
+  __shared__ double s_tot[4 * 256];   // a lane's column sums (in registers: one wave a SIMD fewer)
+  double* tot = s_tot + lane;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) tot[256 * e] = 0.0;
   double* srow = s_row + kTRS * wave;
   if (cw >= C) {   // the wave's columns lie beyond C
     for (int i = wl; i < kTRS; i += 64) srow[i] = 0.0;
+    if (PSQ && wl < kTRS / kTR) s_psq[4 * wl + wave] = 0.0;
   }
-  else if (C < 4) fstats_tile<T, PSQ, false, true>(D, q, c0, acc, psq, srow);
-  else if ((C & 3) == 0 || cw + 256 <= C) fstats_tile<T, PSQ, false, false>(D, q, c0, acc, psq, srow);
-  else fstats_tile<T, PSQ, true, false>(D, q, c0, acc, psq, srow);
+  else if (C < 4) fstats_tile<T, PSQ, false, true>(D, q, c0, tot, s_psq + wave, srow);
+  else if ((C & 3) == 0 || cw + 256 <= C) fstats_tile<T, PSQ, false, false>(D, q, c0, tot, s_psq + wave, srow);
+  else fstats_tile<T, PSQ, true, false>(D, q, c0, tot, s_psq + wave, srow);
   float* ws = D.ws;
   double* colp = ws_dp(ws, W.colpart) + (q.b * W.nstrip + q.s) * C;
 #pragma unroll
   for (int e = 0; e < 4; ++e)
-    if (c0 + e < C) gp(colp)[c0 + e] = acc[e];
-  tile_rows_out(s_row, ws_dp(ws, W.rowpart) + q.ch * (D.B * D.R) + q.b * D.R, q.r_lo, q.r_hi);
-  if constexpr (PSQ) {
-    const double tot = wg_sum_d(psq, s4);
-    if (lane == 0) gp(ws_dp(ws, W.p2))[q.t] = tot;
+    if (c0 + e < C) gp(colp)[c0 + e] = tot[256 * e];
+  tile_rows_out(s_row, ws_dp(ws, W.rowpart) + q.ch * (D.B * D.R) + q.b * D.R, q.r_lo, q.r_hi);   // (a barrier first)
+  if (PSQ && lane == 0) {
+    double p = 0.0;
+    for (int k = 0; k < (q.r_hi - q.r_lo + kTR - 1) / kTR; ++k)
+      p += ((s_psq[4 * k] + s_psq[4 * k + 1]) + s_psq[4 * k + 2]) + s_psq[4 * k + 3];
+    gp(ws_dp(ws, W.p2))[q.t] = p;
   }
 }
 
@@ -537,7 +562,7 @@ __device__ __forceinline__ void m_old4(int mkr, const uint8_t* mq, const float* 
 // two M blocks.  TINY: C < 4.
 template <typename T, int MK, bool RAGGED, bool TINY>
 __device__ __forceinline__ void came1_tile(const DescF& D, const FWs& W, const TilePos& q, const HyperF& h,
-                                           int64_t c0, const float* icol, float clip, double* acc,
+                                           int64_t c0, const float* icol, float clip, double* tot,
                                            double* s_row) {
   const T* G = reinterpret_cast<const T*>(D.grad);
   const int64_t R = D.R, C = D.C;
@@ -598,7 +623,11 @@ __device__ __forceinline__ void came1_tile(const DescF& D, const FWs& W, const T
       }
     }
   };
-  double rp[kRB];
+  double rp[kRB], acc[4] = {0.0, 0.0, 0.0, 0.0};
+  auto fold = [&](int64_t) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) { tot[256 * e] += acc[e]; acc[e] = 0.0; }
+  };
   auto consume = [&]() {
     float mk4[kRB][4];
 #pragma unroll
@@ -660,10 +689,12 @@ __device__ __forceinline__ void came1_tile(const DescF& D, const FWs& W, const T
     issue(r0);
     __builtin_amdgcn_sched_barrier(0);
     reduce(r0 - kRB);
+    if ((r0 - q.r_lo) % kTR == 0) fold(r0);
     __builtin_amdgcn_sched_barrier(0);
     consume();
   }
   reduce(r0 - kRB);
+  fold(r0);
 }
 
 // CAME pass 1: the residual's row and column sums as per-tile partials in the
@@ -683,18 +714,21 @@ __global__ __launch_bounds__(256) void k_came1(const DescF* __restrict__ table, 
   float icol[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) icol[e] = (c0 + e < C) ? gp(ws)[W.invc + q.b * C + c0 + e] : 0.0f;
-  double acc[4] = {0.0, 0.0, 0.0, 0.0};
+  __shared__ double s_tot[4 * 256];   // a lane's column sums (in registers: one wave a SIMD fewer)
+  double* tot = s_tot + lane;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) tot[256 * e] = 0.0;
   double* srow = s_row + kTRS * wave;
   if (q.c_base + 256 * wave >= C) {   // the wave's columns lie beyond C
     for (int i = wl; i < kTRS; i += 64) srow[i] = 0.0;
   }
-  else if ((C & 3) == 0) came1_tile<T, MK, false, false>(D, W, q, h, c0, icol, clip, acc, srow);
-  else if (C < 4) came1_tile<T, MK, true, true>(D, W, q, h, c0, icol, clip, acc, srow);
-  else came1_tile<T, MK, true, false>(D, W, q, h, c0, icol, clip, acc, srow);
+  else if ((C & 3) == 0) came1_tile<T, MK, false, false>(D, W, q, h, c0, icol, clip, tot, srow);
+  else if (C < 4) came1_tile<T, MK, true, true>(D, W, q, h, c0, icol, clip, tot, srow);
+  else came1_tile<T, MK, true, false>(D, W, q, h, c0, icol, clip, tot, srow);
   double* colp = ws_dp(ws, W.colpart) + (q.b * W.nstrip + q.s) * C;
 #pragma unroll
   for (int e = 0; e < 4; ++e)
-    if (c0 + e < C) gp(colp)[c0 + e] = acc[e];
+    if (c0 + e < C) gp(colp)[c0 + e] = tot[256 * e];
   tile_rows_out(s_row, ws_dp(ws, W.rowpart) + q.ch * (D.B * D.R) + q.b * D.R, q.r_lo, q.r_hi);
 }
 
@@ -722,10 +756,29 @@ __device__ __forceinline__ const DescF* find_cs(const DescF* tab, int n, int64_t
   return tab + lo;
 }
 
-// First level of the column reduction for tensors of more than kSplit strips:
-// one workgroup per (batch, 256 columns, group of kSplit strips) sums its strips'
-// partials in strip order (double) into colsum.  k_fblock then adds the nsplit
-// group sums in order.
+// Strip partials src[k C], k0 <= k < k1, in order, those of `fold` strips (8 or 1) first added
+// by themselves; eight loads in flight.
+__device__ __forceinline__ double strip_sum(const double* src, int64_t C, int64_t k0, int64_t k1, int64_t fold) {
+  double sum = 0.0;
+  int64_t k = k0;
+  for (; k + 8 <= k1; k += 8) {
+    double t[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) t[u] = gp(src)[(k + u) * C];
+    double s = fold == 1 ? sum : 0.0;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) s += t[u];
+    sum = fold == 1 ? s : sum + s;
+  }
+  double s = fold == 1 ? sum : 0.0;
+  for (; k < k1; ++k) s += gp(src)[k * C];
+  return fold == 1 ? s : sum + s;
+}
+static_assert(kTRS / kTR == 8, "strip_sum");
+
+// First level of the column reduction for tensors of more than gss strips of kTRS rows: one
+// workgroup per (batch, 256 columns, group of gss) sums its strips' partials (double) into
+// colsum.  k_fblock then adds the nsplit group sums in order.
 __global__ __launch_bounds__(256) void k_fcolsum(const DescF* __restrict__ table, int ntab) {
   const DescF D = *find_cs(table, ntab, (int64_t)blockIdx.x);
   const FWs W = fws_layout(D.B, D.R, D.C, D.tr);
@@ -738,20 +791,10 @@ __global__ __launch_bounds__(256) void k_fcolsum(const DescF* __restrict__ table
   const int64_t b = w / (W.nsplit * ncg);
   const int64_t c = cg * 256 + threadIdx.x;
   if (c >= C) return;
-  const int64_t k0 = sg * kSplit;
-  const int64_t k1 = (k0 + kSplit < W.nstrip) ? k0 + kSplit : W.nstrip;
-  const double* src = ws_dp(D.ws, W.colpart) + b * W.nstrip * C + c;
-  double sum = 0.0;
-  int64_t k = k0;
-  for (; k + 8 <= k1; k += 8) {   // eight loads in flight, summed in order
-    double t[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) t[u] = gp(src)[(k + u) * C];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) sum += t[u];
-  }
-  for (; k < k1; ++k) sum += gp(src)[k * C];
-  gp(ws_dp(D.ws, W.colsum))[(b * W.nsplit + sg) * C + c] = sum;
+  const int64_t ks = W.gss * W.fold, k0 = sg * ks;
+  const int64_t k1 = (k0 + ks < W.nstrip) ? k0 + ks : W.nstrip;
+  gp(ws_dp(D.ws, W.colsum))[(b * W.nsplit + sg) * C + c] =
+      strip_sum(ws_dp(D.ws, W.colpart) + b * W.nstrip * C + c, C, k0, k1, W.fold);
 }
 
 __device__ __forceinline__ const DescF* find_fblk(const DescF* tab, int n, int64_t wg) {
@@ -825,19 +868,11 @@ __global__ __launch_bounds__(1024) void k_fblock(const DescF* __restrict__ table
       }
       for (; k < W.nchunk; ++k) sum += gp(rp)[k * n];
     } else {
-      // the column's strip partials, or k_fcolsum's sums of kSplit strips each
+      // the column's strip partials, or k_fcolsum's sums
       const int64_t b = i / C, c = i - b * C;
-      const int64_t np = W.nsplit > 1 ? W.nsplit : W.nstrip;
-      const double* cp0 = ws_dp(ws, W.nsplit > 1 ? W.colsum : W.colpart) + b * np * C + c;
-      int64_t k = 0;
-      for (; k + 8 <= np; k += 8) {   // eight loads in flight, summed in order
-        double t[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) t[u] = gp(cp0)[(k + u) * C];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) sum += t[u];
-      }
-      for (; k < np; ++k) sum += gp(cp0)[k * C];
+      const bool cs = W.nsplit > 1;
+      const int64_t np = cs ? W.nsplit : W.nstrip;
+      sum = strip_sum(ws_dp(ws, cs ? W.colsum : W.colpart) + b * np * C + c, C, 0, np, cs ? 1 : W.fold);
     }
     float mean = (float)sum / cnt;
     if constexpr (!CONF) mean = mean + h.eps1;
@@ -916,7 +951,22 @@ __global__ __launch_bounds__(256) void k_frows(const DescF* __restrict__ table, 
     float alpha = rho;
     if (h.scale_param) {
       double s = 0.0;
-      for (int64_t k = lane; k < W.ntile; k += 256) s += gp(ws_dp(ws, W.p2))[k];
+      // tiles of kTRS rows, or the short ones of the same rows first (index (b, strip, chunk)),
+      // their loads in flight
+      const double* p2 = ws_dp(ws, W.p2);
+      const uint32_t nch = (uint32_t)W.nchunk, nss = (uint32_t)W.nss, fold = (uint32_t)W.fold;
+      for (uint32_t k = lane; k < (uint32_t)B * nss * nch; k += 256) {
+        if (fold == 1) { s += gp(p2)[k]; continue; }
+        const uint32_t bs = k / nch, ch = k - bs * nch, b = bs / nss, s0 = (bs - b * nss) * fold;
+        const int64_t left = W.nstrip - s0, at = (b * W.nstrip + s0) * W.nchunk + ch;
+        double t[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) t[j] = j < left ? gp(p2)[at + j * W.nchunk] : 0.0;
+        double f = 0.0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) f += t[j];
+        s += f;
+      }
       s = wg_sum_d(s, sd);
       const float nrm = sqrtf((float)s);
       const float rms = nrm / (float)sqrt((double)D.numel);
