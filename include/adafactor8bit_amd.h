@@ -364,10 +364,11 @@ int a8_factored_step(int dtype, int stochastic, const a8_tensor2d* tensors, int 
                      int m_bits, int m_mode, uint64_t sr_step, int came, double beta3, float eps_came,
                      int c_bits, const void* step_scalars, void* stream);
 int64_t a8_factored_workspace_floats(int64_t batch, int64_t rows, int64_t cols);
-/* The same for a tensor stepped in a group (one a8_factored_step call) of `total`
- * elements over all its tensors: a group's tiles are as tall as its size allows, so the
- * workspace of a tensor in a large group is smaller.  The function above is enough for a
- * tensor in any group. */
+/* The same for a tensor stepped only in groups (a8_factored_step calls) of `total` or more
+ * elements over all their tensors: large groups take taller tiles, which need less.  A call
+ * with fewer elements in all writes more than this returned for the larger total, and
+ * a8_factored_step is not told how large a workspace is: when the tensors of a call change,
+ * ask again with the new total.  The function above is enough for a tensor in any group. */
 int64_t a8_factored_group_workspace_floats(int64_t batch, int64_t rows, int64_t cols, int64_t total);
 int64_t a8_table_bytes_2d(int ntensors);
 
