@@ -67,7 +67,7 @@ __host__ __device__ inline int64_t ap_tile(bool g16, int64_t R, int64_t C, int64
 
 // Workspace of one matrix (offsets in floats; partial arrays hold doubles).
 struct ApL {
-  int64_t n_low, nchg, K, Kp, rp, ntr, npass, ntile, nunit, nsc, napp;
+  int64_t n_low, nchg, K, Kp, rp, ntr, ngp, npass, ntile, nunit, nsc, napp;
   int64_t glow, u, ngsq, fin, scal, gpart, ppart, spart, psplit, phalf, pmax, total;
 };
 
@@ -83,6 +83,9 @@ __host__ __device__ inline ApL ap_layout(int64_t R, int64_t C, int64_t r, int64_
   w.rp = (r + 31) / 32 * 32;
   const int64_t tile = trows;
   w.ntr = (w.nchg + tile - 1) / tile;
+  // partial sums of ||G||^2 and ||p||^2: one per tile, or per 32 rows where the tile's height
+  // changes with the group, so that their order depends on the matrix alone
+  w.ngp = tile == kApTileS || tile == kApTileR ? (w.nchg + 31) / 32 : w.ntr;
   w.npass = (w.rp + kApPass - 1) / kApPass;
   w.ntile = w.ntr * w.npass;
   w.nunit = (w.n_low + kApUnit - 1) / kApUnit;
@@ -100,9 +103,9 @@ __host__ __device__ inline ApL ap_layout(int64_t R, int64_t C, int64_t r, int64_
   w.phalf = w.psplit + 3 * w.rp * w.Kp / 2;   // rp % 32 == 0 and Kp % 64 == 0: 16-byte aligned
   const bool half = r % kApWide == 0;
   w.pmax = w.phalf + (half ? w.rp * w.Kp : 0);   // P's largest magnitude, in kPMax parts
-  w.gpart = w.pmax + (half ? kPMax : 0);   // double[ntr]  ||G||^2 per tile
-  w.ppart = w.gpart + 2 * w.ntr;           // double[ntr]  ||p||^2 per tile
-  w.spart = w.ppart + 2 * w.ntr;           // double[3 nsc] sum ngsq s^2, sum u^2, sum g_low^2
+  w.gpart = w.pmax + (half ? kPMax : 0);   // double[ngp]  ||G||^2
+  w.ppart = w.gpart + 2 * w.ngp;           // double[ngp]  ||p||^2
+  w.spart = w.ppart + 2 * w.ngp;           // double[3 nsc] sum ngsq s^2, sum u^2, sum g_low^2
   w.total = w.spart + 6 * w.nsc;
   return w;
 }
@@ -701,18 +704,22 @@ __device__ __forceinline__ void proj_right(const ApDesc& D, const ApL& L, int ti
   }
   if (!pass0) return;
   // row norms: the eight lanes of a row (consecutive lanes) combine
-  double t = 0.0;
 #pragma unroll
   for (int q = 0; q < RB; ++q) {
-    double nq = nr[q];
+    double nq = nr[q], t = 0.0;
     nq += __shfl_xor(nq, 1, 64);
     nq += __shfl_xor(nq, 2, 64);
     nq += __shfl_xor(nq, 4, 64);
     const int64_t ga = row0 + lr + 32 * q;
-    if ((lane & 7) == 0 && ga < R) { gp(D.ws + L.ngsq)[ga] = norm_sq(nq); t += nq; }
+    if ((lane & 7) == 0 && ga < R) { gp(D.ws + L.ngsq)[ga] = norm_sq(nq); t = nq; }
+    t = grp_sum_d(t, 64);
+    if (l == 0) sred[4 * q + w] = t;
   }
-  t = ap_wg_sum(t, sred);
-  if (lane == 0) ws_d_set(D.ws, L.gpart, rt, t);
+  __syncthreads();
+  if (lane < RB && row0 + 32 * lane < R) {
+    const double* sq = sred + 4 * lane;
+    ws_d_set(D.ws, L.gpart, rt * RB + lane, ((sq[0] + sq[1]) + sq[2]) + sq[3]);
+  }
 }
 
 // Left side: tile = 64 columns of G x 256 outputs (one pass).  The A operand is
@@ -1684,7 +1691,7 @@ template <int RB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 void k_ap_proj_r(ApDesc one, const ApDesc* tab, int ntab) {
   __shared__ __attribute__((aligned(16))) uint16_t lds[2 * kApTileR * kApGS];
-  __shared__ double sred[8];
+  __shared__ double sred[4 * RB];
   int local;
   const ApDesc D = ap_pick(one, tab, ntab, 0, xcd_order((int)blockIdx.x, (int)gridDim.x), local);
   const ApL L = ap_layout(D.R, D.C, D.r, D.trows);
@@ -1815,14 +1822,14 @@ void k_ap_proj_l32(ApDesc one, const ApDesc* tab, int ntab) {
 }
 
 // ------------------------------------------------------------ ||p||^2 (scale_parameter)
-// ntr workgroups per matrix, each summing a contiguous share of p^2 in double;
+// ngp workgroups per matrix, each summing a contiguous share of p^2 in double;
 // only the total (k_ap_scalars) is used.
 template <typename T>
 __global__ __launch_bounds__(256) void k_ap_psq(ApDesc D) {
   __shared__ double sd[4];
   const ApL L = ap_layout(D.R, D.C, D.r, D.trows);
   const int64_t n = D.R * D.C;
-  const int64_t chunk = (n + L.ntr - 1) / L.ntr;
+  const int64_t chunk = (n + L.ngp - 1) / L.ngp;
   const int64_t b = (int64_t)blockIdx.x * chunk, e = b + chunk < n ? b + chunk : n;
   const T* P = reinterpret_cast<const T*>(D.param);
   double s = 0.0;
@@ -2235,7 +2242,7 @@ __global__ __launch_bounds__(256) void k_ap_scalars(ApDesc one, const ApDesc* ta
   float* ws = D.ws;
   const int lane = threadIdx.x;
   double pg = 0.0, pp = 0.0, s0 = 0.0, s1 = 0.0, s2 = 0.0;
-  for (int64_t k = lane; k < L.ntr; k += 256) { pg += ws_d(ws, L.gpart, k); pp += ws_d(ws, L.ppart, k); }
+  for (int64_t k = lane; k < L.ngp; k += 256) { pg += ws_d(ws, L.gpart, k); pp += ws_d(ws, L.ppart, k); }
   for (int64_t k = lane; k < L.nsc; k += 256) {
     s0 += ws_d(ws, L.spart, 3 * k);
     s1 += ws_d(ws, L.spart, 3 * k + 1);
@@ -2652,7 +2659,7 @@ static int apollo_run(int phase, int dtype, int stochastic, const a8_apollo_tens
     if (h.scale_param) {   // ||p||^2 of the parameter (fp64 parameters refuse scale_parameter above)
       for (int i = 0; i < n; ++i) {
         const ApDesc& D = tab[(size_t)i];
-        const dim3 grid((unsigned)ap_layout(D.R, D.C, D.r, D.trows).ntr);
+        const dim3 grid((unsigned)ap_layout(D.R, D.C, D.r, D.trows).ngp);
         if (dtype == A8_BF16) hipLaunchKernelGGL(k_ap_psq<__hip_bfloat16>, grid, dim3(256), 0, st, D);
         else if (dtype == A8_F16) hipLaunchKernelGGL(k_ap_psq<__half>, grid, dim3(256), 0, st, D);
         else hipLaunchKernelGGL(k_ap_psq<float>, grid, dim3(256), 0, st, D);
