@@ -169,6 +169,7 @@ struct DescF {
   int has_fira_prev;
   int tiled;           // update runs on tiles (k_fupdt; 2: C % 4 != 0), 0: flat units
   int tr;              // rows per statistics tile
+  int elem;            // statistics load element by element (fewer than 4 columns, rows of 4 GB and more)
 };
 
 struct HyperF {
@@ -364,7 +365,7 @@ __device__ __forceinline__ void win_fix(const Win& w, int cut, V* v) {
   for (int k = 0; k < 4; ++k) v[k] = (w.n & 3) ? t[k] : v[k];
 }
 
-// A window of a matrix of fewer than four columns, element by element.
+// A window element by element (DescF::elem).
 template <typename T, typename V>
 __device__ __forceinline__ void load_tiny(const T* row, int64_t c0, int64_t C, V* out) {
 #pragma unroll
@@ -403,7 +404,7 @@ __device__ __forceinline__ void tile_rows_out(const double* s_row, double* rowpa
   }
 }
 
-// CUT: C cuts one of the wave's windows (C % 4 columns remain of it).  TINY: C < 4.
+// CUT: C cuts one of the wave's windows (C % 4 columns remain of it).  TINY: DescF::elem.
 template <typename T, bool PSQ, bool CUT, bool TINY>
 __device__ __forceinline__ void fstats_tile(const DescF& D, const TilePos& q, int64_t c0, double* tot,
                                             double* s_psq, double* s_row) {
@@ -510,7 +511,7 @@ __global__ __launch_bounds__(256) void k_fstats(const DescF* __restrict__ table,
     for (int i = wl; i < kTRS; i += 64) srow[i] = 0.0;
     if (PSQ && wl < kTRS / kTR) s_psq[4 * wl + wave] = 0.0;
   }
-  else if (C < 4) fstats_tile<T, PSQ, false, true>(D, q, c0, tot, s_psq + wave, srow);
+  else if (D.elem) fstats_tile<T, PSQ, false, true>(D, q, c0, tot, s_psq + wave, srow);
   else if ((C & 3) == 0 || cw + 256 <= C) fstats_tile<T, PSQ, false, false>(D, q, c0, tot, s_psq + wave, srow);
   else fstats_tile<T, PSQ, true, false>(D, q, c0, tot, s_psq + wave, srow);
   float* ws = D.ws;
@@ -559,7 +560,7 @@ __device__ __forceinline__ void m_old4(int mkr, const uint8_t* mq, const float* 
 // U = ((g * inv_row) * inv_col) / clip, M' = lerp(M, U, 1 - beta1),
 // res = (U - M')^2 + eps_came, row and column sums of res (optimizer.py:929-937).
 // RAGGED: C is no multiple of 4, so rows start anywhere and a window's codes may straddle
-// two M blocks.  TINY: C < 4.
+// two M blocks.  TINY: DescF::elem.
 template <typename T, int MK, bool RAGGED, bool TINY>
 __device__ __forceinline__ void came1_tile(const DescF& D, const FWs& W, const TilePos& q, const HyperF& h,
                                            int64_t c0, const float* icol, float clip, double* tot,
@@ -722,8 +723,8 @@ __global__ __launch_bounds__(256) void k_came1(const DescF* __restrict__ table, 
   if (q.c_base + 256 * wave >= C) {   // the wave's columns lie beyond C
     for (int i = wl; i < kTRS; i += 64) srow[i] = 0.0;
   }
+  else if (D.elem) came1_tile<T, MK, true, true>(D, W, q, h, c0, icol, clip, tot, srow);
   else if ((C & 3) == 0) came1_tile<T, MK, false, false>(D, W, q, h, c0, icol, clip, tot, srow);
-  else if (C < 4) came1_tile<T, MK, true, true>(D, W, q, h, c0, icol, clip, tot, srow);
   else came1_tile<T, MK, true, false>(D, W, q, h, c0, icol, clip, tot, srow);
   double* colp = ws_dp(ws, W.colpart) + (q.b * W.nstrip + q.s) * C;
 #pragma unroll
@@ -1917,8 +1918,11 @@ int a8_factored_step(int dtype, int stochastic, const a8_tensor2d* tensors, int 
     D.ws = t.workspace; D.lr = t.lr; D.fira_prev = t.fira_prev_norm; D.has_fira_prev = t.has_fira_prev;
     D.B = t.batch; D.R = t.rows; D.C = t.cols; D.numel = numel;
     D.sr_seed = t.sr_seed;
+    // the tiles' loads take 32-bit byte offsets into a row
+    const int64_t esz = dtype == A8_F64 ? 8 : (dtype == A8_F32 || m32 ? 4 : 2);
+    D.elem = t.cols < 4 || t.cols * esz > 0xFFFFFFFFll ? 1 : 0;
     // coded momentum: whole M blocks per row (then C % 4 == 0 too)
-    D.tiled = t.cols >= 4 &&
+    D.tiled = !D.elem &&
               (!has_m || m32 || (lbm >= 0 && m_block_size <= 256 && t.cols % m_block_size == 0)) ?
               (t.cols % 4 ? 2 : 1) : 0;
     (D.tiled == 0 ? any_flat : D.tiled == 1 ? any_tiled : any_cut) = true;
