@@ -220,3 +220,19 @@ def test_values_off_the_fp16_scale_cost_no_second_projection(shape, value):
                 best[name] = min(best.get(name, 1e9), a.elapsed_time(b))
     print(best, flush=True)
     assert best["odd"] <= 1.22 * best["plain"], best
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["zeros", "outliers", "nonfinite", "tiny", "spread"])
+@pytest.mark.parametrize("cols,rank", [(154, 32), (154, 65), (135, 64), (130, 130)])
+def test_narrow_tiles_of_uneven_gradients(cols, rank, kind):
+    """The narrow tiles' exact split, shared by one, two and four waves, on gradients of every kind."""
+    for shape in ((200, cols), (cols, 200)):
+        print(f"[apollo narrow] {shape} r={rank} {kind}", flush=True)
+        right, G, pt, low, nsq = _low(shape, rank, _gradient(shape, kind, 23))
+        a, b = (G, pt) if right else (pt, G)
+        err = np.abs(low - a @ b)
+        assert np.all(err <= 3 * (cols + 2) * U * (np.abs(a) @ np.abs(b)) + 1e-44)
+        if kind != "tiny":
+            exact = (G * G).sum(axis=1 if right else 0)
+            assert np.all(np.abs(nsq - exact) <= 19 * U * exact)

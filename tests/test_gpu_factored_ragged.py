@@ -88,3 +88,37 @@ def test_ragged_columns_stochastic_rounding(case):
         want = np.asarray(want).astype(np.int64) & 0xFFFF
         assert (got != want).sum() <= 1 + 0.01 * got.size, (case, SHAPES[i])
         assert np.abs(got - want).max() <= 1, (case, SHAPES[i])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", ["plain", "fp32_m", "uf8"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float64])
+def test_ragged_columns_of_every_type(case, dtype):
+    """fp16, bf16 (rounded to nearest) and fp64 parameters, gradients with infinities and NaN: the
+    step of the fp32 twin (same values, non-finite gradients zero).  fp16 and bf16: to half a unit
+    of the type and fp32's 1e-5 of the update, rounded once; fp64: its gradient is that of the
+    twin exactly, its arithmetic fp32 but for the last addition."""
+    from adafactor8bit import Adafactor8Bit
+    kw = dict(CASES[case], scale_parameter=False)
+    eps = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float64: 2.0 ** -24}[dtype]
+    pa = [torch.nn.Parameter(make_param(s, i, 19).to(torch.bfloat16).to(dtype).cuda()) for i, s in enumerate(SHAPES)]
+    pb = [torch.nn.Parameter(p.detach().float()) for p in pa]
+    start = [p.detach().clone() for p in pb]
+    oa, ob = Adafactor8Bit(pa, **kw), Adafactor8Bit(pb, **kw)
+    for i, (a, b) in enumerate(zip(pa, pb)):
+        g = (_grad(SHAPES[i], i, 1) * 16.0).to(torch.bfloat16).float().cuda()
+        f = g.view(-1)
+        f[3::11], f[4::13], f[1::17] = float("inf"), float("nan"), -float("inf")
+        a.grad = g.to(dtype)
+        b.grad = torch.nan_to_num(g, nan=0.0, posinf=0.0, neginf=0.0)
+    oa.step()
+    ob.step()
+    torch.cuda.synchronize()
+    for i, (a, b) in enumerate(zip(pa, pb)):
+        x, y = a.detach().double(), b.detach().double()
+        assert torch.isfinite(x).all()
+        tol = eps * y.abs() + 1e-5 * (y - start[i].double()).abs() + (6e-8 if dtype == torch.float16 else 0.0)
+        assert torch.all((x - y).abs() <= tol), (case, dtype, SHAPES[i], float(((x - y).abs() - tol).max()))
+        for k, v in ob.state[b].items():
+            if torch.is_tensor(v) and v.dtype == torch.uint8:
+                assert torch.equal(v, oa.state[a][k]), (case, dtype, SHAPES[i], k)
