@@ -638,9 +638,11 @@ __device__ __forceinline__ void unit_step(const Desc1D& D, const Hyper1D& h, int
 
 // Occupancy 7 waves per SIMD (at most 72 VGPRs): measured best on MI355X for
 // this streaming step (more resident waves hide the HBM latency of the loads).  The
-// forms that VALU issue bounds (stochastic rounding, element-wise decoding) take 6.
+// forms that VALU issue bounds (stochastic rounding, element-wise decoding) take 6, and so
+// do the momentum codecs chosen at run time, which spill at 72 registers (67 M fp32
+// parameters, B_V 2048: UF4 220 -> 183 us, with a clip 312 -> 283, D8 717 -> 664).
 template <typename T, int VB, int MODE, bool SR, int MK, int KR>
-__global__ __launch_bounds__(kLanes) __attribute__((amdgpu_waves_per_eu((SR || VB != 8) ? 6 : 7)))
+__global__ __launch_bounds__(kLanes) __attribute__((amdgpu_waves_per_eu((SR || VB != 8 || MK == 2) ? 6 : 7)))
 void k_update1d(Desc1D one, const Desc1D* __restrict__ table, int ntab, Hyper1D h) {
   extern __shared__ float s_lds[];  // [nv_wg * 256] AL8 tables | cross-wave partials and fits
   if (h.dsc) {
@@ -677,9 +679,14 @@ void k_update1d(Desc1D one, const Desc1D* __restrict__ table, int ntab, Hyper1D 
 constexpr int kGenMaxMB = 2048;           // M blocks whose absmax LDS holds at once
 constexpr int kGenMaxBV = 1 << 30;        // block_size is a 32-bit int
 
+// Waves per SIMD are stated where one register more than the bound costs one (65 and 81): 67 M
+// fp32 parameters, B_V 384, 939 -> 849 us with momentum, 519 -> 501 without; B_V 4096 378 ->
+// 357.  SUM and APPLYC without momentum are left alone, and their tables take the short power
+// (a clipped step 776 us, 817 with the library's); the other modes the library's (501 us
+// without momentum, 585 with the short one; B_V 131072, UF4 874 and 901).
 template <typename T, int VB, int MODE, bool SR, int MK, int KR>
-__global__ __launch_bounds__(kLanes) void k_update1d_gen(Desc1D one, const Desc1D* __restrict__ table, int ntab,
-                                                         Hyper1D h) {
+__global__ __launch_bounds__(kLanes) __attribute__((amdgpu_waves_per_eu(MK != 0 ? 6 : (MODE == 5 || MODE == 6 ? 1 : 8))))
+void k_update1d_gen(Desc1D one, const Desc1D* __restrict__ table, int ntab, Hyper1D h) {
   constexpr bool kHasM = MK != 0;
   constexpr bool kVbuf = MODE == 2 || MODE == 4;
   constexpr bool kSq = MODE == 1 || MODE == 3 || MODE == 4 || MODE == 5 || MODE == 7;
@@ -715,7 +722,11 @@ __global__ __launch_bounds__(kLanes) void k_update1d_gen(Desc1D one, const Desc1
   const float s_old = kVbuf ? 0.0f : gp(D.v_scale)[blk], lm_old = kVbuf ? 0.0f : gp(D.v_min_log)[blk];
   if (lane == 0) { s_st[0] = 0u; s_st[1] = 0xFFFFFFFFu; }
   for (int i = lane; i < (mpb < kGenMaxMB ? mpb : kGenMaxMB); i += kLanes) s_mab[i] = 0u;
-  if (VB == 8 && !kVbuf) s_tab[lane] = al_decode<254>((uint32_t)lane, s_old, lm_old, KR);
+  if constexpr (VB == 8 && !kVbuf) {
+    // one power a lane, the library's where the kernel is bound by registers, not by issue
+    if (MODE >= 5) s_tab[lane] = al_decode<254>((uint32_t)lane, s_old, lm_old, KR);
+    else s_tab[lane] = lane ? exp2_lib(al_dec_log<254>((float)(lane - 1), s_old, lm_old, KR)) : 0.0f;
+  }
   __syncthreads();
 
   // step scale (unit_step's)
