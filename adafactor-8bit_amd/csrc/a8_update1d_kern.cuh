@@ -641,8 +641,9 @@ __device__ __forceinline__ void unit_step(const Desc1D& D, const Hyper1D& h, int
 // forms that VALU issue bounds (stochastic rounding, element-wise decoding) take 6, and so
 // do the momentum codecs chosen at run time, which spill at 72 registers (67 M fp32
 // parameters, B_V 2048: UF4 220 -> 183 us, with a clip 312 -> 283, D8 717 -> 664).
+// 64-bit parameters take 5: 30 M of them, 300 us at 7 (18 registers spilled), 218 at 5.
 template <typename T, int VB, int MODE, bool SR, int MK, int KR>
-__global__ __launch_bounds__(kLanes) __attribute__((amdgpu_waves_per_eu((SR || VB != 8 || MK == 2) ? 6 : 7)))
+__global__ __launch_bounds__(kLanes) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 5 : (SR || VB != 8 || MK == 2) ? 6 : 7)))
 void k_update1d(Desc1D one, const Desc1D* __restrict__ table, int ntab, Hyper1D h) {
   extern __shared__ float s_lds[];  // [nv_wg * 256] AL8 tables | cross-wave partials and fits
   if (h.dsc) {
