@@ -91,12 +91,10 @@ static_assert(kTRS % kTR == 0, "a tall tile holds whole short ones");
 // rows, k_came1 144 -> 52).  Steps, tiles of 32 / 256 rows: 141 M bf16 elements CAME 605 /
 // 663 us; 201 M Adafactor bf16 508 / 520, fp32 943 / 941, CAME bf16 821 / 850; 262 M
 // Adafactor bf16 674 / 636, fp32 1222 / 1127, CAME bf16 1013 / 977.
-static int64_t group_tile_rows(int64_t total) { return total > (int64_t)kTRS * kTC * 896 ? kTRS : kTR; }
-
-// A tensor's tile rows in such a group.
-static int64_t fws_tile_rows(int64_t R, int64_t group_rows) {
+static int64_t fws_tile_rows(int64_t R, int64_t total) {
+  const int64_t rows = total > (int64_t)kTRS * kTC * 896 ? kTRS : kTR;
   const int64_t r = (R + kTR - 1) / kTR * kTR;
-  return r < group_rows ? r : group_rows;
+  return r < rows ? r : rows;
 }
 
 __host__ __device__ inline FWs fws_layout(int64_t B, int64_t R, int64_t C, int64_t tr) {
@@ -119,7 +117,7 @@ __host__ __device__ inline FWs fws_layout(int64_t B, int64_t R, int64_t C, int64
   w.colsum = w.colpart + 2 * B * w.nstrip * C;
   w.p2 = w.colsum + (w.nsplit > 1 ? 2 * B * w.nsplit * C : 0);
   w.npart = w.p2 + 2 * w.ntile;
-  w.invr = w.npart + 2 * (w.nunit > w.nutile ? w.nunit : w.nutile);
+  w.invr = (w.npart + 2 * (w.nunit > w.nutile ? w.nunit : w.nutile) + 31) / 32 * 32;   // whole lines
   w.invc = w.invr + B * R;
   w.icr = w.invc + B * C;
   w.icc = w.icr + B * R;
@@ -365,11 +363,13 @@ __device__ __forceinline__ void win_fix(const Win& w, int cut, V* v) {
   for (int k = 0; k < 4; ++k) v[k] = (w.n & 3) ? t[k] : v[k];
 }
 
-// A window element by element (DescF::elem).
+// A window element by element (DescF::elem); every load is issued, inside the row.
 template <typename T, typename V>
 __device__ __forceinline__ void load_tiny(const T* row, int64_t c0, int64_t C, V* out) {
 #pragma unroll
-  for (int k = 0; k < 4; ++k) out[k] = (c0 + k < C) ? ld1<T, V>(row, c0 + k) : (V)0;
+  for (int k = 0; k < 4; ++k) out[k] = ld1<T, V>(row, c0 + k < C ? c0 + k : C - 1);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) out[k] = c0 + k < C ? out[k] : (V)0;
 }
 
 // Where a statistics workgroup sits: tensor-local tile t, chunk, strip, batch.
@@ -404,9 +404,22 @@ __device__ __forceinline__ void tile_rows_out(const double* s_row, double* rowpa
   }
 }
 
+// A lane's column sums of kTR rows (acc) to its sums of the tile so far in LDS (tot; in
+// registers they cost a wave per SIMD).  The tile's last kTR rows stay in acc.
+__device__ __forceinline__ void col_fold(double* acc, double* tot) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    tot[256 * e] += acc[e];
+    acc[e] = 0.0;
+  }
+}
+__device__ __forceinline__ double col_sum(const double* acc, const double* tot, int e, const TilePos& q) {
+  return q.r_hi - q.r_lo > kTR ? tot[256 * e] + acc[e] : acc[e];
+}
+
 // CUT: C cuts one of the wave's windows (C % 4 columns remain of it).  TINY: DescF::elem.
 template <typename T, bool PSQ, bool CUT, bool TINY>
-__device__ __forceinline__ void fstats_tile(const DescF& D, const TilePos& q, int64_t c0, double* tot,
+__device__ __forceinline__ void fstats_tile(const DescF& D, const TilePos& q, int64_t c0, double* acc, double* tot,
                                             double* s_psq, double* s_row) {
   const T* G = reinterpret_cast<const T*>(D.grad);
   const T* P = reinterpret_cast<const T*>(D.param);
@@ -432,10 +445,8 @@ __device__ __forceinline__ void fstats_tile(const DescF& D, const TilePos& q, in
       }
     }
   };
-  double rp[kRB], acc[4] = {0.0, 0.0, 0.0, 0.0}, psq = 0.0;
-  auto fold = [&](int64_t r0) {   // the kTR rows before r0
-#pragma unroll
-    for (int e = 0; e < 4; ++e) { tot[256 * e] += acc[e]; acc[e] = 0.0; }
+  double rp[kRB], psq = 0.0;
+  auto fold_psq = [&](int64_t r0) {   // of the kTR rows before r0
     if constexpr (PSQ) {
       psq = grp_sum_d(psq, 64);
       if (wl == 0) s_psq[4 * ((r0 - q.r_lo - 1) / kTR)] = psq;
@@ -481,18 +492,22 @@ __device__ __forceinline__ void fstats_tile(const DescF& D, const TilePos& q, in
     issue(r0);
     __builtin_amdgcn_sched_barrier(0);
     reduce(r0 - kRB);
-    if ((r0 - q.r_lo) % kTR == 0) fold(r0);
+    if ((r0 - q.r_lo) % kTR == 0) {
+      col_fold(acc, tot);
+      fold_psq(r0);
+    }
     __builtin_amdgcn_sched_barrier(0);
     consume();
   }
   reduce(r0 - kRB);
-  fold(r0);
+  fold_psq(r0);
 }
 
 // Row sums and column sums of g^2 (and sum p^2) as per-tile partials, accumulated
 // in double (optimizer.py:2211-2219).
 template <typename T, bool PSQ>
-__global__ __launch_bounds__(256) void k_fstats(const DescF* __restrict__ table, int ntab) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? (PSQ ? 4 : 6) : (PSQ ? 5 : 7))))
+void k_fstats(const DescF* __restrict__ table, int ntab) {
   __shared__ double s_row[4 * kTRS];
   __shared__ double s_psq[4 * (kTRS / kTR)];   // [kTR rows][wave]
   const DescF D = *find_tile(table, ntab, (int64_t)blockIdx.x);
@@ -502,23 +517,26 @@ __global__ __launch_bounds__(256) void k_fstats(const DescF* __restrict__ table,
   const int wave = __builtin_amdgcn_readfirstlane(lane >> 6);
   const int64_t C = D.C;
   const int64_t cw = q.c_base + 256 * wave, c0 = cw + 4 * wl;   // the wave's first column, the lane's
-  __shared__ double s_tot[4 * 256];   // a lane's column sums (in registers: one wave a SIMD fewer)
+  __shared__ double s_tot[4 * 256];
   double* tot = s_tot + lane;
+  double acc[4] = {0.0, 0.0, 0.0, 0.0};
+  if (q.r_hi - q.r_lo > kTR) {
 #pragma unroll
-  for (int e = 0; e < 4; ++e) tot[256 * e] = 0.0;
+    for (int e = 0; e < 4; ++e) tot[256 * e] = 0.0;
+  }
   double* srow = s_row + kTRS * wave;
   if (cw >= C) {   // the wave's columns lie beyond C
     for (int i = wl; i < kTRS; i += 64) srow[i] = 0.0;
     if (PSQ && wl < kTRS / kTR) s_psq[4 * wl + wave] = 0.0;
   }
-  else if (D.elem) fstats_tile<T, PSQ, false, true>(D, q, c0, tot, s_psq + wave, srow);
-  else if ((C & 3) == 0 || cw + 256 <= C) fstats_tile<T, PSQ, false, false>(D, q, c0, tot, s_psq + wave, srow);
-  else fstats_tile<T, PSQ, true, false>(D, q, c0, tot, s_psq + wave, srow);
+  else if (D.elem) fstats_tile<T, PSQ, false, true>(D, q, c0, acc, tot, s_psq + wave, srow);
+  else if ((C & 3) == 0 || cw + 256 <= C) fstats_tile<T, PSQ, false, false>(D, q, c0, acc, tot, s_psq + wave, srow);
+  else fstats_tile<T, PSQ, true, false>(D, q, c0, acc, tot, s_psq + wave, srow);
   float* ws = D.ws;
   double* colp = ws_dp(ws, W.colpart) + (q.b * W.nstrip + q.s) * C;
 #pragma unroll
   for (int e = 0; e < 4; ++e)
-    if (c0 + e < C) gp(colp)[c0 + e] = tot[256 * e];
+    if (c0 + e < C) gp(colp)[c0 + e] = col_sum(acc, tot, e, q);
   tile_rows_out(s_row, ws_dp(ws, W.rowpart) + q.ch * (D.B * D.R) + q.b * D.R, q.r_lo, q.r_hi);   // (a barrier first)
   if (PSQ && lane == 0) {
     double p = 0.0;
@@ -563,7 +581,7 @@ __device__ __forceinline__ void m_old4(int mkr, const uint8_t* mq, const float* 
 // two M blocks.  TINY: DescF::elem.
 template <typename T, int MK, bool RAGGED, bool TINY>
 __device__ __forceinline__ void came1_tile(const DescF& D, const FWs& W, const TilePos& q, const HyperF& h,
-                                           int64_t c0, const float* icol, float clip, double* tot,
+                                           int64_t c0, const float* icol, float clip, double* acc, double* tot,
                                            double* s_row) {
   const T* G = reinterpret_cast<const T*>(D.grad);
   const int64_t R = D.R, C = D.C;
@@ -624,11 +642,7 @@ __device__ __forceinline__ void came1_tile(const DescF& D, const FWs& W, const T
       }
     }
   };
-  double rp[kRB], acc[4] = {0.0, 0.0, 0.0, 0.0};
-  auto fold = [&](int64_t) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) { tot[256 * e] += acc[e]; acc[e] = 0.0; }
-  };
+  double rp[kRB];
   auto consume = [&]() {
     float mk4[kRB][4];
 #pragma unroll
@@ -690,12 +704,11 @@ __device__ __forceinline__ void came1_tile(const DescF& D, const FWs& W, const T
     issue(r0);
     __builtin_amdgcn_sched_barrier(0);
     reduce(r0 - kRB);
-    if ((r0 - q.r_lo) % kTR == 0) fold(r0);
+    if ((r0 - q.r_lo) % kTR == 0) col_fold(acc, tot);
     __builtin_amdgcn_sched_barrier(0);
     consume();
   }
   reduce(r0 - kRB);
-  fold(r0);
 }
 
 // CAME pass 1: the residual's row and column sums as per-tile partials in the
@@ -715,21 +728,24 @@ __global__ __launch_bounds__(256) void k_came1(const DescF* __restrict__ table, 
   float icol[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) icol[e] = (c0 + e < C) ? gp(ws)[W.invc + q.b * C + c0 + e] : 0.0f;
-  __shared__ double s_tot[4 * 256];   // a lane's column sums (in registers: one wave a SIMD fewer)
+  __shared__ double s_tot[4 * 256];
   double* tot = s_tot + lane;
+  double acc[4] = {0.0, 0.0, 0.0, 0.0};
+  if (q.r_hi - q.r_lo > kTR) {
 #pragma unroll
-  for (int e = 0; e < 4; ++e) tot[256 * e] = 0.0;
+    for (int e = 0; e < 4; ++e) tot[256 * e] = 0.0;
+  }
   double* srow = s_row + kTRS * wave;
   if (q.c_base + 256 * wave >= C) {   // the wave's columns lie beyond C
     for (int i = wl; i < kTRS; i += 64) srow[i] = 0.0;
   }
-  else if (D.elem) came1_tile<T, MK, true, true>(D, W, q, h, c0, icol, clip, tot, srow);
-  else if ((C & 3) == 0) came1_tile<T, MK, false, false>(D, W, q, h, c0, icol, clip, tot, srow);
-  else came1_tile<T, MK, true, false>(D, W, q, h, c0, icol, clip, tot, srow);
+  else if (D.elem) came1_tile<T, MK, true, true>(D, W, q, h, c0, icol, clip, acc, tot, srow);
+  else if ((C & 3) == 0) came1_tile<T, MK, false, false>(D, W, q, h, c0, icol, clip, acc, tot, srow);
+  else came1_tile<T, MK, true, false>(D, W, q, h, c0, icol, clip, acc, tot, srow);
   double* colp = ws_dp(ws, W.colpart) + (q.b * W.nstrip + q.s) * C;
 #pragma unroll
   for (int e = 0; e < 4; ++e)
-    if (c0 + e < C) gp(colp)[c0 + e] = tot[256 * e];
+    if (c0 + e < C) gp(colp)[c0 + e] = col_sum(acc, tot, e, q);
   tile_rows_out(s_row, ws_dp(ws, W.rowpart) + q.ch * (D.B * D.R) + q.b * D.R, q.r_lo, q.r_hi);
 }
 
@@ -956,8 +972,8 @@ __global__ __launch_bounds__(256) void k_frows(const DescF* __restrict__ table, 
       // their loads in flight
       const double* p2 = ws_dp(ws, W.p2);
       const uint32_t nch = (uint32_t)W.nchunk, nss = (uint32_t)W.nss, fold = (uint32_t)W.fold;
-      for (uint32_t k = lane; k < (uint32_t)B * nss * nch; k += 256) {
-        if (fold == 1) { s += gp(p2)[k]; continue; }
+      for (uint32_t k = lane; fold == 1 && k < (uint32_t)B * nss * nch; k += 256) s += gp(p2)[k];
+      for (uint32_t k = lane; fold != 1 && k < (uint32_t)B * nss * nch; k += 256) {
         const uint32_t bs = k / nch, ch = k - bs * nch, b = bs / nss, s0 = (bs - b * nss) * fold;
         const int64_t left = W.nstrip - s0, at = (b * W.nstrip + s0) * W.nchunk + ch;
         double t[8];
@@ -1845,7 +1861,7 @@ int64_t a8_factored_workspace_floats(int64_t batch, int64_t rows, int64_t cols) 
 
 int64_t a8_factored_group_workspace_floats(int64_t batch, int64_t rows, int64_t cols, int64_t total) {
   if (batch <= 0 || rows <= 0 || cols <= 0) return 0;
-  return fws_layout(batch, rows, cols, fws_tile_rows(rows, group_tile_rows(total))).total;
+  return fws_layout(batch, rows, cols, fws_tile_rows(rows, total)).total;
 }
 
 int64_t a8_table_bytes_2d(int ntensors) { return (int64_t)sizeof(DescF) * (int64_t)ntensors; }
@@ -1889,7 +1905,6 @@ int a8_factored_step(int dtype, int stochastic, const a8_tensor2d* tensors, int 
   bool any_tiled = false, any_cut = false, any_flat = false;
   int64_t total = 0;
   for (int i = 0; i < ntensors; ++i) total += tensors[i].batch * tensors[i].rows * tensors[i].cols;
-  const int64_t group_rows = group_tile_rows(total);
   for (int i = 0; i < ntensors; ++i) {
     const a8_tensor2d& t = tensors[i];
     if (t.batch <= 0 || t.rows <= 0 || t.cols <= 0) return set_error(A8_ERR_SIZE, "empty factored tensor");
@@ -1926,7 +1941,7 @@ int a8_factored_step(int dtype, int stochastic, const a8_tensor2d* tensors, int 
               (!has_m || m32 || (lbm >= 0 && m_block_size <= 256 && t.cols % m_block_size == 0)) ?
               (t.cols % 4 ? 2 : 1) : 0;
     (D.tiled == 0 ? any_flat : D.tiled == 1 ? any_tiled : any_cut) = true;
-    D.tr = (int)fws_tile_rows(t.rows, group_rows);
+    D.tr = (int)fws_tile_rows(t.rows, total);
     const FWs W = fws_layout(t.batch, t.rows, t.cols, D.tr);
     D.tile_begin = tiles;
     D.utile_begin = utiles;
