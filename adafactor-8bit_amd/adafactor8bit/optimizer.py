@@ -213,7 +213,7 @@ class Adafactor8Bit(Optimizer):
         super().__init__(params, defaults)
         self._apollo_seed_counter = 1
         self._sr_seed_counter = 1
-        self._ws = {}   # device workspaces (tensor tables, norm buffers, v_buf)
+        self._ws = {}   # device workspaces (tensor tables, norm buffers, APOLLO and factored workspaces)
 
     def add_param_group(self, param_group):
         """``Optimizer.add_param_group`` plus a check that every parameter's route

@@ -16,13 +16,16 @@
 // One step of a group of matrices is five launches over a device table of
 // per-matrix descriptors (each kernel finds its matrix by a binary search of a
 // compact first-workgroup array):
-//   k_ap_proj    bf16 G: MFMA projection (v_mfma_f32_32x32x16_bf16) of 64-row
-//                (right) or 64-column (left) tiles of G against P^T split into
-//                three bf16 terms (3 x 8 significand bits carry fp32's 24; all
-//                products land in one fp32 accumulator), reading G once: the
-//                same pass scrubs non-finite entries and accumulates the channel
-//                norms of G.  fp32 G: the same tiles with G split into three
-//                bf16 terms as well (six products per pair of terms).
+//   k_ap_proj    MFMA projection, reading G once: the same pass takes non-finite
+//                entries as zero and accumulates the channel norms of G.  bf16 G
+//                at ranks that are a multiple of 256 (k_ap_proj_w): tiles of 256
+//                channels x 256 outputs with G and two terms of P^T as scaled
+//                fp16, or G in bf16 and three bf16 terms of P^T where those do not
+//                fit.  Other ranks (k_ap_proj_r, k_ap_proj_l): tiles of 96 or 32
+//                rows (right) or 64 columns (left) against the three bf16 terms
+//                (3 x 8 significand bits carry fp32's 24).  fp32 G (k_ap_proj_r32,
+//                k_ap_proj_l32): 64-channel tiles with G split into three bf16
+//                terms as well (six products per pair of terms).
 //   k_ap_low     low-rank V/M EMA and re-encode, u
 //   k_ap_scale   channel (or tensor) norms of u and g_low, per-workgroup partials
 //   k_ap_scalars one workgroup per matrix: alpha, Fira, step, decay
@@ -45,7 +48,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kApTile = 64;     // G columns per left-side projection tile (and fp32 G's right-side tile)
 constexpr int kApRB = 3;        // 32-row blocks per right-side bf16 projection tile
 constexpr int kApTileR = 32 * kApRB;   // G rows per right-side bf16 projection tile
-constexpr int kApTileS = 32;           // the same in a group with few of them (ap_few_tiles)
+constexpr int kApTileS = 32;           // the same in a group with few of them (apollo_run)
 constexpr int kApPass = 256;    // low-rank outputs per projection pass (4 waves x 64)
 constexpr int kApUnit = 2048;   // low-rank elements per k_ap_low workgroup (8 per lane)
 constexpr int kApScR = 16;      // right side: g_low rows per k_ap_scale workgroup
@@ -552,9 +555,11 @@ constexpr int kApTS = 40;   // LDS row stride (halves) of the left side's transp
 // one 16-k sub-step of one), and add their accumulators through LDS at the end in a fixed
 // order.  Without the split three of four waves had no MFMAs at rank 64: five uneven
 // matrices, k_ap_proj_l 80 -> 41 us, k_ap_proj_r (with lower tiles) 153 -> 33.
-// A K of at most 128 (two slabs of the right side) leaves too little to share: a step over
-// 16384 x 128 at rank 64 takes 42.0 us split and 41.6 not, over 128 x 16384 43.4 and 43.9,
-// and such shapes keep the reduction in one wave, the order of an unsplit sum.
+// A K of at most 128 (two slabs of the right side) keeps the reduction in one wave and with
+// it the order of an unsplit sum: splitting it is worth nothing (a step over 16384 x 128 at
+// rank 64 takes 42.0 us split and 41.6 not, over 128 x 16384 43.4 and 43.9, the same within
+// the runs' spread), and the other order moved a code of a stored bf16 trajectory of the
+// tests, which compares the low-rank codes with the reference's.
 __device__ __forceinline__ int ap_nkg(int64_t rp, int64_t K) {
   return K <= 128 || rp > 128 ? 1 : (rp <= 64 ? 4 : 2);
 }
@@ -897,6 +902,11 @@ __device__ __forceinline__ void proj_left(const ApDesc& D, const ApL& L, int til
 // non-zero products or more errs less as well (0.97), one with 5 errs 1.03 times as much
 // (7.5e-8), one with a single product 5.0e-8 in place of 3.3e-8 of its rms (a rounding to
 // fp32 alone: 2.6e-8 rms, 6.0e-8 at most).
+//
+// Rank 256 over 1.1e9 elements: three bf16 terms 1577 us, two fp16 terms 1293, with the
+// barrier inside the MFMA stream 1241, with each slab tested for itself 1176.  Matrix cores are
+// busy for 49% of the cycles at the 1.7 GHz the chip holds here; the last round of tiles (7.2
+// per CU) leaves a tenth idle.
 //
 // Four matrices of 32000 x 2048 at rank 256, a step (in brackets with three bf16 terms from
 // the first slab on): normal gradients 761 us (836), nine tenths of the rows zero 713 (780),
@@ -1851,7 +1861,7 @@ __global__ __launch_bounds__(256) void k_ap_psq(ApDesc D) {
 // (the channel or tensor scale, optimizer.py:2997-3001), so it takes the hardware
 // square root and reciprocal (<= 2 ulp), as the 1-D step's Adam denominator does.  FULL: the unit lies
 // inside g_low and u is 16-byte aligned, so every access is a vector access.
-// AL8 blocks of >= 512 elements decode through an LDS table of the block's
+// AL8 blocks of >= 1024 elements decode through an LDS table of the block's
 // 255 code values (one correctly rounded exp2 per lane per block).
 template <int VB, int MK, bool FULL>
 __device__ __forceinline__ void ap_low_unit(const ApDesc& D, const ApL& L, int unit, const ApHyp& h, float* xw,
@@ -2470,8 +2480,6 @@ __global__ __launch_bounds__(256) void k_ap_apply(ApDesc one, const ApDesc* tab,
 }
 
 hipError_t apollo_upload_qmap(const float* q8, const float* q4) { return upload_qmap_tu(q8, q4); }
-
-// ------------------------------------------------------------ rocBLAS (fp32 G)
 
 template <int VB>
 static void launch_low(int mkt, unsigned nb, const ApDesc& one, const ApDesc* tab, int ntab, const ApHyp& h,

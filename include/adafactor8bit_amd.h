@@ -395,7 +395,7 @@ typedef struct a8_apollo_tensor {
   int has_fira_prev;       /* 0 on the first Fira step */
   const float* lr;         /* device learning rate, or NULL for lr_val */
   float* workspace;        /* a8_apollo_workspace_floats(rows, cols, rank, channel) floats, kept
-                              across steps (it caches the bf16 split of P^T) */
+                              across steps (it caches the split of P^T) */
   uint64_t sr_seed;
   /* per-step fields, read by a8_apollo_step_multi (a8_apollo_step takes them as arguments) */
   int first_step;          /* V initialised as g_low^2 * beta_val (no low-rank state yet) */
@@ -447,7 +447,7 @@ int64_t a8_apollo_workspace_floats(int64_t rows, int64_t cols, int64_t rank, int
  * with t the device step, when t - last_proj_step >= proj_gap the step takes
  * current_proj_seed = apollo_seed, apollo_seed = next_seed(that seed) (the
  * reference's seed chain, optimizer.py:152-155, restated on the device) and
- * last_proj_step = t, and regenerates P^T (proj_t, written in place) and its bf16
+ * last_proj_step = t, and regenerates P^T (proj_t, written in place) and its
  * split with a8_apollo_proj_gen's generator; fresh = 2 set by the caller rebuilds
  * only the split from proj_t.  proj_fresh, step and bias_factor of the records are
  * then not read, so a step so launched can be captured in a HIP graph and
